@@ -158,19 +158,33 @@ def _materials(n, w, h, colours, g):
     return out.cpu().numpy()
 
 
-class _Served:
-    """A server, its context and its resident libraries, closed in that order."""
+class _Service:
+    """What a serving program keeps: one server, and the four resident libraries of its context."""
 
-    def __init__(self, mats):
+    def __init__(self):
         self.ctx = _binding().Context(0)
-        self.libs = [self.ctx.library_from_pixels(m) for m in mats]
+        self.libs = [self.ctx.library_from_pixels(_materials(n, 64, 64, "mix", _gen(1, n))) for n in (1000, 2500, 5000, 10000)]
         self.server = self.ctx.server()
 
-    def __del__(self):
+    def close(self):
         self.server.close()
         for lib in self.libs:
             lib.close()
         self.ctx.close()
+
+
+_serving = None
+
+
+def _service(wanted):
+    """The service, made once; a program that does other work has none."""
+    global _serving
+    if wanted and _serving is None:
+        _serving = _Service()
+    elif not wanted and _serving is not None:
+        _serving.close()
+        _serving = None
+    return _serving
 
 
 def _job_params(case, seed):
@@ -205,7 +219,7 @@ def _images(case, seed):
 
 def prepare(case, seed):
     kind, g = case["kind"], _gen(seed)
-    mh = _binding()
+    mh, service = _binding(), _service(case["kind"] == "served")
     if kind in ("job", "oneshot"):
         tw, th = case["width"] // case["gw"], case["height"] // case["gh"]
         target = _target(case["width"], case["height"], g)
@@ -221,11 +235,10 @@ def prepare(case, seed):
         if kind == "batch":
             mats = [_materials(int(round(math.exp(rng.uniform(math.log(case["lo"]), math.log(case["hi"]))))), 64, 64, "flat", g)
                     for _ in range(case["libs"])]
-            ctx, keep = _context(), None
+            ctx = _context()
             libs = [ctx.library_from_pixels(m) for m in mats]
         else:
-            keep = _Served([_materials(n, 64, 64, "mix", g) for n in (1000, 2500, 5000, 10000)])
-            ctx, libs = keep.ctx, keep.libs
+            ctx, libs = service.ctx, service.libs
         cw, ch = max(j[1] for j in jobs) * 16 + 64, max(j[2] for j in jobs) * 16 + 64
         canvas = [_target(cw, ch, g) for _ in range(4)]  # the jobs' targets are crops of these
         cells = [j[1] * j[2] for j in jobs]
@@ -238,7 +251,7 @@ def prepare(case, seed):
             mj.append(ctx.job(libs[lib], canvas[k % 4].data_ptr() + (oy * cw + ox) * 3, gw * 16, gh * 16, p,
                               grid.data_ptr() + 4 * at, image.data_ptr() + 768 * at, cw * 3))
             at += cells[k]
-        s = dict(case=case, libs=libs, canvas=canvas, grid=grid, image=image, jobs=mj, keep=keep)
+        s = dict(case=case, libs=libs, canvas=canvas, grid=grid, image=image, jobs=mj, service=service)
         if kind == "batch":
             torch.cuda.synchronize()
             s["batch"] = ctx.batch(mj)
@@ -270,7 +283,7 @@ def run(s):
         s["batch"].run()
         return s["grid"], s["image"]
     if kind == "served":
-        server = s["keep"].server
+        server = s["service"].server
         if case["at_once"]:
             server.submit_many(s["jobs"])
             server.drain()
