@@ -403,8 +403,14 @@ __device__ __forceinline__ void topk_run(const TopkSeg& s, int32_t q0, int32_t r
                 if (s.out_idx) gstore(s.out_idx, o, m);
                 if (s.out_d) gstore(s.out_d, o, __uint_as_float((uint32_t)(key >> 32)));
                 // the key is {m, d} as one little-endian word: m in the low
-                // half (CandRec::m, offset 0), the distance bits in the high
-                if (s.out_cand) gstore((uint64_t*)s.out_cand, o, key);
+                // half (CandRec::m, offset 0), the distance bits in the high;
+                // the GUI score's rows hold the distance itself (sqrt is
+                // monotone, so the order stands)
+                if (s.out_cand) {
+                    const float d = __uint_as_float((uint32_t)(key >> 32));
+                    gstore((uint64_t*)s.out_cand, o,
+                           s.root ? make_key(__float_as_uint(sqrtf(d)), m) : key);
+                }
             } else if (s.out_cand) {
                 // padded (chain) rows: ranks beyond k, -1 with an infinite distance
                 gstore((uint64_t*)s.out_cand, o, (uint64_t)0x7f800000u << 32 | 0xffffffffu);
@@ -445,10 +451,10 @@ int32_t topk_blocks(int32_t nq, int32_t run) { return nq > 0 ? (nq + run - 1) / 
 
 void launch_topk(const float* mL, const float* mA, const float* mB, int32_t n, const MatBlocks& blk,
                  const float* query, int32_t nq, int32_t k, int32_t* out_idx, float* out_d,
-                 CandRec* out_cand, int32_t out_stride, hipStream_t stream) {
+                 CandRec* out_cand, int32_t out_stride, bool root, hipStream_t stream) {
     if (k > n) k = n;
     if (nq <= 0 || n <= 0 || k <= 0) return;
-    const TopkSeg s{mL, mA, mB, query, out_idx, out_d, out_cand, n, nq, k, out_stride, blk};
+    const TopkSeg s{mL, mA, mB, query, out_idx, out_d, out_cand, n, nq, k, out_stride, blk, root};
     const int32_t run = topk_run_length(nq);
     hipLaunchKernelGGL(topk_kernel, dim3(topk_blocks(nq, run)), dim3(64), 0, stream, s, run);
 }

@@ -217,13 +217,12 @@ int run_place(mh_context* ctx, const mh_library* lib, const float* d_cell_lab, i
               uint8_t* d_stage, float* d_dist, float* d_score, int32_t* d_stats,
               CandRec* cand_buf = nullptr) {
     const int32_t cells = gw * gh;
-    // the raster chain stages its candidate rows in LDS when they fit
-    const bool staged = raster && place_raster_lds_bytes(gw, lib->n, true) <= ctx->max_lds;
-    size_t lds = raster ? place_raster_lds_bytes(gw, lib->n, staged)
-                        : place_lds_bytes(cells, lib->n);
+    const int32_t form = raster ? raster_form(gw, lib->n, d_stage || d_dist || d_score, true, ctx->max_lds) : -1;
+    size_t lds =
+        form >= 0 ? place_raster_lds_bytes(gw, lib->n, form) : place_lds_bytes(cells, lib->n);
     // state beyond LDS: the general chain with grid and counts in HBM (it
     // reads the neighbours from the grid, so a raster run starts it empty)
-    const bool hbm = lds > ctx->max_lds;
+    const bool hbm = raster ? form < 0 : lds > ctx->max_lds;
     if (hbm) {
         lds = 0;
         if (raster) fill_i32(d_grid, cells, kEmpty, ctx->stream);
@@ -234,7 +233,7 @@ int run_place(mh_context* ctx, const mh_library* lib, const float* d_cell_lab, i
     const int32_t K = lib->n < kMaxCand ? lib->n : kMaxCand;
     phase_begin(ctx, MH_PHASE_TOPK);
     launch_topk(lib->d_L, lib->d_A, lib->d_B, lib->n, library_blocks(lib), d_cell_lab, cells, K,
-                nullptr, nullptr, cand, kCandStride, ctx->stream);
+                nullptr, nullptr, cand, kCandStride, score_mode == MH_SCORE_DISTANCE, ctx->stream);
     phase_end(ctx, MH_PHASE_TOPK);
     PlaceJob job;
     job.lab4 = lib->d_lab4;
@@ -245,17 +244,17 @@ int run_place(mh_context* ctx, const mh_library* lib, const float* d_cell_lab, i
     job.grid = d_grid;
     job.usage = d_usage;
     job.zero_usage = zero_usage ? 1 : 0;
+    job.form = form;
     job.grid_w = gw;
     job.grid_h = gh;
     job.max_usage = max_usage;
     job.weight = weight;
-    job.score_sqrt = score_mode == MH_SCORE_DISTANCE ? 1 : 0;
     job.stage = d_stage;
     job.dist = d_dist;
     job.score = d_score;
     job.stats = d_stats;
     phase_begin(ctx, MH_PHASE_PLACE);
-    launch_place_single(job, raster && !hbm, staged, lds, ctx->stream);
+    launch_place_single(job, raster && !hbm, lds, ctx->stream);
     phase_end(ctx, MH_PHASE_PLACE);
     HIPCHK(hipGetLastError());
     return MH_OK;
@@ -874,7 +873,15 @@ static int library_upload_lab(mh_library* lib) {
     HIPCHK(hipMemcpy(lib->d_L, L.data(), sizeof(float) * n, hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(lib->d_A, A.data(), sizeof(float) * n, hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(lib->d_B, B.data(), sizeof(float) * n, hipMemcpyHostToDevice));
-    return library_build_blocks(lib);
+    CHK(library_build_blocks(lib));
+    // largest adjacency terms, for the placement's prepared lists (a library
+    // that has none in the narrowest grid does not read them)
+    if (place_raster_lds_bytes(1, n, kRasterLists) <= lib->ctx->max_lds) {
+        launch_near_terms(lib->d_lab4, n, lib->ctx->stream);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipStreamSynchronize(lib->ctx->stream));
+    }
+    return MH_OK;
 }
 
 int mh_library_from_lab(mh_context* ctx, const float* lab, int32_t n, mh_library** out) {
@@ -1213,7 +1220,7 @@ int mh_nearest_n(mh_context* ctx, const mh_library* lib, const float* query, int
     CHK(slot(ctx, S_OUT0, (size_t)nq * kk, &d_i));
     CHK(slot(ctx, S_OUT1, (size_t)nq * kk, &d_d));
     launch_topk(lib->d_L, lib->d_A, lib->d_B, lib->n, library_blocks(lib), d_q, nq, kk, d_i, d_d,
-                nullptr, kk, ctx->stream);
+                nullptr, kk, false, ctx->stream);
     HIPCHK(hipGetLastError());
     CHK(download(ctx, idx, d_i, (size_t)nq * kk));
     CHK(download(ctx, sqdist, d_d, (size_t)nq * kk));
@@ -1259,9 +1266,11 @@ int mh_place(mh_context* ctx, const mh_library* lib, const float* cell_lab,
     bool empty_grid = true;
     for (int32_t i = 0; i < cells && empty_grid; ++i) empty_grid = grid[i] == MH_EMPTY;
     const bool raster = !order && empty_grid;
+    bool unused = true;  // fresh counts: the chain need not read them
+    for (int32_t i = 0; i < lib->n && unused; ++i) unused = usage[i] == 0;
     CHK(run_place(ctx, lib, d_lab, p->grid_w, p->grid_h, p->max_usage, p->weight, p->score_mode,
                   raster, d_order,
-                  order ? n_order : cells, d_grid, d_usage, false, d_stage, d_dist, d_score,
+                  order ? n_order : cells, d_grid, d_usage, unused, d_stage, d_dist, d_score,
                   d_stats));
     int32_t st[6];
     CHK(download(ctx, grid, d_grid, (size_t)cells));

@@ -2,7 +2,7 @@
 // continuous-batching request loop (mh_server_*).
 //
 // A batch runs every job's whole pipeline with one launch per stage:
-//   cell Lab means -> K nearest -> placement chains (a wave per job) ->
+//   cell Lab means -> K nearest -> placement chains (a workgroup per job) ->
 //   annealing chains (a wave per job) -> cell averages + adjustments ->
 //   composite.
 // Wide stages find their job through a segment table (block -> job by
@@ -48,7 +48,6 @@ struct JobSpec {
     bool sa = false, adjust = false;
     int32_t anneal_kind = 0;  // the annealing variant (mh::anneal_kind)
     bool place_hbm = false;   // placement state in HBM (library beyond LDS)
-    bool place_staged = false;  // the LDS chain's staged candidate rows fit too
     float strength = 0.0f;
     const float* term = nullptr;
     const float* temps = nullptr;
@@ -91,8 +90,7 @@ int check_job(const mh_context* ctx, const mh_job& j, JobSpec* s) {
     s->strength = k < 0.0f ? 0.0f : (k > 1.0f ? 1.0f : k);  // src/main.rs:162
     s->adjust = s->strength > 0.0f;
     // placement state beyond LDS runs the chain with grid and counts in HBM
-    s->place_hbm = place_raster_lds_bytes(s->gw, s->n, false) > ctx->max_lds;
-    s->place_staged = place_raster_lds_bytes(s->gw, s->n, true) <= ctx->max_lds;
+    s->place_hbm = raster_form(s->gw, s->n, false, false, ctx->max_lds) < 0;
     s->anneal_kind = s->sa ? anneal_kind(s->cells, s->n, s->gw, s->gh, ctx->max_lds) : 0;
     if (s->anneal_kind < 0)
         return fail(MH_ERR_UNSUPPORTED, "annealing a %d x %d grid: a side of 65,536 or more", s->gw,
@@ -139,8 +137,6 @@ struct BatchPlan {
     int32_t lab_blocks = 0, lab_cpb = 4;
     int32_t n_topk = 0, topk_blocks = 0, topk_run = 1;
     size_t place_lds = 0;
-    bool place_staged = false;  // the LDS chains stage their candidate rows
-    int32_t place_score = kScoreSq;  // kScoreSq / kScoreDist / kScoreMixed over the jobs
     // placement entries: raster chains with state in LDS first, then the
     // chains with state in HBM, whose grids start empty (filled per launch)
     int32_t n_place_lds = 0;
@@ -197,14 +193,11 @@ T* at(uint8_t* base, size_t off) {
 }
 
 // Fill the host image `h` of a batch block whose device copy lives at `d`;
-// job i's working memory is at job_mem[i].  stage_rows: the raster chains
-// stage their candidate rows in LDS when every job's fit (52 KB more per
-// chain).  A batch's one or two chain launches gain from it (the chain time
-// is the batch's critical path); the server keeps several batches' chains
-// and wide stages on the GPU at once, where the larger LDS footprint costs
-// more in chains and blocks resident per CU than the staging saves.
+// job i's working memory is at job_mem[i].  labs: the placement chains keep
+// material Labs in LDS where they fit (the batch's chains have the CUs to
+// themselves; the server's share them with other batches' stages).
 int build_plan(const std::vector<JobSpec>& specs, const std::vector<uint8_t*>& job_mem, uint8_t* h,
-               uint8_t* d, bool stage_rows, BatchPlan* p) {
+               uint8_t* d, bool labs, BatchPlan* p) {
     const int32_t n = (int32_t)specs.size();
     p->n_jobs = n;
     plan_bytes(n, p);
@@ -231,9 +224,6 @@ int build_plan(const std::vector<JobSpec>& specs, const std::vector<uint8_t*>& j
     p->lab_cpb = cell_lab_cells_per_block(all_cells);
     p->topk_run = p->tune_topk_run > 0 ? p->tune_topk_run : topk_run_length(topk_queries);
     p->place_lds = 0;
-    p->place_staged = stage_rows;  // until a job's staged rows do not fit
-    size_t lds_plain = 0, lds_staged = 0;
-    p->place_score = kScoreSq;
     p->hbm_grids.clear();
     p->n_place_lds = 0;
     std::vector<PlaceJob> hbm_place;
@@ -263,7 +253,8 @@ int build_plan(const std::vector<JobSpec>& specs, const std::vector<uint8_t*>& j
             topk_st[p->n_topk] = (int32_t)topk_blocks;
             topk[p->n_topk] = TopkSeg{lib->d_L, lib->d_A, lib->d_B, cell_lab, nullptr, nullptr,
                                       cand, s.n, s.cells, s.n < kMaxCand ? s.n : kMaxCand,
-                                      kCandStride, library_blocks(lib)};
+                                      kCandStride, library_blocks(lib),
+                                      j.params.score_mode == MH_SCORE_DISTANCE ? 1 : 0};
             ++p->n_topk;
             topk_blocks += topk_blocks_of(s.cells, p->topk_run);
         }
@@ -277,23 +268,20 @@ int build_plan(const std::vector<JobSpec>& specs, const std::vector<uint8_t*>& j
         pj.grid = grid;
         pj.usage = at<uint32_t>(m, s.o_usage);
         pj.zero_usage = 1;
+        pj.form = raster_form(s.gw, s.n, false, labs, lib->ctx->max_lds);
         pj.grid_w = s.gw;
         pj.grid_h = s.gh;
         pj.max_usage = j.params.max_usage;
         pj.weight = j.params.weight;
-        pj.score_sqrt = j.params.score_mode == MH_SCORE_DISTANCE ? 1 : 0;
         pj.stats = d_stats + (size_t)i * kStatsInts;
         if (s.place_hbm) {
             hbm_place.push_back(pj);
             p->hbm_grids.emplace_back(grid, s.cells);
         } else {
             place[p->n_place_lds++] = pj;
-            lds_plain = std::max(lds_plain, place_raster_lds_bytes(s.gw, s.n, false));
-            lds_staged = std::max(lds_staged, place_raster_lds_bytes(s.gw, s.n, true));
-            p->place_staged = p->place_staged && s.place_staged;
+            p->place_lds =
+                std::max(p->place_lds, place_raster_lds_bytes(s.gw, s.n, pj.form));
         }
-        const int32_t kind = pj.score_sqrt ? kScoreDist : kScoreSq;
-        p->place_score = i == 0 || p->place_score == kind ? kind : kScoreMixed;
         // a10-a12: annealing chain
         if (s.sa) {
             AnnealJob aj{};
@@ -325,7 +313,6 @@ int build_plan(const std::vector<JobSpec>& specs, const std::vector<uint8_t*>& j
         comp_blocks += composite_blocks(s.gw * s.tw, s.gh * s.th, p->comp_threads);
     }
     for (size_t h = 0; h < hbm_place.size(); ++h) place[p->n_place_lds + h] = hbm_place[h];
-    p->place_lds = p->place_staged ? lds_staged : lds_plain;
     p->n_anneal = 0;
     for (int kind = 0; kind < 3; ++kind) {
         p->anneal_start[kind] = p->n_anneal;
@@ -377,12 +364,10 @@ void enqueue_chains(const BatchPlan& p, uint8_t* d, hipStream_t s,
     pe.mark(MH_PHASE_PLACE, 0, s);
     const PlaceJob* pj = at<PlaceJob>(d, p.o_place);
     if (p.n_place_lds > 0)
-        launch_place_batch(pj, p.n_place_lds, true, p.place_staged, p.place_score, p.place_lds,
-                           s);
+        launch_place_batch(pj, p.n_place_lds, true, p.place_lds, s);
     if (p.n_jobs > p.n_place_lds) {
         for (const auto& g : p.hbm_grids) fill_i32(g.first, g.second, kEmpty, s);
-        launch_place_batch(pj + p.n_place_lds, p.n_jobs - p.n_place_lds, false, false,
-                           p.place_score, 0, s);
+        launch_place_batch(pj + p.n_place_lds, p.n_jobs - p.n_place_lds, false, 0, s);
     }
     pe.mark(MH_PHASE_PLACE, 1, s);
     pe.mark(MH_PHASE_ANNEAL, 0, s);
@@ -996,7 +981,7 @@ struct StreamSlot {
 // candidate lists (cell Labs, K nearest), which fill the device, run on two
 // wide streams, consecutive batches alternating (so one batch's launch tail
 // overlaps the next batch's start); each batch's chains (placement,
-// annealing: one wave per job, latency-bound) run on one of a few chain
+// annealing: a workgroup or wave per job, latency-bound) run on one of a few chain
 // streams after an event from the wide stream; its output stages
 // (adjustment, composite: wide again) run on that chain stream's output
 // stream after an event from the chain stream, so a batch's outputs never

@@ -13,7 +13,8 @@ constexpr int32_t kEmpty = -1;       // MH_EMPTY
 constexpr int32_t kMaxCand = 100;    // K = min(n, 100), src/main.rs:348
 constexpr int32_t kCandStride = 128; // per-cell candidate row (padded)
 
-// One candidate of a cell: material and squared distance, 8 bytes (one
+// One candidate of a cell: material and colour distance as the job's score
+// takes it (squared, or its square root for the GUI score), 8 bytes (one
 // 64-bit load).  Rows of kCandStride, ranks ascending (sqdist, idx); ranks
 // >= K hold {-1, +inf}.  A candidate's Lab is read from the library's lab4
 // where a penalty needs it.
@@ -25,7 +26,7 @@ static_assert(sizeof(CandRec) == 8, "one 64-bit word per candidate");
 
 // One placement chain (one wave).  All pointers are device pointers.
 struct PlaceJob {
-    const float4* lab4;      // n material Labs {l,a,b,0}
+    const float4* lab4;      // n material Labs {l,a,b} and their largest adjacency terms
     int32_t n;
     const CandRec* cand;      // cells x kCandStride
     const int32_t* order;     // n_order cell indices, or nullptr = raster
@@ -33,10 +34,10 @@ struct PlaceJob {
     int32_t* grid;            // cells, in/out
     uint32_t* usage;          // n, in/out
     int32_t zero_usage;       // 1: start from zero counts instead of reading `usage`
+    int32_t form;             // raster chain: kRasterPlain, kRasterLists or kRasterLabs
     int32_t grid_w, grid_h;
     int32_t max_usage;
     float weight;
-    int32_t score_sqrt;       // 1: candidates score sqrt(sqdist) + penalty (GUI variant)
     uint8_t* stage;           // optional per-cell outputs
     float* dist;
     float* score;
@@ -111,6 +112,7 @@ struct TopkSeg {
     CandRec* out_cand;   // optional; rows padded with {-1, +inf} up to out_stride
     int32_t n, nq, k, out_stride;
     MatBlocks blk;
+    int32_t root;        // 1: out_cand holds sqrt(sqdist) (GUI score)
 };
 
 // Finishing one placed grid: per-cell adjustment and compositing.
@@ -135,11 +137,13 @@ void launch_cell_lab(const uint8_t* rgb, int64_t row_stride, int32_t per_row,
                      uint8_t* out_rgb = nullptr);
 void launch_sim_full(const float4* lab, int32_t n, float* out, hipStream_t stream);
 void launch_sim_packed(const float4* lab, int32_t n, float* out, hipStream_t stream);
+// lab[i].w = material i's largest adjacency term to another material.
+void launch_near_terms(float4* lab, int32_t n, hipStream_t stream);
 void launch_term_full(const float4* lab, int32_t n, float* out, hipStream_t stream);
 // out_idx / out_d / out_cand may be null.
 void launch_topk(const float* mL, const float* mA, const float* mB, int32_t n, const MatBlocks& blk,
                  const float* query, int32_t nq, int32_t k, int32_t* out_idx, float* out_d,
-                 CandRec* out_cand, int32_t out_stride, hipStream_t stream);
+                 CandRec* out_cand, int32_t out_stride, bool root, hipStream_t stream);
 // Batched launches over segment tables: starts[j] is the first block of
 // segment j (starts[n_segs] = total).  *_blocks give each segment's count.
 // cells per block (4 or 16) for a launch over total_cells cells
@@ -166,19 +170,21 @@ void launch_composite_batch(const CompSeg* d_segs, const int32_t* d_starts, int3
 // General chain: any cell order, pre-filled grid and usage (state in LDS).
 size_t place_lds_bytes(int32_t cells, int32_t n);
 // Raster chain: generate_mosaic's raster order from an empty grid, where
-// only the up and left neighbours can be filled.  `staged`: the LDS also
-// holds two groups of candidate rows (52 KB more), copied in ahead of the
-// chain; the chain runs unstaged where that does not fit.
-size_t place_raster_lds_bytes(int32_t grid_w, int32_t n, bool staged);
+// only the up and left neighbours can be filled (a workgroup per job).  Its
+// LDS holds the usage counts alone (kRasterPlain: one wave walks the rows),
+// also the prepared candidate lists (kRasterLists), also the material Labs
+// (kRasterLabs; read from memory otherwise).  raster_form: the first of
+// kRasterLabs (if labs), kRasterLists, kRasterPlain that fits max_lds bytes,
+// the grid and the run (outputs: it wants every cell's stage, distance or
+// score), -1 if none does.
+constexpr int32_t kRasterPlain = 0, kRasterLists = 1, kRasterLabs = 2;
+int32_t raster_form(int32_t grid_w, int32_t n, bool outputs, bool labs, size_t max_lds);
+size_t place_raster_lds_bytes(int32_t grid_w, int32_t n, int32_t form);
 // One job passed by value (kernel argument), or n_jobs jobs from a device
-// array (one wave each); `staged` as for place_raster_lds_bytes.
-void launch_place_single(const PlaceJob& job, bool raster, bool staged, size_t lds_bytes,
-                         hipStream_t stream);
-// score_kind: kScoreSq or kScoreDist when every job scores alike, else
-// kScoreMixed (each job's score_sqrt is read).
-enum : int32_t { kScoreSq = 0, kScoreDist = 1, kScoreMixed = 2 };
-void launch_place_batch(const PlaceJob* d_jobs, int32_t n_jobs, bool raster, bool staged,
-                        int32_t score_kind, size_t lds_bytes, hipStream_t stream);
+// array; lds_bytes 0 (general chain): grid and counts in the job's buffers.
+void launch_place_single(const PlaceJob& job, bool raster, size_t lds_bytes, hipStream_t stream);
+void launch_place_batch(const PlaceJob* d_jobs, int32_t n_jobs, bool raster, size_t lds_bytes,
+                        hipStream_t stream);
 // Annealing variants: the grid in LDS with 16-bit material ids (libraries
 // under 32,768 materials) or 32-bit ids, or in HBM with hashed LDS stamps
 // (grids too large for LDS; sides below 65,536).
