@@ -568,7 +568,7 @@ def main():
         out["tiles_placed_per_s"] = sv["tiles_placed_per_s"]
         out["sa_proposals_per_s"] = sv["sa_proposals_per_s"]
         # roofline of the dominant kernel: the placement chains of each
-        # served batch (one wave per job), 16 B + 12 K B of algorithmic
+        # served batch (one workgroup per job), 16 B + 12 K B of algorithmic
         # traffic per tile placed (K = 100 for every library of the stream)
         if pt["launches"]:
             per_launch = pt["cells"] / pt["launches"] * (16 + 12 * 100)

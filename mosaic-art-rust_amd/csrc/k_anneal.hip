@@ -4,24 +4,23 @@
 // optimize_greedy, src/optimizer.rs:41-198).
 //
 // Annealing keeps the reference's one-proposal-at-a-time semantics exactly
-// while evaluating 64 proposals per round on one wave:
+// while a workgroup evaluates 64 proposals a round:
 //   * proposal `it` draws x1,y1,x2,y2,u from a counter RNG keyed by (seed,it),
 //     so any proposal can be evaluated out of order;
 //   * skipped proposals (same cell / empty cell) do not cool, and emptiness
 //     never changes under swaps, so proposal j's temperature index is the
 //     number of non-skipped proposals before it (a ballot prefix count) and
 //     T comes from a table built by the sequential f32 recurrence T *= decay;
-//   * every lane computes its delta on the round-start grid; accepted lanes
-//     stamp the two cells they would write (LDS atomicMax of
-//     round<<6 | 63-lane, i.e. the lowest writer wins); a lane whose read set
-//     (both cells and their 4-neighbours) holds a stamp from a lower lane is a
-//     conflict.  Lanes before the first conflict read exactly what the serial
-//     chain would have read, so they commit; the rest are re-drawn next round.
+//   * a round commits the proposals before the first that may have been
+//     evaluated on other values than the serial chain would have read; the
+//     rest are evaluated again in the next round;
 //   * the running cost is accumulated in proposal order (f32, as the
 //     reference's `current_cost += delta`).
 // Result: grid, costs and counts are bit-identical to the serial chain.
 #include "mh_device.hpp"
 #include "mh_kernels.hpp"
+
+#include <type_traits>
 
 namespace mh {
 
@@ -49,144 +48,121 @@ __device__ __forceinline__ void gput(HbmGrid* g, int32_t i, int32_t v) {
     __hip_atomic_store((MH_GAS int32_t*)g->p + i, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// One adjacency term 1/(sim(a,b)+1): a gather from the library's term
-// matrix when it is resident, else computed from the Lab table (same bits).
-// The source is a type rather than a run-time test inside every read, so a
-// caller's gathers are straight-line code that the compiler issues together
-// (behind a test per read, each gather was waited for on its own).
-struct TermMatrix {
-    const float* term;
-    int32_t n;
-    __device__ __forceinline__ float operator()(int32_t a, int32_t b) const {
-        return gload(term, (int64_t)a * n + b);
-    }
-};
+// One adjacency term 1/(sim(a,b)+1) from a Lab table in memory or in LDS.
 struct TermLab {
     const float4* lab4;
     __device__ __forceinline__ float operator()(int32_t a, int32_t b) const {
         return adj_term(gload4(lab4, a), gload4(lab4, b));
     }
 };
-
-// calculate_swap_delta (src/adjacency.rs:133-214) on a grid in any address
-// space.  Term order: neighbours of p1 (Up, Down, Left, Right, skipping p2),
-// then of p2 (skipping p1), then the mutual term when adjacent.
-//
-// Branch-free form: the eight neighbour slots are read first, then every
-// term of both rows (m1 and m2) is requested at once -- an absent slot reads
-// a valid dummy entry -- so the gathers cost one memory latency instead of
-// one each.  Absent terms are added as +0.0: the sums start at +0 and only
-// grow, and x + (+0) == x bit for bit, so this equals skipping them.
-//
-// The neighbour slots (Up, Down, Left, Right of p1, then of p2) are read by
-// swap_slots, which callers may issue together with their own reads of p1
-// and p2; a slot outside the grid reads its own cell, always in bounds, and
-// swap_delta_core masks it out.
-template <typename G>
-__device__ __forceinline__ void swap_slots(const G* grid, int32_t gw, int32_t gh, int32_t x1,
-                                           int32_t y1, int32_t x2, int32_t y2, int32_t nb[8]) {
-    const int32_t p1 = y1 * gw + x1, p2 = y2 * gw + x2;
-    nb[0] = gget(grid, y1 > 0 ? p1 - gw : p1);
-    nb[1] = gget(grid, y1 < gh - 1 ? p1 + gw : p1);
-    nb[2] = gget(grid, x1 > 0 ? p1 - 1 : p1);
-    nb[3] = gget(grid, x1 < gw - 1 ? p1 + 1 : p1);
-    nb[4] = gget(grid, y2 > 0 ? p2 - gw : p2);
-    nb[5] = gget(grid, y2 < gh - 1 ? p2 + gw : p2);
-    nb[6] = gget(grid, x2 > 0 ? p2 - 1 : p2);
-    nb[7] = gget(grid, x2 < gw - 1 ? p2 + 1 : p2);
-}
-
-// swap_delta_core in two parts, so that a caller can do other work while
-// the gathers are in flight: swap_terms requests every term (m1 and m2 must
-// be material ids), swap_sum adds them in the reference's order.
-struct SwapTerms {
-    float r1[8], r2[8];  // T(m1, a_i), T(m2, a_i)
-    float tm;            // T(m1, m2)
-    bool ok[8];          // slot i holds a neighbour that is not the partner
-    bool is_adj;
+struct TermLds {
+    const float4* labs;
+    __device__ __forceinline__ float operator()(int32_t a, int32_t b) const {
+        return adj_term(labs[a], labs[b]);
+    }
 };
 
-template <typename TS>
-__device__ __forceinline__ void swap_terms(int32_t gw, int32_t gh, const TS& T, int32_t x1,
-                                           int32_t y1, int32_t x2, int32_t y2, int32_t m1,
-                                           int32_t m2, const int32_t nb[8], SwapTerms& st) {
+// calculate_swap_delta (src/adjacency.rs:133-214): neighbours of p1 (Up,
+// Down, Left, Right, skipping p2), then of p2 (skipping p1), then the mutual
+// term when adjacent.  Absent terms are added as +0.0: the sums start at +0
+// and only grow, and x + (+0) == x bit for bit, so this equals skipping them.
+__device__ float swap_delta_dev(const int32_t* grid, int32_t gw, int32_t gh, const TermLab& T,
+                                int32_t x1, int32_t y1, int32_t x2, int32_t y2) {
     const int32_t p1 = y1 * gw + x1, p2 = y2 * gw + x2;
-    const bool in[8] = {y1 > 0, y1 < gh - 1, x1 > 0, x1 < gw - 1,
-                        y2 > 0, y2 < gh - 1, x2 > 0, x2 < gw - 1};
-    const int32_t pos[8] = {p1 - gw, p1 + gw, p1 - 1, p1 + 1, p2 - gw, p2 + gw, p2 - 1, p2 + 1};
-    int32_t a[8];
-    st.is_adj = false;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int32_t other = i < 4 ? p2 : p1;
-        const bool self = in[i] && pos[i] == other;  // the swap partner
-        if (i < 4) st.is_adj = st.is_adj || self;
-        const int32_t g = in[i] ? nb[i] : kEmpty;
-        st.ok[i] = in[i] && !self && g != kEmpty;
-        a[i] = st.ok[i] ? g : 0;
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        st.r1[i] = T(m1, a[i]);
-        st.r2[i] = T(m2, a[i]);
-    }
-    st.tm = T(m1, m2);
-}
-
-__device__ __forceinline__ float swap_sum(const SwapTerms& st) {
+    const int32_t m1 = gget(grid, p1), m2 = gget(grid, p2);
+    if (m1 == kEmpty || m2 == kEmpty || m1 == m2) return 0.0f;
     float old_cost = 0.0f, new_cost = 0.0f;
+    bool adjacent = false;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {  // p1's neighbours: old with m1, new with m2
-        old_cost += st.ok[i] ? st.r1[i] : 0.0f;
-        new_cost += st.ok[i] ? st.r2[i] : 0.0f;
+    for (int i = 0; i < 8; ++i) {
+        const int32_t x = i < 4 ? x1 : x2, y = i < 4 ? y1 : y2, p = i < 4 ? p1 : p2;
+        const int k = i & 3;
+        const bool in = k == 0 ? y > 0 : k == 1 ? y < gh - 1 : k == 2 ? x > 0 : x < gw - 1;
+        const int32_t q = k == 0 ? p - gw : k == 1 ? p + gw : k == 2 ? p - 1 : p + 1;
+        const bool self = in && q == (i < 4 ? p2 : p1);  // the swap partner
+        adjacent = adjacent || self;
+        const int32_t a = in && !self ? gget(grid, q) : kEmpty;
+        const float t1 = a != kEmpty ? T(m1, a) : 0.0f, t2 = a != kEmpty ? T(m2, a) : 0.0f;
+        old_cost += i < 4 ? t1 : t2;
+        new_cost += i < 4 ? t2 : t1;
     }
-#pragma unroll
-    for (int i = 4; i < 8; ++i) {  // p2's neighbours: old with m2, new with m1
-        old_cost += st.ok[i] ? st.r2[i] : 0.0f;
-        new_cost += st.ok[i] ? st.r1[i] : 0.0f;
+    if (adjacent) {
+        const float t = T(m1, m2);
+        old_cost += t;
+        new_cost += t;
     }
-    old_cost += st.is_adj ? st.tm : 0.0f;
-    new_cost += st.is_adj ? st.tm : 0.0f;
     return new_cost - old_cost;
 }
 
-template <typename TS>
-__device__ __forceinline__ float swap_delta_core(int32_t gw, int32_t gh, const TS& T, int32_t x1,
-                                                 int32_t y1, int32_t x2, int32_t y2, int32_t m1,
-                                                 int32_t m2, const int32_t nb[8]) {
-    if (m1 == kEmpty || m2 == kEmpty) return 0.0f;
-    if (m1 == m2) return 0.0f;
-    SwapTerms st;
-    swap_terms(gw, gh, T, x1, y1, x2, y2, m1, m2, nb, st);
-    return swap_sum(st);
+// s + t[0] + t[1] + ... + t[n - 1] in this order, each addition rounded to
+// f32, by one wave: s and every t are >= 0, t is 16-byte aligned and readable
+// to the next multiple of four, where it is +0.0 past n.
+//
+// One dependent addition after another takes 9 ns (its read included); 256
+// are done at once where their result is known to be the same.  While the
+// sum stays in one binade it is a whole multiple of the binade's ulp, and so
+// adding t adds t rounded to a multiple of the ulp, whatever the sum is --
+// unless t lies half way between two multiples, when the sum's last bit
+// decides.  The rounded terms are whole numbers of ulps, whose sum has no
+// order.  Blocks with a half-way term and blocks that leave the binade (the
+// first few hundred terms, mostly) are added one by one.
+__device__ float sum_in_order(float s, const float* t, int32_t n) {
+    const int lane = threadIdx.x & 63;
+    const float4* v = reinterpret_cast<const float4*>(t);
+    const int32_t n4 = (n + 3) / 4;
+    for (int32_t base = 0; base < n4; base += 64) {
+        const int32_t len = min(64, n4 - base);
+        float4 q = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (lane < len) q = v[base + lane];
+        const uint32_t bits = __float_as_uint(s), exponent = bits >> 23;
+        if (exponent >= 23 && exponent < 250) {
+            // 1 / ulp(s); the products are exact (those below the normal range are 0 here)
+            const float inv = __uint_as_float((277u - exponent) << 23);
+            const float f[4] = {q.x * inv, q.y * inv, q.z * inv, q.w * inv};
+            bool plain = true;
+            uint32_t sum = 0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float r = __builtin_rintf(f[i]);
+                plain = plain && f[i] <= 4194304.0f && __builtin_fabsf(f[i] - r) != 0.5f;
+                sum += (uint32_t)r;
+            }
+            if (!wave_ballot(!plain)) {
+                const uint32_t m = ((bits & 0x7fffffu) | 0x800000u) + wave_sum_u32(sum);
+                if (m < 0x1000000u) {
+                    s = __uint_as_float((bits & 0xff800000u) | (m & 0x7fffffu));
+                    continue;
+                }
+            }
+        }
+        for (int32_t i = base; i < base + len; ++i) {
+            const float4 a = v[i];
+            s = s + a.x;
+            s = s + a.y;
+            s = s + a.z;
+            s = s + a.w;
+        }
+    }
+    return s;
 }
 
+// calculate_total_cost (src/adjacency.rs:91-130) by one workgroup: the terms
+// of `chunk` cells at a time are computed in parallel into scratch (right
+// term, down term per cell), then the first wave adds them in the reference's
+// order (raster, right before down).  An absent term is stored as +0.0: the
+// running sum starts at +0 and only grows, and x + (+0) == x bit for bit, so
+// adding it leaves the sum exactly as the reference's skipped addition does.
+// scratch holds 2*chunk + 2 floats and is 16-byte aligned.  The result is
+// returned to the first wave.
 template <typename G, typename TS>
-__device__ float swap_delta_dev(const G* grid, int32_t gw, int32_t gh, const TS& T,
-                                int32_t x1, int32_t y1, int32_t x2, int32_t y2) {
-    int32_t nb[8];
-    swap_slots(grid, gw, gh, x1, y1, x2, y2, nb);
-    return swap_delta_core(gw, gh, T, x1, y1, x2, y2, gget(grid, y1 * gw + x1),
-                           gget(grid, y2 * gw + x2), nb);
-}
-
-// calculate_total_cost (src/adjacency.rs:91-130) by one wave: the terms of
-// `chunk` cells at a time are computed in parallel into scratch (right term,
-// down term per cell), then lane 0 adds them in the reference's order
-// (raster, right before down).  An absent term is stored as +0.0: the running
-// sum starts at +0 and only grows, and x + (+0) == x bit for bit, so adding
-// it leaves the sum exactly as the reference's skipped addition does.
-// scratch holds 2*chunk + 2 floats and is 16-byte aligned.
-// The result is broadcast to every lane.
-template <typename G, typename TS>
-__device__ float total_cost_wave(const G* grid, int32_t gw, int32_t gh, const TS& T,
-                                 float* scratch, int32_t chunk) {
-    const int lane = threadIdx.x;
+__device__ float total_cost_block(const G* grid, int32_t gw, int32_t gh, const TS& T,
+                                  float* scratch, int32_t chunk) {
+    const int tid = threadIdx.x;
     const int32_t cells = gw * gh;
     float total = 0.0f;
     for (int32_t base = 0; base < cells; base += chunk) {
         const int32_t len = min(chunk, cells - base);
-        for (int32_t i = lane; i < len; i += 64) {
+        for (int32_t i = tid; i < len; i += blockDim.x) {
             const int32_t c = base + i;
             const int32_t x = c % gw, y = c / gw;
             const int32_t m = gget(grid, c);
@@ -204,335 +180,596 @@ __device__ float total_cost_wave(const G* grid, int32_t gw, int32_t gh, const TS
             scratch[2 * i] = tr;
             scratch[2 * i + 1] = td;
         }
-        if ((len & 1) != 0 && lane == 0) {  // pad to a whole float4
+        if ((len & 1) != 0 && tid == 0) {  // pad to a whole float4
             scratch[2 * len] = 0.0f;
             scratch[2 * len + 1] = 0.0f;
         }
         __syncthreads();
-        if (lane == 0) {
-            const float4* v = reinterpret_cast<const float4*>(scratch);
-            const int32_t n4 = (2 * len + 3) / 4;
-            for (int32_t i = 0; i < n4; ++i) {
-                const float4 t = v[i];
-                total = total + t.x;
-                total = total + t.y;
-                total = total + t.z;
-                total = total + t.w;
-            }
-        }
+        if (tid < 64) total = sum_in_order(total, scratch, 2 * len);
         __syncthreads();
     }
-    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(total)));
+    return total;
 }
 
 // ---------------------------------------------------------- annealing
-// Stamp words per job: one per cell plus slack, a multiple of 4 (the words
-// double as the cost scratch: 2 floats per cell of a chunk + 2 of padding).
-__host__ __device__ __forceinline__ int32_t stamp_words(int32_t cells) {
-    return (cells + 8) & ~3;
-}
-// One word per lane for packing a round's accepted deltas.
-constexpr int32_t kPackWords = 64;
-// Proposal draws, made ahead in blocks of 128 iterations (two per lane) into
-// a ring of 256 slots of three words: x1 | y1 << 16, x2 | y2 << 16, u (both
-// sides are below 2^16: a grid in LDS is far smaller, and the HBM variant
-// requires it).
-constexpr int32_t kRing = 256;
-constexpr int32_t kRingWords = 3 * kRing;
-// Stamp table of the HBM variant: cell p stamps word p mod kHashStamps.  Two
-// cells sharing a word can only make a lane see a conflict that is not there,
-// which ends the round early; the commits stay those of the serial chain.
+// What bounds it is the latency of a round, and how many proposals a round
+// commits.  A round runs on seven waves of one workgroup, a barrier between
+// its three phases (s: the first proposal of the round; lane l of the first
+// four waves: proposal s + l):
+//   * reads: slot wave w reads the swap's two cells and its two of their
+//     eight neighbour cells (w = 0, 1: Up and Down, Left and Right of the
+//     first cell; 2, 3: of the second), and those materials' Labs;
+//   * terms: the four adjacency terms of its two neighbours with the swap's
+//     two materials, to LDS;
+//   * decisions: wave 0 adds a swap's terms in the reference's order, decides
+//     it, finds how many proposals can be committed, and swaps.
+// Meanwhile three waves, on the SIMDs that wait for wave 0 then, draw later
+// proposals and add the last round's deltas to the running cost.  (The fifth
+// wave would share wave 0's SIMD: it ends after the set-up.)
+//
+// A round's prefix that can be committed, `first`, is found in one of two
+// ways, by which is longer for the share p of proposals that are accepted:
+//   * expecting all of them to be accepted (the usual case: annealing starts
+//     hot): in the first phase every lane stamps its two cells (the lowest
+//     lane wins).  A neighbour stamped by a lower lane k is taken to be what
+//     k's swap moves there: k's other material, whose Lab is in LDS.  A lane
+//     one of whose own cells is stamped by a lower lane ends the prefix, and
+//     so does one with a neighbour taken from a lane that is then rejected.
+//     The lanes before `first` have 2 cells each, all different, so who wrote
+//     a cell last, and what k held, is as assumed.  A lane ends it with a
+//     probability of (4 + 16 (1 - p)) / cells for each lane below it.
+//   * expecting none: every lane reads the cells as they are, accepted lanes
+//     stamp theirs, and a lane with a lower lane's stamp on any of its ten
+//     cells ends the prefix: 20 p / cells.
+// The second is better for p < 5/9.
+//
+// Measured against one wave that gathered its terms from a matrix of all pairs
+// and added the initial cost one term after another: 1,000 proposals on 20 x
+// 15 cells 332 -> 149 us (200 rounds -> 97), 2,000 on 80 x 60 340 -> 116 (100
+// -> 54), 2,000 on 206 x 116 600 -> 187, 20,000 on 200 x 120 1,650 -> 742.  A
+// round takes 1.6 us for 3.3: its three phases 0.45 each, and the barriers.
+constexpr int kSlotWaves = 4, kIdleWave = 4, kDraw1Wave = 5, kDraw2Wave = 6, kCostWave = 7;
+constexpr int32_t kAnnealThreads = 512;
+static_assert(kAnnealThreads == 64 * (kCostWave + 1), "one wave a role");
+
+// Stamps, tag << 7 | (63 - lane) << 1 | cell (0: the first of the swap): one
+// word per cell, or for grids of more cells kHashStamps words that cells
+// share (p mod kHashStamps).  A shared word can make a lane see a stamp that
+// is not its cell's: that only ends the prefix early, or is found out by
+// comparing the cells (substituted neighbours).  The words double as scratch
+// of the initial cost (2 floats per cell of a chunk + 2 of padding).
 constexpr int32_t kHashStamps = 16384;
+__host__ __device__ __forceinline__ int32_t stamp_words(int32_t cells) {
+    return cells > kHashStamps ? kHashStamps : (cells + 8) & ~3;
+}
+constexpr uint32_t kTagEnd = (1u << 25) - 1u;  // (odd: pack buffers alternate across the wrap)
+// Proposal draws, made ahead into a ring of three words a slot: x1 | y1 << 16,
+// x2 | y2 << 16, u (both sides are below 2^16: a grid in LDS is far smaller,
+// and the HBM variant requires it).
+constexpr int32_t kRing = 256;
 
-// kHbm: the grid stays in HBM (the job's own grid, swapped in place) and the
-// stamps are hashed into kHashStamps LDS words, for grids too large for LDS.
-template <typename G, bool kHbm>
-__global__ __launch_bounds__(64) void anneal_kernel(AnnealJob single,
-                                                    const AnnealJob* __restrict__ jobs) {
-    extern __shared__ __align__(16) uint32_t sm[];
-    const AnnealJob job = uniform_copy(jobs ? jobs[blockIdx.x] : single);
-    const int lane = threadIdx.x;
-    const int32_t gw = job.grid_w, gh = job.grid_h;
-    const int32_t cells = gw * gh;
-    const int32_t stamps = kHbm ? kHashStamps : stamp_words(cells);
-    const int32_t stamp_cells = kHbm ? kHashStamps : cells;  // words cleared between uses
-    uint32_t* stamp = sm;
-    auto sidx = [&](int32_t p) { return kHbm ? (p & (kHashStamps - 1)) : p; };
-    float* pack_s = reinterpret_cast<float*>(sm + stamps);
-    uint32_t* ring_xy1 = sm + stamps + kPackWords;
-    uint32_t* ring_xy2 = ring_xy1 + kRing;
-    float* ring_u = reinterpret_cast<float*>(ring_xy2 + kRing);
-    HbmGrid hbm{job.grid};
-    auto grid_s = [&]() {
-        if constexpr (kHbm)
-            return &hbm;
-        else
-            return reinterpret_cast<G*>(sm + stamps + kPackWords + kRingWords);
-    }();
+// LDS in words, behind the stamps: Labs of the swaps' materials (64 of the
+// first, 64 of the second), the terms (4 waves x 64 x {m1 with a, m2 with a,
+// m1 with b, m2 with b} for the wave's neighbours a, b), the mutual terms,
+// two rounds' accepted deltas, the ring, control words, the grid, the
+// library's Labs (where they fit).
+constexpr int32_t kLabWords = 2 * 64 * 4, kTermWords = kSlotWaves * 64 * 4, kMutualWords = 64,
+                  kPackWords = 2 * 64, kCtrlWords = 8;
+constexpr int32_t kFixedWords =
+    kLabWords + kTermWords + kMutualWords + kPackWords + 3 * kRing + kCtrlWords;
+__host__ __device__ __forceinline__ int32_t grid_words(int32_t cells, int32_t kind) {
+    return kind == kAnnealHbm ? 0 : (kind == kAnnealNarrow ? (cells + 7) / 8 * 4 : (cells + 3) & ~3);
+}
 
-    if constexpr (!kHbm)
-        for (int32_t i = lane; i < cells; i += 64) grid_s[i] = (G)gload(job.grid, i);
-    __syncthreads();
+// The control words: what a round leaves for the next, then a run's results.
+enum { kCtrlRound = 0, kCtrlCost = 2, kCtrlBest = 3, kCtrlImproved = 4 };
+__device__ __forceinline__ uint32_t pack_round(int32_t advance, bool hopeful, int32_t accepted) {
+    return (uint32_t)advance | (hopeful ? 128u : 0u) | (uint32_t)accepted << 8;
+}
 
-    // the stamp words double as the cost scratch (2 terms per cell + padding)
-    const TermMatrix TM{job.term, job.n};
-    const TermLab TL{job.lab4};
-    float* cost_scratch = reinterpret_cast<float*>(stamp);
-    const int32_t chunk = (stamps / 2 - 1) & ~1;
-    float cost = job.term ? total_cost_wave(grid_s, gw, gh, TM, cost_scratch, chunk)
-                          : total_cost_wave(grid_s, gw, gh, TL, cost_scratch, chunk);
-    for (int32_t i = lane; i < stamp_cells; i += 64) stamp[i] = 0u;
-    __syncthreads();
+template <typename G>
+struct AnnealShared {
+    uint32_t* stamp;
+    float4* lab_m;     // [2][64]
+    float4* terms;     // [kSlotWaves][64]
+    float* mutual;     // [64]
+    float* pack;       // [2][64]
+    uint32_t *ring_xy1, *ring_xy2;
+    float* ring_u;
+    uint32_t* ctrl;
+    const float4* labs;  // nullptr: read from the job's table in memory
+    bool hashed;
+    __device__ __forceinline__ int32_t at(int32_t p) const {
+        return hashed ? p & (kHashStamps - 1) : p;
+    }
+};
 
-    const float initial = cost;
-    float best = cost;
-    int64_t improved = 0, accepted = 0, evaluated = 0, rounds = 0;
-    int64_t s = 0, kbase = 0;
+// How the waves follow the run, alike in each: the round's first proposal,
+// its number, how its prefix is found, and the deltas the last round left.
+struct Rounds {
+    int64_t s = 0;
     uint32_t tag = 1;
-    const int64_t max_iter = job.max_iter;
+    bool hopeful;
+    int32_t pending = 0;
+    __device__ __forceinline__ void next(const uint32_t* ctrl) {
+        const uint32_t v = (uint32_t)__builtin_amdgcn_readfirstlane((int32_t)ctrl[kCtrlRound]);
+        s += v & 127u;
+        hopeful = (v & 128u) != 0u;
+        pending = (int32_t)(v >> 8);
+        ++tag;
+    }
+};
 
-    // Proposal `it` is drawn once, in a block of 128 made by the whole wave
-    // (refill) a round or two before the round that first needs it; a round
-    // re-evaluating proposals after a conflict reads them again instead of
-    // drawing them again.  A round refills, while its term gathers are in
-    // flight, when fewer than 128 proposals past its window start are drawn;
-    // a round advances the window by at most 64, so the next window is
-    // always drawn.  A block never overwrites a slot of the round's window
-    // [s, s + 64): it fills [filled, filled + 128) with s + 64 <= filled <
-    // s + 128, inside [s + 64, s + 256).
-    int64_t filled = 0;
-    auto refill = [&]() {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int64_t j = filled + 64 * h + lane;
-            const uint32_t slot = (uint32_t)j & (kRing - 1);
-            uint32_t a = 0, b = 0;
-            float uj = 0.0f;
-            if (j < max_iter) {
-                a = (uint32_t)draw_range(job.seed, (uint64_t)j, 0, gw) |
-                    ((uint32_t)draw_range(job.seed, (uint64_t)j, 1, gh) << 16);
-                b = (uint32_t)draw_range(job.seed, (uint64_t)j, 2, gw) |
-                    ((uint32_t)draw_range(job.seed, (uint64_t)j, 3, gh) << 16);
-                if (!job.greedy) uj = draw_unit(job.seed, (uint64_t)j);
-            }
-            ring_xy1[slot] = a;
-            ring_xy2[slot] = b;
-            ring_u[slot] = uj;
-        }
-        filled += 128;
-    };
-    refill();
-    __syncthreads();  // other lanes' draws are read below
-    // The serial cost sum of a round's accepted deltas (packed in proposal
-    // order into pack_s, see below) runs in the next round, after that
-    // round's term gathers are requested, so it overlaps their latency; the
-    // last round's runs after the loop.  pend: the count waiting (-1: none).
-    int32_t pend = -1;
-    auto serial_sum = [&](int32_t n_acc) {
-        // Eight deltas at a time come back as two uniform 16-byte LDS reads,
-        // so the chain adds VGPRs (no lane reads into SGPRs between the adds).
-        const float4* pack4 = reinterpret_cast<const float4*>(pack_s);
-        if (job.greedy) {  // optimize_greedy counts every accepted swap
-            for (int32_t q = 0; q < n_acc; q += 8) {
-                const float4 u0 = pack4[q >> 2], u1 = pack4[(q >> 2) + 1];
-                const float v[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
-#pragma unroll
-                for (int i = 0; i < 8; ++i) cost = cost + v[i];
-            }
-            improved += n_acc;
-        } else {
-            uint32_t better_n = 0;
-            for (int32_t q = 0; q < n_acc; q += 8) {
-                const float4 u0 = pack4[q >> 2], u1 = pack4[(q >> 2) + 1];
-                const float v[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    cost = cost + v[i];
-                    better_n += cost < best ? 1u : 0u;
-                    best = __builtin_fminf(best, cost);
-                }
-            }
-            improved += better_n;
-        }
-    };
-    while (s < max_iter) {
-        const int64_t it = s + lane;
-        const bool active = it < max_iter;
+// Stamps of an old round look like this round's once the tags wrap.
+template <typename G>
+__device__ __forceinline__ void wrap_tags(const AnnealShared<G>& S, Rounds& R, int32_t words, int tid) {
+    if (R.tag < kTagEnd) return;
+    __syncthreads();
+    if (tid < 64 * kSlotWaves)
+        for (int32_t i = tid; i < words; i += 64 * kSlotWaves) S.stamp[i] = 0u;
+    R.tag = 1;
+    __syncthreads();
+}
+
+// End of a phase: this wave's LDS operations are complete, then all waves
+// meet.  (__syncthreads would also wait for loads in flight: the temperatures,
+// which are requested a phase before their use.)
+__device__ __forceinline__ void phase_end() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// The Labs of two neighbours and (waves 0 and 1) of one of the swap's
+// materials, requested together.
+template <typename G>
+__device__ __forceinline__ void load_labs(const AnnealJob& job, const AnnealShared<G>& S, int32_t a,
+                                          int32_t b, int32_t m, bool want_m, float4& la, float4& lb,
+                                          float4& lm) {
+    a = max(a, 0);
+    b = max(b, 0);
+    m = max(m, 0);
+    if (S.labs) {
+        la = S.labs[a];
+        lb = S.labs[b];
+        if (want_m) lm = S.labs[m];
+    } else {
+        la = gload4(job.lab4, a);
+        lb = gload4(job.lab4, b);
+        if (want_m) lm = gload4(job.lab4, m);
+    }
+}
+
+template <typename G, bool kHbm>
+__device__ __forceinline__ void slot_wave(const AnnealJob& job, const AnnealShared<G>& S, G* grid,
+                                          int w, int lane, Rounds R, int32_t words,
+                                          AnnealOut* out) {
+    const int32_t gw = job.grid_w, gh = job.grid_h;
+    const bool vertical = !(w & 1), second = w >= 2;
+    const int32_t step = vertical ? gw : 1, bound = vertical ? gh : gw;
+    const int64_t max_iter = job.max_iter;
+    int64_t kbase = 0, accepted = 0, evaluated = 0, rounds = 0;  // (wave 0's)
+    while (R.s < max_iter) {
+        wrap_tags(S, R, words, w * 64 + lane);
+        // ---- reads
+        const int64_t it = R.s + lane;
         const uint32_t slot = (uint32_t)it & (kRing - 1);
-        const uint32_t xy1 = ring_xy1[slot], xy2 = ring_xy2[slot];
-        // Every ring slot up to `filled` holds in-grid coordinates (zeros past
-        // max_iter), so all lanes read both cells and their neighbour slots
-        // at once, before the skip test.
+        const uint32_t xy1 = S.ring_xy1[slot], xy2 = S.ring_xy2[slot];
         const int32_t x1 = (int32_t)(xy1 & 0xffffu), y1 = (int32_t)(xy1 >> 16);
         const int32_t x2 = (int32_t)(xy2 & 0xffffu), y2 = (int32_t)(xy2 >> 16);
-        const int32_t m1 = gget(grid_s, y1 * gw + x1), m2 = gget(grid_s, y2 * gw + x2);
-        int32_t nb[8];
-        swap_slots(grid_s, gw, gh, x1, y1, x2, y2, nb);
-        const bool skip = !active || (x1 == x2 && y1 == y2) || m1 == kEmpty || m2 == kEmpty;
-        const uint64_t nonskip = wave_ballot(!skip);
-        // every lane requests its swap's terms (a skipped lane those of
-        // material 0, which exists when any lane is not skipped), then the
-        // temperature and the uniform draw; the draws of later proposals and
-        // the previous round's serial sum run while they are in flight
-        SwapTerms st;
-        if (nonskip) {
-            const int32_t g1 = skip ? 0 : m1, g2 = skip ? 0 : m2;
-            if (job.term)
-                swap_terms(gw, gh, TM, x1, y1, x2, y2, g1, g2, nb, st);
-            else
-                swap_terms(gw, gh, TL, x1, y1, x2, y2, g1, g2, nb, st);
-        }
-        float temp = 1.0f, u = 0.0f;
-        if (!skip && !job.greedy) {
-            temp = gload(job.temps, kbase + lanes_before(nonskip));
-            u = ring_u[slot];
-        }
-        if (filled < s + 128) refill();  // read from the next round on, after its barriers
-        if (pend >= 0) serial_sum(pend);
-        float delta = 0.0f;
-        bool acc = false;
-        if (!skip) {
-            delta = m1 == m2 ? 0.0f : swap_sum(st);  // swap_delta_core's value
-            if (job.greedy) {
-                acc = delta < 0.0f;
-            } else if (delta < 0.0f) {
-                acc = true;
-            } else {
-                // Metropolis test u < exp(x), x = -delta/T (src/optimizer.rs:77-84).
-                // An estimate from the hardware reciprocal and exp2 is within
-                // 2^-15 of exp(x), relative, down to 2^-126 (below, it may be 0,
-                // and u is either 0 or at least 2^-24), so it decides alone
-                // unless u lies within 2^-10 of it (or it is 0 or not finite);
-                // those lanes compute x and exp exactly.
-                const float e = __builtin_amdgcn_exp2f(-delta * __builtin_amdgcn_rcpf(temp) *
-                                                       1.44269504f);
-                if (__builtin_fabsf(u - e) > e * (1.0f / 1024.0f))
-                    acc = u < e;
-                else
-                    acc = u < exp_f32(-delta / temp);
-            }
-        }
         const int32_t p1 = y1 * gw + x1, p2 = y2 * gw + x2;
-        const uint32_t mine = (tag << 6) | (uint32_t)(63 - lane);
-        if (acc) {
-            atomicMax(&stamp[sidx(p1)], mine);
-            atomicMax(&stamp[sidx(p2)], mine);
+        const int32_t centre = second ? p2 : p1, partner = second ? p1 : p2;
+        const int32_t along = vertical ? (second ? y2 : y1) : (second ? x2 : x1);
+        const bool in_a = along > 0, in_b = along < bound - 1;
+        // a neighbour outside the grid reads its own cell, always in bounds
+        const int32_t qa = in_a ? centre - step : centre, qb = in_b ? centre + step : centre;
+        const int32_t m1 = gget(grid, p1), m2 = gget(grid, p2);
+        const int32_t a = gget(grid, qa), b = gget(grid, qb);
+        const bool skip = it >= max_iter || p1 == p2 || m1 == kEmpty || m2 == kEmpty;
+        float4 la = make_float4(0, 0, 0, 0), lb = la, lm = la;
+        if (job.n > 0) load_labs(job, S, a, b, w == 0 ? m1 : m2, w < 2, la, lb, lm);
+        uint64_t nonskip = 0;
+        float temp = 1.0f, u = 0.0f;
+        const uint32_t mine = (R.tag << 7) | ((uint32_t)(63 - lane) << 1);
+        if (w == 0) {
+            nonskip = wave_ballot(!skip);
+            if (!skip) {
+                if (R.hopeful) {
+                    atomicMax(&S.stamp[S.at(p1)], mine);
+                    atomicMax(&S.stamp[S.at(p2)], mine | 1u);
+                }
+                if (!job.greedy) {
+                    temp = gload(job.temps, kbase + lanes_before(nonskip));
+                    u = S.ring_u[slot];
+                }
+            }
         }
-        __syncthreads();
-        bool conflict = false;
-        if (!skip) {
-            // read set: both cells and their in-grid neighbours, as ten fixed
-            // slots (an out-of-grid neighbour re-reads its own cell, which is
-            // checked anyway), so the reads are issued together
-            const int32_t q[10] = {p1,
-                                   p2,
-                                   y1 > 0 ? p1 - gw : p1,
-                                   y1 < gh - 1 ? p1 + gw : p1,
-                                   x1 > 0 ? p1 - 1 : p1,
-                                   x1 < gw - 1 ? p1 + 1 : p1,
-                                   y2 > 0 ? p2 - gw : p2,
-                                   y2 < gh - 1 ? p2 + gw : p2,
-                                   x2 > 0 ? p2 - 1 : p2,
-                                   x2 < gw - 1 ? p2 + 1 : p2};
+        if (w < 2) S.lab_m[w * 64 + lane] = lm;
+        phase_end();
+        // ---- terms
+        const float4 l1 = S.lab_m[lane], l2 = S.lab_m[64 + lane];
+        int32_t first = 64;
+        if (R.hopeful) {
+            const uint32_t va = S.stamp[S.at(qa)], vb = S.stamp[S.at(qb)];
+            if (w == 0) {
+                const uint32_t v1 = S.stamp[S.at(p1)], v2 = S.stamp[S.at(p2)];
+                const bool taken = !skip && ((v1 >> 1) != (mine >> 1) || (v2 >> 1) != (mine >> 1));
+                const uint64_t t = wave_ballot(taken);
+                first = t ? __ffsll((unsigned long long)t) - 1 : 64;
+            }
+            // stamped in this round by a lower lane: above this lane's stamps
+            bool sub_a = va > (mine | 1u), sub_b = vb > (mine | 1u);
+            if (wave_ballot(sub_a || sub_b)) {
+                const int32_t ka = 63 - (int32_t)((va >> 1) & 63u), kb = 63 - (int32_t)((vb >> 1) & 63u);
+                uint32_t ca = va & 1u, cb = vb & 1u;  // which of k's cells
+                if (S.hashed) {
+                    auto which = [&](int32_t k, int32_t q, bool& sub) {
+                        const uint32_t ks = (uint32_t)(R.s + k) & (kRing - 1);
+                        const uint32_t k1 = S.ring_xy1[ks], k2 = S.ring_xy2[ks];
+                        const bool is1 = (int32_t)(k1 >> 16) * gw + (int32_t)(k1 & 0xffffu) == q;
+                        const bool is2 = (int32_t)(k2 >> 16) * gw + (int32_t)(k2 & 0xffffu) == q;
+                        sub = sub && (is1 || is2);
+                        return is1 ? 0u : 1u;
+                    };
+                    ca = which(ka, qa, sub_a);
+                    cb = which(kb, qb, sub_b);
+                }
+                // k's first cell gets its second material, and the reverse
+                const float4 na = S.lab_m[(ca ? 0 : 64) + ka], nb = S.lab_m[(cb ? 0 : 64) + kb];
+                la = make_float4(sub_a ? na.x : la.x, sub_a ? na.y : la.y, sub_a ? na.z : la.z, 0.0f);
+                lb = make_float4(sub_b ? nb.x : lb.x, sub_b ? nb.y : lb.y, sub_b ? nb.z : lb.z, 0.0f);
+            }
+        }
+        const bool self_a = in_a && qa == partner, self_b = in_b && qb == partner;
+        const bool ok_a = in_a && !self_a && a != kEmpty, ok_b = in_b && !self_b && b != kEmpty;
+        const float t1a = adj_term(l1, la), t2a = adj_term(l2, la);
+        const float t1b = adj_term(l1, lb), t2b = adj_term(l2, lb);
+        S.terms[w * 64 + lane] = make_float4(ok_a ? t1a : 0.0f, ok_a ? t2a : 0.0f,
+                                             ok_b ? t1b : 0.0f, ok_b ? t2b : 0.0f);
+        // the partner as a neighbour of the first cell: the mutual term
+        if (!second && (self_a || self_b)) S.mutual[lane] = self_a ? t1a : t1b;
+        phase_end();
+        // ---- decisions
+        if (w == 0) {
+            const float4 v0 = S.terms[lane], v1 = S.terms[64 + lane], v2 = S.terms[128 + lane],
+                         v3 = S.terms[192 + lane];
+            const bool adjacent = p1 - p2 == gw || p2 - p1 == gw || (y1 == y2 && (x1 - x2 == 1 || x2 - x1 == 1));
+            // the first cell's neighbours: old with m1, new with m2; the second's the reverse
+            float old_cost = v0.x, new_cost = v0.y;
+            old_cost += v0.z;
+            new_cost += v0.w;
+            old_cost += v1.x;
+            new_cost += v1.y;
+            old_cost += v1.z;
+            new_cost += v1.w;
+            old_cost += v2.y;
+            new_cost += v2.x;
+            old_cost += v2.w;
+            new_cost += v2.z;
+            old_cost += v3.y;
+            new_cost += v3.x;
+            old_cost += v3.w;
+            new_cost += v3.z;
+            if (adjacent) {
+                const float t = S.mutual[lane];
+                old_cost += t;
+                new_cost += t;
+            }
+            const float delta = m1 == m2 ? 0.0f : new_cost - old_cost;
+            bool acc = false;
+            if (!skip) {
+                if (delta < 0.0f) {
+                    acc = true;
+                } else if (!job.greedy) {
+                    // Metropolis test u < exp(x), x = -delta/T (src/optimizer.rs:77-84).
+                    // An estimate from the hardware reciprocal and exp2 is within
+                    // 2^-15 of exp(x), relative, down to 2^-126 (below, it may be 0,
+                    // and u is either 0 or at least 2^-24), so it decides alone
+                    // unless u lies within 2^-10 of it (or it is 0 or not finite);
+                    // those lanes compute x and exp exactly.
+                    const float e = __builtin_amdgcn_exp2f(-delta * __builtin_amdgcn_rcpf(temp) *
+                                                           1.44269504f);
+                    if (__builtin_fabsf(u - e) > e * (1.0f / 1024.0f))
+                        acc = u < e;
+                    else
+                        acc = u < exp_f32(-delta / temp);
+                }
+            }
+            const int64_t remain = max_iter - R.s;
+            if ((int64_t)first > remain) first = (int32_t)remain;
+            const uint64_t acc_all = wave_ballot(acc);
+            const uint64_t below = first >= 64 ? ~0ull : (1ull << first) - 1ull;
+            const uint64_t rejected = nonskip & ~acc_all & below;
+            if (!R.hopeful || rejected) {
+                if (!R.hopeful && acc) {
+                    atomicMax(&S.stamp[S.at(p1)], mine);
+                    atomicMax(&S.stamp[S.at(p2)], mine);
+                }
+                // (one wave's LDS operations are done in order)
+                asm volatile("" ::: "memory");
+                const int32_t q[8] = {y1 > 0 ? p1 - gw : p1, y1 < gh - 1 ? p1 + gw : p1,
+                                      x1 > 0 ? p1 - 1 : p1,  x1 < gw - 1 ? p1 + 1 : p1,
+                                      y2 > 0 ? p2 - gw : p2, y2 < gh - 1 ? p2 + gw : p2,
+                                      x2 > 0 ? p2 - 1 : p2,  x2 < gw - 1 ? p2 + 1 : p2};
+                bool conflict = false;
 #pragma unroll
-            for (int i = 0; i < 10; ++i) {
-                const uint32_t v = stamp[sidx(q[i])];
-                conflict |= (v >> 6) == tag && (int)(63 - (v & 63u)) < lane;
+                for (int i = 0; i < 8; ++i) {
+                    const uint32_t v = S.stamp[S.at(q[i])];
+                    const int32_t k = 63 - (int32_t)((v >> 1) & 63u);
+                    conflict |= v > (mine | 1u) && (!R.hopeful || ((rejected >> k) & 1ull) != 0ull);
+                }
+                if (!R.hopeful)
+                    conflict |= S.stamp[S.at(p1)] > (mine | 1u) || S.stamp[S.at(p2)] > (mine | 1u);
+                const uint64_t c = wave_ballot(conflict && !skip);
+                first = min(first, c ? __ffsll((unsigned long long)c) - 1 : 64);
             }
-        }
-        const uint64_t cmask = wave_ballot(conflict);
-        int32_t first = cmask ? (__ffsll((unsigned long long)cmask) - 1) : 64;
-        const int64_t remain = max_iter - s;
-        if ((int64_t)first > remain) first = (int32_t)remain;
-        const uint64_t commit = first >= 64 ? ~0ull : ((1ull << first) - 1ull);
-        const uint64_t accmask = wave_ballot(acc) & commit;
-        __syncthreads();
-        if (lane < first) {
-            if (acc) {
-                // no lower lane of this round wrote p1 or p2 (that would be a
-                // conflict), so the round-start reads m1, m2 are still current
-                gput(grid_s, p1, m2);
-                gput(grid_s, p2, m1);
+            const uint64_t commit = first >= 64 ? ~0ull : (1ull << first) - 1ull;
+            const uint64_t accmask = acc_all & commit;
+            if (lane_in(accmask)) {
+                // no lower lane of this round wrote p1 or p2
+                gput(grid, p1, m2);
+                gput(grid, p2, m1);
             }
-            if (job.trace_delta) gstore(job.trace_delta, it, skip ? __int_as_float(0x7fc00000) : delta);
-            if (job.trace_accept) gstore(job.trace_accept, it, (uint8_t)(acc ? 1 : 0));
+            if (lane < first) {
+                if (job.trace_delta) gstore(job.trace_delta, it, skip ? __int_as_float(0x7fc00000) : delta);
+                if (job.trace_accept) gstore(job.trace_accept, it, (uint8_t)(acc ? 1 : 0));
+            }
+            // an HBM grid's swaps are complete at agent scope before the next
+            // round's reads (the barrier below orders the waves)
+            if constexpr (kHbm) __threadfence();
+            // the accepted deltas in proposal order, +0.0 past the last
+            float* const pack = S.pack + (R.tag & 1u) * 64;
+            const int32_t n_acc = __popcll(accmask), n_ev = __popcll(nonskip & commit);
+            pack[lane] = 0.0f;
+            if (lane_in(accmask)) pack[lanes_before(accmask)] = delta;
+            if (lane == 0)
+                S.ctrl[kCtrlRound] = pack_round(first, !job.greedy && 9 * n_acc > 5 * n_ev, n_acc);
+            accepted += n_acc;
+            evaluated += n_ev;
+            kbase += n_ev;
+            ++rounds;
         }
-        // an HBM grid's swaps are complete at agent scope before the next
-        // round's reads (the barriers below order the lanes)
-        if constexpr (kHbm) __threadfence();
-        // Running cost in proposal order (f32, as the reference's
-        // `current_cost += delta`).  The committed accepted deltas are packed
-        // into words 0..n-1 of pack_s in proposal order (the other words hold
-        // +0.0; pack_s is 16-byte aligned), so the serial sum reads them by a
-        // counter instead of walking the mask.  Every lane runs the same
-        // uniform loop, so cost / best / improved stay identical across the
-        // wave.  Adding a +0.0 past the last delta changes nothing: the cost is
-        // never -0.0 and never below best.  best = fminf(best, cost) equals
-        // `cost < best ? cost : best` here (no NaN, no -0.0) and keeps the
-        // compare off the dependent chain.
-        pack_s[lane] = 0.0f;
-        if (lane_in(accmask)) pack_s[lanes_before(accmask)] = delta;
-        __syncthreads();  // other lanes' writes, not this lane's own stores, are read next round
-        pend = __popcll(accmask);
-        accepted += __popcll(accmask);
-        const int64_t ev = __popcll(nonskip & commit);
-        evaluated += ev;
-        kbase += ev;
-        s += first;
-        ++rounds;
-        ++tag;
-        if (tag >= (1u << 26)) {
-            __syncthreads();
-            for (int32_t i = lane; i < stamp_cells; i += 64) stamp[i] = 0u;
-            tag = 1;
-        }
-        __syncthreads();
+        phase_end();
+        R.next(S.ctrl);
     }
+    if (w == 0) {
+        out->accepted = accepted;
+        out->evaluated = evaluated;
+        out->rounds = rounds;
+    }
+}
 
-    if (pend >= 0) serial_sum(pend);
+// The draw waves: in a round that starts with proposals up to `filled` drawn,
+// the block of 64 behind them, one draw after the decisions phase has begun
+// and one in the next round's first phase (when this SIMD's slot wave has
+// least to do).  filled >= s + 128 holds in every round when its decisions
+// start (the next window ends there at the latest), and a block is only
+// drawn where it overwrites slots before s (filled <= s + 192).
+template <typename G>
+__device__ __forceinline__ void draw_wave(const AnnealJob& job, const AnnealShared<G>& S, int w,
+                                          int lane, Rounds R, int32_t words) {
+    const uint32_t k = w == kDraw1Wave ? 0u : 2u;
+    uint32_t* const ring = w == kDraw1Wave ? S.ring_xy1 : S.ring_xy2;
+    int64_t filled = kRing;
+    bool drawing = false;
+    uint32_t x = 0;
+    while (R.s < job.max_iter) {
+        wrap_tags(S, R, words, w * 64 + lane);
+        if (drawing) {
+            const uint64_t j = (uint64_t)(filled - 64 + lane);
+            ring[j & (kRing - 1)] = x | (uint32_t)draw_range(job.seed, j, k + 1, job.grid_h) << 16;
+        }
+        phase_end();
+        phase_end();
+        drawing = filled <= R.s + kRing - 64;
+        if (drawing) {
+            x = (uint32_t)draw_range(job.seed, (uint64_t)(filled + lane), k, job.grid_w);
+            filled += 64;
+        }
+        phase_end();
+        R.next(S.ctrl);
+    }
+}
 
+// The running cost: the accepted deltas of a round, packed in proposal order,
+// added in the next round.  As in sum_in_order, the 64 sums are those of the
+// deltas rounded to the cost's ulp as long as none is half way and the cost
+// stays strictly inside its binade; their prefix sums come from one scan.
+// Otherwise one dependent addition after another.
+struct CostSum {
+    float cost, best;
+    int64_t improved = 0;
+    __device__ __forceinline__ void add(const float* pack, int32_t n_acc, bool greedy, int lane) {
+        const float d = pack[lane];
+        const uint32_t bits = __float_as_uint(cost), exponent = bits >> 23;
+        if (greedy) improved += n_acc;  // optimize_greedy counts every accepted swap
+        if (exponent >= 23 && exponent < 250) {
+            const float f = d * __uint_as_float((277u - exponent) << 23);
+            const float r = __builtin_rintf(f);
+            const bool plain = __builtin_fabsf(f) <= 4194304.0f && __builtin_fabsf(f - r) != 0.5f;
+            int32_t m = (int32_t)r;
+            // inclusive sums over the lanes: within rows of 16, then over rows
+            m += __builtin_amdgcn_update_dpp(0, m, 0x111, 0xF, 0xF, false);
+            m += __builtin_amdgcn_update_dpp(0, m, 0x112, 0xF, 0xF, false);
+            m += __builtin_amdgcn_update_dpp(0, m, 0x114, 0xF, 0xF, false);
+            m += __builtin_amdgcn_update_dpp(0, m, 0x118, 0xF, 0xF, false);
+            m += __builtin_amdgcn_update_dpp(0, m, 0x142, 0xA, 0xF, false);
+            m += __builtin_amdgcn_update_dpp(0, m, 0x143, 0xC, 0xF, false);
+            m += (int32_t)((bits & 0x7fffffu) | 0x800000u);
+            if (!wave_ballot(!plain || m <= 0x800000 || m >= 0x1000000)) {
+                const float c = __uint_as_float((bits & 0xff800000u) | ((uint32_t)m & 0x7fffffu));
+                if (!greedy && wave_ballot(c < best)) {
+                    // new bests: below the best before the round and all
+                    // sums before it (floats of one sign order like their bits)
+                    const uint32_t low = min(__float_as_uint(c), __float_as_uint(best));
+                    uint32_t p = low;
+                    for (int k = 1; k < 64; k <<= 1) {
+                        const uint32_t o = (uint32_t)__shfl_up((int)p, k, 64);
+                        p = lane >= k ? min(p, o) : p;
+                    }
+                    const uint32_t before = (uint32_t)__shfl_up((int)p, 1, 64);
+                    const bool record = lane == 0 ? c < best : __float_as_uint(c) < before;
+                    improved += __popcll(wave_ballot(record));
+                    best = readlane_f(__uint_as_float(p), 63);
+                }
+                cost = readlane_f(c, 63);
+                return;
+            }
+        }
+        const float4* pack4 = reinterpret_cast<const float4*>(pack);
+        uint32_t better = 0;
+        for (int32_t q = 0; q < n_acc; q += 8) {
+            const float4 u0 = pack4[q >> 2], u1 = pack4[(q >> 2) + 1];
+            const float v[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
+            // Adding a +0.0 past the last delta changes nothing.  best =
+            // fminf(best, cost) equals `cost < best ? cost : best` here (no
+            // NaN, no -0.0) and keeps the compare off the dependent chain.
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                cost = cost + v[i];
+                better += cost < best ? 1u : 0u;
+                best = __builtin_fminf(best, cost);
+            }
+        }
+        if (!greedy) improved += better;
+    }
+};
+
+// The cost wave; it also draws u for the draw waves' blocks.
+template <typename G>
+__device__ __forceinline__ void cost_wave(const AnnealJob& job, const AnnealShared<G>& S, int lane,
+                                          Rounds R, int32_t words) {
+    CostSum C;
+    C.cost = C.best = __uint_as_float(uniform_copy(S.ctrl[kCtrlCost]));
+    int64_t filled = kRing;
+    bool drawing = false;
+    while (R.s < job.max_iter) {
+        wrap_tags(S, R, words, kCostWave * 64 + lane);
+        if (drawing) {
+            const uint64_t j = (uint64_t)(filled - 64 + lane);
+            S.ring_u[j & (kRing - 1)] = draw_unit(job.seed, j);
+        }
+        phase_end();
+        if (R.pending) C.add(S.pack + ((R.tag - 1) & 1u) * 64, R.pending, job.greedy != 0, lane);
+        phase_end();
+        drawing = filled <= R.s + kRing - 64;
+        if (drawing) filled += 64;
+        phase_end();
+        R.next(S.ctrl);
+    }
+    if (R.pending) C.add(S.pack + ((R.tag - 1) & 1u) * 64, R.pending, job.greedy != 0, lane);
+    if (lane == 0) {
+        S.ctrl[kCtrlCost] = __float_as_uint(C.cost);
+        S.ctrl[kCtrlBest] = __float_as_uint(C.best);
+        reinterpret_cast<int64_t*>(S.ctrl)[kCtrlImproved / 2] = C.improved;
+    }
+}
+
+// kHbm: the grid stays in HBM (the job's own grid, swapped in place), for
+// grids too large for LDS.
+template <typename G, bool kHbm>
+__global__ __launch_bounds__(kAnnealThreads) void anneal_kernel(AnnealJob single,
+                                                                const AnnealJob* __restrict__ jobs) {
+    extern __shared__ __align__(16) uint32_t sm[];
+    const AnnealJob job = uniform_copy(jobs ? jobs[blockIdx.x] : single);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int32_t cells = job.grid_w * job.grid_h;
+    const int32_t words = stamp_words(cells);
+    typedef typename std::conditional<kHbm, HbmGrid, G>::type Grid;
+    AnnealShared<Grid> S;
+    S.stamp = sm;
+    S.lab_m = reinterpret_cast<float4*>(sm + words);
+    S.terms = S.lab_m + 2 * 64;
+    S.mutual = reinterpret_cast<float*>(S.terms + kSlotWaves * 64);
+    S.pack = S.mutual + kMutualWords;
+    S.ring_xy1 = reinterpret_cast<uint32_t*>(S.pack + kPackWords);
+    S.ring_xy2 = S.ring_xy1 + kRing;
+    S.ring_u = reinterpret_cast<float*>(S.ring_xy2 + kRing);
+    S.ctrl = S.ring_xy2 + 2 * kRing;
+    S.hashed = cells > kHashStamps;
+    uint32_t* const grid_at = sm + words + kFixedWords;
+    const int32_t kind = kHbm ? kAnnealHbm : sizeof(G) == 2 ? kAnnealNarrow : kAnnealWide;
+    float4* const labs = reinterpret_cast<float4*>(grid_at + grid_words(cells, kind));
+    S.labs = job.labs_in_lds ? labs : nullptr;
+    HbmGrid hbm{job.grid};
+    Grid* grid;
+    if constexpr (kHbm) {
+        grid = &hbm;
+    } else {
+        grid = reinterpret_cast<G*>(grid_at);
+        for (int32_t i = tid; i < cells; i += kAnnealThreads) grid[i] = (G)gload(job.grid, i);
+    }
+    if (S.labs)
+        for (int32_t i = tid; i < job.n; i += kAnnealThreads) labs[i] = gload4(job.lab4, i);
+    // the first proposals (coordinates are in the grid past max_iter too)
+    if (tid < kRing) {
+        S.ring_xy1[tid] = (uint32_t)draw_range(job.seed, tid, 0, job.grid_w) |
+                          (uint32_t)draw_range(job.seed, tid, 1, job.grid_h) << 16;
+        S.ring_xy2[tid] = (uint32_t)draw_range(job.seed, tid, 2, job.grid_w) |
+                          (uint32_t)draw_range(job.seed, tid, 3, job.grid_h) << 16;
+        S.ring_u[tid] = draw_unit(job.seed, tid);
+    }
+    __syncthreads();
+    float* const scratch = reinterpret_cast<float*>(S.stamp);
+    const int32_t chunk = (words / 2 - 1) & ~1;
+    const float initial =
+        S.labs ? total_cost_block(grid, job.grid_w, job.grid_h, TermLds{S.labs}, scratch, chunk)
+               : total_cost_block(grid, job.grid_w, job.grid_h, TermLab{job.lab4}, scratch, chunk);
+    for (int32_t i = tid; i < words; i += kAnnealThreads) S.stamp[i] = 0u;
+    if (tid == 0) S.ctrl[kCtrlCost] = __float_as_uint(initial);
+    __syncthreads();
+
+    Rounds R;
+    R.hopeful = !job.greedy;
+    AnnealOut r{};
+    if (w < kSlotWaves)
+        slot_wave<Grid, kHbm>(job, S, grid, w, lane, R, words, &r);
+    else if (w == kDraw1Wave || w == kDraw2Wave)
+        draw_wave(job, S, w, lane, R, words);
+    else if (w == kCostWave)
+        cost_wave(job, S, lane, R, words);
+    else
+        return;
+    __syncthreads();
     if constexpr (!kHbm)
-        for (int32_t i = lane; i < cells; i += 64) gstore(job.grid, i, (int32_t)grid_s[i]);
-    if (lane == 0 && job.result) {
-        AnnealOut r;
+        if (w < kSlotWaves)
+            for (int32_t i = tid; i < cells; i += 64 * kSlotWaves) gstore(job.grid, i, (int32_t)grid[i]);
+    if (tid == 0 && job.result) {
         r.initial_cost = initial;
-        r.final_cost = cost;
-        r.best_cost = job.greedy ? cost : best;
-        r.improved = improved;
-        r.accepted = accepted;
-        r.iterations = max_iter;
-        r.evaluated = evaluated;
-        r.rounds = rounds;
+        r.final_cost = __uint_as_float(S.ctrl[kCtrlCost]);
+        r.best_cost = job.greedy ? r.final_cost : __uint_as_float(S.ctrl[kCtrlBest]);
+        r.improved = reinterpret_cast<const int64_t*>(S.ctrl)[kCtrlImproved / 2];
+        r.iterations = job.max_iter;
         *job.result = r;
     }
 }
 
 int32_t anneal_kind(int32_t cells, int32_t n, int32_t gw, int32_t gh, size_t max_lds) {
-    if (n < 32768 && anneal_lds_bytes(cells, kAnnealNarrow) <= max_lds) return kAnnealNarrow;
-    if (anneal_lds_bytes(cells, kAnnealWide) <= max_lds) return kAnnealWide;
-    if (gw < 65536 && gh < 65536 && anneal_lds_bytes(cells, kAnnealHbm) <= max_lds)
+    if (n < 32768 && anneal_lds_bytes(cells, kAnnealNarrow, 0) <= max_lds) return kAnnealNarrow;
+    if (anneal_lds_bytes(cells, kAnnealWide, 0) <= max_lds) return kAnnealWide;
+    if (gw < 65536 && gh < 65536 && anneal_lds_bytes(cells, kAnnealHbm, 0) <= max_lds)
         return kAnnealHbm;
     return -1;
 }
 
-size_t anneal_lds_bytes(int32_t cells, int32_t kind) {
-    if (kind == kAnnealHbm)
-        return (size_t)(kHashStamps + kPackWords + kRingWords) * sizeof(uint32_t);
-    return (size_t)(stamp_words(cells) + kPackWords + kRingWords) * sizeof(uint32_t) +
-           (size_t)cells * (kind == kAnnealNarrow ? sizeof(int16_t) : sizeof(int32_t));
+size_t anneal_lds_bytes(int32_t cells, int32_t kind, int32_t labs) {
+    return sizeof(uint32_t) * ((size_t)stamp_words(cells) + kFixedWords + grid_words(cells, kind)) +
+           sizeof(float4) * (size_t)labs;
 }
 
 namespace {
 template <typename... A>
 void launch_anneal(int32_t kind, dim3 grid, size_t lds_bytes, hipStream_t stream, A... args) {
+    const dim3 threads(kAnnealThreads);
     if (kind == kAnnealNarrow)
-        hipLaunchKernelGGL((anneal_kernel<int16_t, false>), grid, dim3(64), lds_bytes, stream,
+        hipLaunchKernelGGL((anneal_kernel<int16_t, false>), grid, threads, lds_bytes, stream,
                            args...);
     else if (kind == kAnnealWide)
-        hipLaunchKernelGGL((anneal_kernel<int32_t, false>), grid, dim3(64), lds_bytes, stream,
+        hipLaunchKernelGGL((anneal_kernel<int32_t, false>), grid, threads, lds_bytes, stream,
                            args...);
     else
-        hipLaunchKernelGGL((anneal_kernel<int32_t, true>), grid, dim3(64), lds_bytes, stream,
+        hipLaunchKernelGGL((anneal_kernel<int32_t, true>), grid, threads, lds_bytes, stream,
                            args...);
 }
 }  // namespace
@@ -562,41 +799,37 @@ hipError_t anneal_configure(int max_lds) {
 }
 
 // ------------------------------------------------ cost / delta / penalty
-__global__ __launch_bounds__(64) void total_cost_kernel(const int32_t* __restrict__ grid,
+__global__ __launch_bounds__(kAnnealThreads) void total_cost_kernel(const int32_t* __restrict__ grid,
                                                         int32_t gw, int32_t gh,
                                                         const float4* __restrict__ lab4,
-                                                        const float* __restrict__ term, int32_t n,
                                                         float* __restrict__ scratch, int32_t chunk,
                                                         float* __restrict__ out) {
-    const float t = term ? total_cost_wave(grid, gw, gh, TermMatrix{term, n}, scratch, chunk)
-                         : total_cost_wave(grid, gw, gh, TermLab{lab4}, scratch, chunk);
+    const float t = total_cost_block(grid, gw, gh, TermLab{lab4}, scratch, chunk);
     if (threadIdx.x == 0) *out = t;
 }
 
 void launch_total_cost(const int32_t* grid, int32_t gw, int32_t gh, const float4* lab4,
-                       const float* term, int32_t n, float* scratch, int32_t chunk, float* out,
+                       float* scratch, int32_t chunk, float* out,
                        hipStream_t stream) {
-    hipLaunchKernelGGL(total_cost_kernel, dim3(1), dim3(64), 0, stream, grid, gw, gh, lab4, term, n,
+    hipLaunchKernelGGL(total_cost_kernel, dim3(1), dim3(kAnnealThreads), 0, stream, grid, gw, gh, lab4,
                        scratch, chunk, out);
 }
 
 __global__ void swap_delta_kernel(const int32_t* __restrict__ grid, int32_t gw, int32_t gh,
-                                  const float4* __restrict__ lab4, const float* __restrict__ term,
-                                  int32_t n, const int32_t* __restrict__ pairs, int32_t p,
+                                  const float4* __restrict__ lab4,
+                                  const int32_t* __restrict__ pairs, int32_t p,
                                   float* __restrict__ out) {
     const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= p) return;
     const int32_t* q = pairs + 4 * (int64_t)i;
-    out[i] = term ? swap_delta_dev(grid, gw, gh, TermMatrix{term, n}, q[0], q[1], q[2], q[3])
-                  : swap_delta_dev(grid, gw, gh, TermLab{lab4}, q[0], q[1], q[2], q[3]);
+    out[i] = swap_delta_dev(grid, gw, gh, TermLab{lab4}, q[0], q[1], q[2], q[3]);
 }
 
 void launch_swap_deltas(const int32_t* grid, int32_t gw, int32_t gh, const float4* lab4,
-                        const float* term, int32_t n, const int32_t* pairs, int32_t p, float* out,
-                        hipStream_t stream) {
+                        const int32_t* pairs, int32_t p, float* out, hipStream_t stream) {
     if (p <= 0) return;
     hipLaunchKernelGGL(swap_delta_kernel, dim3((p + 255) / 256), dim3(256), 0, stream, grid, gw, gh,
-                       lab4, term, n, pairs, p, out);
+                       lab4, pairs, p, out);
 }
 
 // calculate_penalty (src/adjacency.rs:63-88): Up, Down, Left, Right.

@@ -260,27 +260,6 @@ int run_place(mh_context* ctx, const mh_library* lib, const float* d_cell_lab, i
     return MH_OK;
 }
 
-int library_terms(const mh_library* clib, hipStream_t stream, const float** out) {
-    mh_library* lib = const_cast<mh_library*>(clib);
-    *out = nullptr;
-    if (lib->n == 0 || lib->n > kTermMatrixMaxN) return MH_OK;
-    std::lock_guard<std::mutex> g(lib->cache_mu);
-    if (!lib->d_term) {
-        float* t = nullptr;
-        HIPCHK(hipMalloc(&t, sizeof(float) * (size_t)lib->n * lib->n));
-        launch_term_full(lib->d_lab4, lib->n, t, stream);
-        hipError_t e = hipGetLastError();
-        if (e == hipSuccess) e = hipStreamSynchronize(stream);
-        if (e != hipSuccess) {
-            hipFree(t);
-            return fail(MH_ERR_HIP, "term matrix: %s", hipGetErrorString(e));
-        }
-        lib->d_term = t;
-    }
-    *out = lib->d_term;
-    return MH_OK;
-}
-
 // Resized tiles + their average RGB for cell size tw x th, cached per
 // library (the resize depends only on material and cell size).
 int library_tiles(const mh_library* clib, int32_t tw, int32_t th, hipStream_t stream,
@@ -353,9 +332,8 @@ int library_tiles_cached(const mh_library* clib, int32_t tw, int32_t th, const u
 }
 
 // temps_ready: the temperature table, already on the device (else the
-// context's cached table).  noalloc: allocate nothing -- the adjacency terms
-// come from the Lab table (bit-identical to the library's term matrix) and
-// temps_ready must be given whenever a proposal can read it.
+// context's cached table).  noalloc: allocate nothing -- temps_ready must be
+// given whenever a proposal can read it.
 int run_anneal(mh_context* ctx, const mh_library* lib, int32_t* d_grid, int32_t gw, int32_t gh,
                const mh_anneal_params* p, float* d_trace_delta, uint8_t* d_trace_accept,
                AnnealOut* d_out, const float* temps_ready, bool noalloc) {
@@ -364,7 +342,8 @@ int run_anneal(mh_context* ctx, const mh_library* lib, int32_t* d_grid, int32_t 
     if (kind < 0)
         return fail(MH_ERR_UNSUPPORTED, "annealing a %d x %d grid: a side of 65,536 or more", gw,
                     gh);
-    const size_t lds = anneal_lds_bytes(cells, kind);
+    const bool labs = anneal_lds_bytes(cells, kind, lib->n) <= ctx->max_lds;
+    const size_t lds = anneal_lds_bytes(cells, kind, labs ? lib->n : 0);
     const float* temps = temps_ready;
     int rc;
     if (!p->greedy && !temps && !noalloc) {
@@ -374,12 +353,10 @@ int run_anneal(mh_context* ctx, const mh_library* lib, int32_t* d_grid, int32_t 
     }
     if (!p->greedy && !temps && p->max_iterations > 0)
         return fail(MH_ERR_INVALID_ARGUMENT, "annealing without a temperature table");
-    const float* term = nullptr;
-    if (!noalloc && (rc = library_terms(lib, ctx->stream, &term))) return rc;
     AnnealJob job;
     job.lab4 = lib->d_lab4;
-    job.term = term;
     job.n = lib->n;
+    job.labs_in_lds = labs ? 1 : 0;
     job.grid = d_grid;
     job.grid_w = gw;
     job.grid_h = gh;
@@ -512,10 +489,9 @@ void library_release(mh_library* lib) {
     lib->d_pidx = nullptr;
     lib->d_box = nullptr;
     if (lib->d_sim) hipFree(lib->d_sim);
-    if (lib->d_term) hipFree(lib->d_term);
     if (lib->d_pixels) hipFree(lib->d_pixels);
     lib->d_lab4 = nullptr;
-    lib->d_L = lib->d_A = lib->d_B = lib->d_sim = lib->d_term = nullptr;
+    lib->d_L = lib->d_A = lib->d_B = lib->d_sim = nullptr;
     lib->d_pixels = nullptr;
     for (PixelGroup& g : lib->groups) {
         if (g.d_index) hipFree(g.d_index);
@@ -1310,10 +1286,7 @@ int mh_total_cost(mh_context* ctx, const mh_library* lib, const int32_t* grid, i
     CHK(upload(ctx, S_GRID, grid, (size_t)cells, &d_grid));
     CHK(slot(ctx, S_OUT0, (size_t)chunk * 2 + 4, &d_scratch));
     CHK(slot(ctx, S_OUT1, 1, &d_out));
-    const float* term = nullptr;
-    CHK(library_terms(lib, ctx->stream, &term));
-    launch_total_cost(d_grid, gw, gh, lib->d_lab4, term, lib->n, d_scratch, chunk, d_out,
-                      ctx->stream);
+    launch_total_cost(d_grid, gw, gh, lib->d_lab4, d_scratch, chunk, d_out, ctx->stream);
     HIPCHK(hipGetLastError());
     CHK(download(ctx, out, d_out, 1));
     return sync(ctx);
@@ -1364,9 +1337,7 @@ int mh_swap_deltas(mh_context* ctx, const mh_library* lib, const int32_t* grid, 
     CHK(upload(ctx, S_GRID, grid, (size_t)cells, &d_grid));
     CHK(upload(ctx, S_IN0, pairs, (size_t)p * 4, &d_pairs));
     CHK(slot(ctx, S_OUT0, (size_t)p, &d_out));
-    const float* term = nullptr;
-    CHK(library_terms(lib, ctx->stream, &term));
-    launch_swap_deltas(d_grid, gw, gh, lib->d_lab4, term, lib->n, d_pairs, p, d_out, ctx->stream);
+    launch_swap_deltas(d_grid, gw, gh, lib->d_lab4, d_pairs, p, d_out, ctx->stream);
     HIPCHK(hipGetLastError());
     CHK(download(ctx, out, d_out, (size_t)p));
     return sync(ctx);
@@ -1546,7 +1517,7 @@ __global__ __launch_bounds__(64) void temps_kernel(float t0, float decay, int64_
 }
 
 // generate_mosaic minus file I/O on the context stream into `b`.  noalloc:
-// no device allocation anywhere (no context scratch, term matrix, cached
+// no device allocation anywhere (no context scratch, cached
 // temperature table or tile build; no phase events).
 int enqueue_generate(mh_context* ctx, const mh_library* lib, const uint8_t* d_target, int32_t width,
                      int32_t height, const mh_job_params* p, const JobBufs& b,

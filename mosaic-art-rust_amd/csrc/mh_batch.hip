@@ -10,7 +10,7 @@
 // Every job's result is what mh_generate_device gives for it alone: the
 // kernels are the same and no state crosses jobs.
 //
-// The server keeps libraries resident (Lab table, term matrix, resized
+// The server keeps libraries resident (Lab table, resized
 // tiles), admits queued jobs while their device footprint fits a memory
 // budget, and launches what has been admitted as one batch on a free stream
 // slot; batches on different slots overlap on the device.  A scheduler
@@ -49,7 +49,6 @@ struct JobSpec {
     int32_t anneal_kind = 0;  // the annealing variant (mh::anneal_kind)
     bool place_hbm = false;   // placement state in HBM (library beyond LDS)
     float strength = 0.0f;
-    const float* term = nullptr;
     const float* temps = nullptr;
     const uint8_t* tiles = nullptr;
     const uint8_t* tile_avg = nullptr;
@@ -115,12 +114,11 @@ int check_job(const mh_context* ctx, const mh_job& j, JobSpec* s) {
     return MH_OK;
 }
 
-// Library-resident inputs of a job: term matrix, temperature table, resized
+// Library-resident inputs of a job: temperature table, resized
 // tiles (each built once, on `stream`).
 int prepare_job(mh_context* ctx, JobSpec* s, hipStream_t stream) {
     const mh_job_params& p = s->job.params;
     if (s->sa) {
-        CHK(library_terms(s->job.lib, stream, &s->term));
         CHK(get_temps(ctx, p.initial_temperature, p.temperature_decay, p.optimization_iterations,
                       &s->temps));
     }
@@ -286,8 +284,9 @@ int build_plan(const std::vector<JobSpec>& specs, const std::vector<uint8_t*>& j
         if (s.sa) {
             AnnealJob aj{};
             aj.lab4 = lib->d_lab4;
-            aj.term = s.term;
             aj.n = s.n;
+            const int32_t kind = s.anneal_kind;
+            aj.labs_in_lds = labs && anneal_lds_bytes(s.cells, kind, s.n) <= lib->ctx->max_lds ? 1 : 0;
             aj.grid = grid;
             aj.grid_w = s.gw;
             aj.grid_h = s.gh;
@@ -296,10 +295,9 @@ int build_plan(const std::vector<JobSpec>& specs, const std::vector<uint8_t*>& j
             aj.seed = j.params.seed;
             aj.greedy = 0;
             aj.result = d_aout + i;
-            const int32_t kind = s.anneal_kind;
             by_kind[kind].push_back(aj);
             job_of_kind[kind].push_back(i);
-            const size_t al = anneal_lds_bytes(s.cells, kind);
+            const size_t al = anneal_lds_bytes(s.cells, kind, aj.labs_in_lds ? s.n : 0);
             if (al > p->anneal_lds[kind]) p->anneal_lds[kind] = al;
         }
         // a13-a16: adjustments, composite

@@ -224,8 +224,22 @@ __device__ __forceinline__ float sq_distance(float ql, float qa, float qb, float
 
 // One adjacency term 1/(sim+1) (src/adjacency.rs:82, :110, :174).
 // get_similarity(i,i) = 0.0, which the distance formula also gives.
+//
+// The square root and the reciprocal are the hardware's estimates, each
+// corrected by a fused residual step (Markstein): equal to the correctly
+// rounded ones, without the scaling for ranges that cannot occur: the sum of
+// squares is raised to 2^-64 at least (the distance is then lost in the + 1
+// anyway), and an infinite one gives NaN and so the final max's 0.  Equal to
+// 1.0f / (sqrtf(d) + 1.0f) for every non-negative float d: all 2^31 were
+// compared on the device.  19 instructions for 45.
 __device__ __forceinline__ float adj_term(float4 p, float4 q) {
-    return 1.0f / (lab_distance(p, q) + 1.0f);
+    const float dl = p.x - q.x, da = p.y - q.y, db = p.z - q.z;
+    const float d = __builtin_fmaxf(dl * dl + da * da + db * db, 0x1p-64f);
+    const float r = __builtin_amdgcn_rsqf(d);
+    const float g = d * r;
+    const float x = __builtin_fmaf(__builtin_fmaf(-g, g, d), 0.5f * r, g) + 1.0f;
+    const float c = __builtin_amdgcn_rcpf(x);
+    return __builtin_fmaxf(__builtin_fmaf(__builtin_fmaf(-x, c, 1.0f), c, c), 0.0f);
 }
 
 // ----------------------------------------------------------- counter RNG
@@ -530,6 +544,17 @@ __device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
     v = v < t ? v : t;
     t = (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x143, 0xC, 0xF, false);
     v = v < t ? v : t;
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// Sum (mod 2^32) over the 64 lanes, the same way.
+__device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xF, 0xF, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xF, 0xF, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false);
     return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 

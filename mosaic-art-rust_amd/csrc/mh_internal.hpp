@@ -132,10 +132,9 @@ struct mh_library {
     float4* d_box = nullptr;
     int32_t nb = 0;
     float* d_sim = nullptr;    // n x n after build_similarities
-    float* d_term = nullptr;   // n x n 1/(sim+1), built on first use by the cost kernels
     uint8_t* d_pixels = nullptr;
     std::vector<PixelGroup> groups;  // materials grouped by size (empty: Labs only)
-    // lazily built device caches (term matrix, resized tiles per cell size)
+    // lazily built device caches (resized tiles per cell size)
     std::mutex cache_mu;
     std::map<std::pair<int32_t, int32_t>, mh::host::TileSet> tiles;
 };
@@ -163,11 +162,6 @@ MatBlocks library_blocks(const mh_library* lib);
 void batch_release(mh_batch* b);
 int get_temps(mh_context* ctx, float t0, float decay, int64_t len, const float** out);
 void fill_i32(int32_t* p, int64_t n, int32_t v, hipStream_t s);
-// Term matrix 1/(sim+1) of the library (nullptr above kTermMatrixMaxN
-// materials); built once on `stream`, which is then synchronised so any
-// stream may read it.
-constexpr int32_t kTermMatrixMaxN = 16384;
-int library_terms(const mh_library* lib, hipStream_t stream, const float** out);
 // Resized tiles + average RGB for cell size tw x th, built once on `stream`
 // (then synchronised).
 int library_tiles(const mh_library* lib, int32_t tw, int32_t th, hipStream_t stream,

@@ -49,10 +49,9 @@ struct AnnealOut {
     int64_t improved, accepted, iterations, evaluated, rounds;
 };
 
-// One annealing chain (one wave).
+// One annealing chain (one workgroup).
 struct AnnealJob {
     const float4* lab4;
-    const float* term;        // n x n adjacency terms, or nullptr (computed from lab4)
     int32_t n;
     int32_t* grid;            // cells, in/out
     int32_t grid_w, grid_h;
@@ -60,6 +59,7 @@ struct AnnealJob {
     const float* temps;       // temperature after k non-skipped proposals
     uint64_t seed;
     int32_t greedy;
+    int32_t labs_in_lds;      // LDS holds the library's Labs too
     float* trace_delta;       // optional, max_iter entries
     uint8_t* trace_accept;
     AnnealOut* result;
@@ -139,7 +139,6 @@ void launch_sim_full(const float4* lab, int32_t n, float* out, hipStream_t strea
 void launch_sim_packed(const float4* lab, int32_t n, float* out, hipStream_t stream);
 // lab[i].w = material i's largest adjacency term to another material.
 void launch_near_terms(float4* lab, int32_t n, hipStream_t stream);
-void launch_term_full(const float4* lab, int32_t n, float* out, hipStream_t stream);
 // out_idx / out_d / out_cand may be null.
 void launch_topk(const float* mL, const float* mA, const float* mB, int32_t n, const MatBlocks& blk,
                  const float* query, int32_t nq, int32_t k, int32_t* out_idx, float* out_d,
@@ -191,16 +190,15 @@ void launch_place_batch(const PlaceJob* d_jobs, int32_t n_jobs, bool raster, siz
 enum : int32_t { kAnnealNarrow = 0, kAnnealWide = 1, kAnnealHbm = 2 };
 // The first variant that holds the job in max_lds bytes of LDS, -1 if none.
 int32_t anneal_kind(int32_t cells, int32_t n, int32_t gw, int32_t gh, size_t max_lds);
-size_t anneal_lds_bytes(int32_t cells, int32_t kind);
+// labs: the Labs that LDS holds too (the library's, or 0).
+size_t anneal_lds_bytes(int32_t cells, int32_t kind, int32_t labs);
 void launch_anneal_single(const AnnealJob& job, int32_t kind, size_t lds_bytes, hipStream_t stream);
 void launch_anneal_batch(const AnnealJob* d_jobs, int32_t n_jobs, int32_t kind, size_t lds_bytes,
                          hipStream_t stream);
 void launch_total_cost(const int32_t* grid, int32_t gw, int32_t gh, const float4* lab4,
-                       const float* term, int32_t n, float* scratch, int32_t chunk, float* out,
-                       hipStream_t stream);
+                       float* scratch, int32_t chunk, float* out, hipStream_t stream);
 void launch_swap_deltas(const int32_t* grid, int32_t gw, int32_t gh, const float4* lab4,
-                        const float* term, int32_t n, const int32_t* pairs, int32_t p, float* out,
-                        hipStream_t stream);
+                        const int32_t* pairs, int32_t p, float* out, hipStream_t stream);
 void launch_penalties(const int32_t* grid, int32_t gw, int32_t gh, const float4* lab4, float weight,
                       const int32_t* queries, int32_t nq, float* out, hipStream_t stream);
 // n images of sw x sh (contiguous) -> dw x dh tiles; image m lands in tile
