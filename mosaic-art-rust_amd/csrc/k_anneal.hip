@@ -94,101 +94,207 @@ __device__ float swap_delta_dev(const int32_t* grid, int32_t gw, int32_t gh, con
     return new_cost - old_cost;
 }
 
-// s + t[0] + t[1] + ... + t[n - 1] in this order, each addition rounded to
-// f32, by one wave: s and every t are >= 0, t is 16-byte aligned and readable
-// to the next multiple of four, where it is +0.0 past n.
-//
-// One dependent addition after another takes 9 ns (its read included); 256
-// are done at once where their result is known to be the same.  While the
-// sum stays in one binade it is a whole multiple of the binade's ulp, and so
-// adding t adds t rounded to a multiple of the ulp, whatever the sum is --
-// unless t lies half way between two multiples, when the sum's last bit
-// decides.  The rounded terms are whole numbers of ulps, whose sum has no
-// order.  Blocks with a half-way term and blocks that leave the binade (the
-// first few hundred terms, mostly) are added one by one.
-__device__ float sum_in_order(float s, const float* t, int32_t n) {
-    const int lane = threadIdx.x & 63;
-    const float4* v = reinterpret_cast<const float4*>(t);
-    const int32_t n4 = (n + 3) / 4;
-    for (int32_t base = 0; base < n4; base += 64) {
-        const int32_t len = min(64, n4 - base);
-        float4 q = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (lane < len) q = v[base + lane];
-        const uint32_t bits = __float_as_uint(s), exponent = bits >> 23;
-        if (exponent >= 23 && exponent < 250) {
-            // 1 / ulp(s); the products are exact (those below the normal range are 0 here)
-            const float inv = __uint_as_float((277u - exponent) << 23);
-            const float f[4] = {q.x * inv, q.y * inv, q.z * inv, q.w * inv};
-            bool plain = true;
-            uint32_t sum = 0;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float r = __builtin_rintf(f[i]);
-                plain = plain && f[i] <= 4194304.0f && __builtin_fabsf(f[i] - r) != 0.5f;
-                sum += (uint32_t)r;
-            }
-            if (!wave_ballot(!plain)) {
-                const uint32_t m = ((bits & 0x7fffffu) | 0x800000u) + wave_sum_u32(sum);
-                if (m < 0x1000000u) {
-                    s = __uint_as_float((bits & 0xff800000u) | (m & 0x7fffffu));
-                    continue;
-                }
-            }
+// ------------------------------------------------------------ ordered sums
+// s + t[0] + t[1] + ... in this order, each addition rounded to f32.  One
+// dependent addition after another takes 10 ns (its read included), but most
+// results are known without: while the sum s stays in one binade it is a
+// whole number of the binade's ulps, and adding t adds t rounded to a whole
+// number of ulps, whatever s is -- unless t lies half way between two, when
+// the sum's last bit decides.  Whole numbers add in any order.
+struct Ulps {
+    uint32_t bits;
+    // s in the normal range, its ulp and 1 / ulp too; else one by one
+    __device__ __forceinline__ bool valid() const { return (bits >> 23) >= 23 && (bits >> 23) < 250; }
+    __device__ __forceinline__ float per_unit() const {  // 1 / ulp(s)
+        return __uint_as_float((277u - (bits >> 23)) << 23);
+    }
+    __device__ __forceinline__ int32_t count() const {
+        return (int32_t)((bits & 0x7fffffu) | 0x800000u);
+    }
+    // the float of m ulps, 2^23 <= m < 2^24
+    __device__ __forceinline__ float value(int32_t m) const {
+        return __uint_as_float((bits & 0xff800000u) | ((uint32_t)m & 0x7fffffu));
+    }
+};
+// f = t / ulp (exact but for what is rounded to 0 anyway): whether its whole
+// number is certain, and small enough that 256 of them fit 32 bits.
+__device__ __forceinline__ bool certain(float f, float r) {
+    return __builtin_fabsf(f) <= 4194304.0f && __builtin_fabsf(f - r) != 0.5f;
+}
+// Inclusive sums over the lanes: within rows of 16, then over the rows.
+__device__ __forceinline__ int32_t wave_scan_add(int32_t m) {
+    m += __builtin_amdgcn_update_dpp(0, m, 0x111, 0xF, 0xF, false);
+    m += __builtin_amdgcn_update_dpp(0, m, 0x112, 0xF, 0xF, false);
+    m += __builtin_amdgcn_update_dpp(0, m, 0x114, 0xF, 0xF, false);
+    m += __builtin_amdgcn_update_dpp(0, m, 0x118, 0xF, 0xF, false);
+    m += __builtin_amdgcn_update_dpp(0, m, 0x142, 0xA, 0xF, false);
+    m += __builtin_amdgcn_update_dpp(0, m, 0x143, 0xC, 0xF, false);
+    return m;
+}
+
+// Inclusive minima over the lanes, the same way (no NaN).
+__device__ __forceinline__ float wave_scan_min(float v) {
+#define MH_MIN_STEP(CTRL, ROWS)                                                                    \
+    v = __builtin_fminf(v, __int_as_float(__builtin_amdgcn_update_dpp(                             \
+                               __float_as_int(v), __float_as_int(v), CTRL, ROWS, 0xF, false)))
+    MH_MIN_STEP(0x111, 0xF);
+    MH_MIN_STEP(0x112, 0xF);
+    MH_MIN_STEP(0x114, 0xF);
+    MH_MIN_STEP(0x118, 0xF);
+    MH_MIN_STEP(0x142, 0xA);
+    MH_MIN_STEP(0x143, 0xC);
+#undef MH_MIN_STEP
+    return v;
+}
+
+// Adds the 64 lanes' t to s in lane order; returns each lane's sum (lane 63's
+// is the total, which s becomes).  A lane that is half way, or whose sum
+// leaves the inside of the binade, is added as it is, after the lanes below.
+__device__ __forceinline__ float add_lanes(float& s, float t, int lane) {
+    float c = s;
+    int done = -1;  // the last lane added
+    for (;;) {
+        const Ulps U{__float_as_uint(s)};
+        int32_t m = 0;
+        bool stop = true;
+        if (U.valid()) {
+            const float f = t * U.per_unit(), r = __builtin_rintf(f);
+            const bool sure = certain(f, r);
+            m = U.count() + wave_scan_add(sure ? (int32_t)r : 0);
+            stop = !sure || m <= 0x800000 || m >= 0x1000000;
         }
-        for (int32_t i = base; i < base + len; ++i) {
-            const float4 a = v[i];
-            s = s + a.x;
-            s = s + a.y;
-            s = s + a.z;
-            s = s + a.w;
+        // (a lane that adds nothing changes nothing)
+        const uint64_t at = wave_ballot(stop && t != 0.0f);
+        if (!at) {
+            if (lane > done) c = wave_ballot(t != 0.0f) ? U.value(m) : s;
+            s = readlane_f(c, 63);
+            return c;
+        }
+        const int l = __ffsll((unsigned long long)at) - 1;
+        const float v = lane > done && lane < l && U.valid() ? U.value(m) : s;
+        if (lane > done) c = v;
+        if (l > 0) s = readlane_f(c, l - 1);
+        s = s + readlane_f(t, l);
+        if (lane >= l) c = s;
+        if (lane <= l) t = 0.0f;
+        done = l;
+    }
+}
+
+// The total alone, for sums that start at 0, in whose first binades many terms
+// are half way: at once, or one by one (8 cycles each).
+__device__ __forceinline__ float sum_lanes(float s, float t) {
+    const Ulps U{__float_as_uint(s)};
+    if (U.valid()) {
+        const float f = t * U.per_unit(), r = __builtin_rintf(f);
+        if (!wave_ballot(!certain(f, r))) {
+            const uint32_t m = (uint32_t)U.count() + wave_sum_u32((uint32_t)r);
+            if (m < 0x1000000u) return U.value((int32_t)m);
         }
     }
+#pragma unroll
+    for (int i = 0; i < 64; ++i) s = s + readlane_f(t, i);
     return s;
 }
 
-// calculate_total_cost (src/adjacency.rs:91-130) by one workgroup: the terms
-// of `chunk` cells at a time are computed in parallel into scratch (right
-// term, down term per cell), then the first wave adds them in the reference's
-// order (raster, right before down).  An absent term is stored as +0.0: the
-// running sum starts at +0 and only grows, and x + (+0) == x bit for bit, so
-// adding it leaves the sum exactly as the reference's skipped addition does.
-// scratch holds 2*chunk + 2 floats and is 16-byte aligned.  The result is
-// returned to the first wave.
+// calculate_total_cost (src/adjacency.rs:91-130) by one workgroup of
+// kAnnealThreads, in the reference's order (raster, right before down).  An
+// absent term is added as +0.0: the running sum starts at +0 and only grows,
+// and x + (+0) == x bit for bit, so this equals skipping it.
+//
+// A wave takes 128 cells, two a lane, and rounds their 256 terms to the
+// sum's ulps; the waves' sums are added while they are certain and stay in
+// the binade.  Otherwise the wave whose turn it is adds its terms 64 at a time
+// or one by one, and the waves after it round theirs again.  (Some 10 to 20 times a
+// run: mostly the binades of the first few hundred terms.)  24,000 cells:
+// 50 us, 450 us one by one.  lds: kCostWords words, 16-byte aligned.
+// The result is returned to every wave.
+constexpr int32_t kCostWaves = 8, kCostWords = 256 + 2 * kCostWaves + 4;
+constexpr int32_t kAnnealThreads = 64 * kCostWaves;
+
 template <typename G, typename TS>
-__device__ float total_cost_block(const G* grid, int32_t gw, int32_t gh, const TS& T,
-                                  float* scratch, int32_t chunk) {
-    const int tid = threadIdx.x;
+__device__ float total_cost_block(const G* grid, int32_t gw, int32_t gh, const TS& T, uint32_t* lds) {
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    float* const strip = reinterpret_cast<float*>(lds);
+    uint32_t* const sums = lds + 256;                // two buffers of kCostWaves
+    uint32_t* const total = sums + 2 * kCostWaves;
     const int32_t cells = gw * gh;
-    float total = 0.0f;
-    for (int32_t base = 0; base < cells; base += chunk) {
-        const int32_t len = min(chunk, cells - base);
-        for (int32_t i = tid; i < len; i += blockDim.x) {
-            const int32_t c = base + i;
-            const int32_t x = c % gw, y = c / gw;
-            const int32_t m = gget(grid, c);
-            float tr = 0.0f, td = 0.0f;
+    constexpr uint32_t kUnsure = 0xffffffffu;
+    float s = 0.0f;
+    int buffer = 0;
+    constexpr int32_t kStep = 128 * kCostWaves;
+    const int32_t step_x = kStep % gw, step_y = kStep / gw;
+    const int32_t c0 = w * 128 + 2 * lane;
+    int32_t x0 = c0 % gw, y0 = c0 / gw;
+    for (int32_t base = 0; base < cells; base += kStep) {
+        const int32_t c = base + c0;
+        int32_t x = x0, y = y0;
+        x0 += step_x;
+        y0 += step_y + (x0 >= gw ? 1 : 0);
+        x0 -= x0 >= gw ? gw : 0;
+        float t[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int32_t p = c + i;
+            const int32_t m = p < cells ? gget(grid, p) : kEmpty;
             if (m != kEmpty) {
-                if (x < gw - 1) {
-                    const int32_t r = gget(grid, c + 1);
-                    if (r != kEmpty) tr = T(m, r);
-                }
-                if (y < gh - 1) {
-                    const int32_t d = gget(grid, c + gw);
-                    if (d != kEmpty) td = T(m, d);
+                const int32_t r = x < gw - 1 ? gget(grid, p + 1) : kEmpty;
+                const int32_t d = y < gh - 1 ? gget(grid, p + gw) : kEmpty;
+                if (r != kEmpty) t[2 * i] = T(m, r);
+                if (d != kEmpty) t[2 * i + 1] = T(m, d);
+            }
+            ++x;
+            if (x == gw) {
+                x = 0;
+                ++y;
+            }
+        }
+        for (int32_t done = 0; done < kCostWaves;) {
+            const Ulps U{__float_as_uint(s)};
+            bool sure = true;
+            uint32_t sum = 0;
+            const float inv = U.per_unit();
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float f = t[i] * inv, r = __builtin_rintf(f);
+                sure = sure && certain(f, r);
+                sum += (uint32_t)r;
+            }
+            if (!U.valid()) {  // sure of nothing but zeros
+                sure = t[0] == 0.0f && t[1] == 0.0f && t[2] == 0.0f && t[3] == 0.0f;
+                sum = 0;
+            }
+            sum = wave_ballot(!sure) ? kUnsure : wave_sum_u32(sum);
+            if (lane == 0) sums[buffer + w] = sum;
+            __syncthreads();
+            int32_t m = U.count();
+            bool going = true;
+#pragma unroll
+            for (int k = 0; k < kCostWaves; ++k) {
+                const uint32_t v = (uint32_t)__builtin_amdgcn_readfirstlane((int32_t)sums[buffer + k]);
+                going = going && (k < done || (v != kUnsure && (uint32_t)m + v < 0x1000000u));
+                if (going && k >= done) {
+                    m += (int32_t)v;
+                    done = k + 1;
                 }
             }
-            scratch[2 * i] = tr;
-            scratch[2 * i + 1] = td;
+            buffer ^= kCostWaves;
+            s = U.value(m);
+            if (done == kCostWaves) break;
+            if (w == done) {
+                reinterpret_cast<float4*>(strip)[lane] = make_float4(t[0], t[1], t[2], t[3]);
+                asm volatile("" ::: "memory");  // (one wave's LDS operations are done in order)
+#pragma unroll 1
+                for (int i = 0; i < 4; ++i) s = sum_lanes(s, strip[64 * i + lane]);
+                if (lane == 0) *total = __float_as_uint(s);
+            }
+            __syncthreads();
+            s = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int32_t)*total));
+            ++done;
         }
-        if ((len & 1) != 0 && tid == 0) {  // pad to a whole float4
-            scratch[2 * len] = 0.0f;
-            scratch[2 * len + 1] = 0.0f;
-        }
-        __syncthreads();
-        if (tid < 64) total = sum_in_order(total, scratch, 2 * len);
-        __syncthreads();
     }
-    return total;
+    return s;
 }
 
 // ---------------------------------------------------------- annealing
@@ -225,22 +331,21 @@ __device__ float total_cost_block(const G* grid, int32_t gw, int32_t gh, const T
 //
 // Measured against one wave that gathered its terms from a matrix of all pairs
 // and added the initial cost one term after another: 1,000 proposals on 20 x
-// 15 cells 332 -> 149 us (200 rounds -> 97), 2,000 on 80 x 60 340 -> 116 (100
-// -> 54), 2,000 on 206 x 116 600 -> 187, 20,000 on 200 x 120 1,650 -> 742.  A
-// round takes 1.6 us for 3.3: its three phases 0.45 each, and the barriers.
+// 15 cells 332 -> 150 us (200 rounds -> 97), 2,000 on 80 x 60 340 -> 105 (100
+// -> 54), 2,000 on 206 x 116 600 -> 147, 20,000 on 200 x 120 1,650 -> 701.  A
+// round takes 1.5 us for 3.3: its three phases 0.45 each, and the barriers.
 constexpr int kSlotWaves = 4, kIdleWave = 4, kDraw1Wave = 5, kDraw2Wave = 6, kCostWave = 7;
-constexpr int32_t kAnnealThreads = 512;
 static_assert(kAnnealThreads == 64 * (kCostWave + 1), "one wave a role");
 
 // Stamps, tag << 7 | (63 - lane) << 1 | cell (0: the first of the swap): one
 // word per cell, or for grids of more cells kHashStamps words that cells
 // share (p mod kHashStamps).  A shared word can make a lane see a stamp that
 // is not its cell's: that only ends the prefix early, or is found out by
-// comparing the cells (substituted neighbours).  The words double as scratch
-// of the initial cost (2 floats per cell of a chunk + 2 of padding).
+// comparing the cells (substituted neighbours).  The words double as the
+// initial cost's.
 constexpr int32_t kHashStamps = 16384;
 __host__ __device__ __forceinline__ int32_t stamp_words(int32_t cells) {
-    return cells > kHashStamps ? kHashStamps : (cells + 8) & ~3;
+    return cells > kHashStamps ? kHashStamps : (cells < kCostWords ? kCostWords : (cells + 3) & ~3);
 }
 constexpr uint32_t kTagEnd = (1u << 25) - 1u;  // (odd: pack buffers alternate across the wrap)
 // Proposal draws, made ahead into a ring of three words a slot: x1 | y1 << 16,
@@ -572,66 +677,22 @@ __device__ __forceinline__ void draw_wave(const AnnealJob& job, const AnnealShar
 }
 
 // The running cost: the accepted deltas of a round, packed in proposal order,
-// added in the next round.  As in sum_in_order, the 64 sums are those of the
-// deltas rounded to the cost's ulp as long as none is half way and the cost
-// stays strictly inside its binade; their prefix sums come from one scan.
-// Otherwise one dependent addition after another.
+// added in the next round (+0.0 past the last changes nothing).
 struct CostSum {
     float cost, best;
     int64_t improved = 0;
     __device__ __forceinline__ void add(const float* pack, int32_t n_acc, bool greedy, int lane) {
-        const float d = pack[lane];
-        const uint32_t bits = __float_as_uint(cost), exponent = bits >> 23;
-        if (greedy) improved += n_acc;  // optimize_greedy counts every accepted swap
-        if (exponent >= 23 && exponent < 250) {
-            const float f = d * __uint_as_float((277u - exponent) << 23);
-            const float r = __builtin_rintf(f);
-            const bool plain = __builtin_fabsf(f) <= 4194304.0f && __builtin_fabsf(f - r) != 0.5f;
-            int32_t m = (int32_t)r;
-            // inclusive sums over the lanes: within rows of 16, then over rows
-            m += __builtin_amdgcn_update_dpp(0, m, 0x111, 0xF, 0xF, false);
-            m += __builtin_amdgcn_update_dpp(0, m, 0x112, 0xF, 0xF, false);
-            m += __builtin_amdgcn_update_dpp(0, m, 0x114, 0xF, 0xF, false);
-            m += __builtin_amdgcn_update_dpp(0, m, 0x118, 0xF, 0xF, false);
-            m += __builtin_amdgcn_update_dpp(0, m, 0x142, 0xA, 0xF, false);
-            m += __builtin_amdgcn_update_dpp(0, m, 0x143, 0xC, 0xF, false);
-            m += (int32_t)((bits & 0x7fffffu) | 0x800000u);
-            if (!wave_ballot(!plain || m <= 0x800000 || m >= 0x1000000)) {
-                const float c = __uint_as_float((bits & 0xff800000u) | ((uint32_t)m & 0x7fffffu));
-                if (!greedy && wave_ballot(c < best)) {
-                    // new bests: below the best before the round and all
-                    // sums before it (floats of one sign order like their bits)
-                    const uint32_t low = min(__float_as_uint(c), __float_as_uint(best));
-                    uint32_t p = low;
-                    for (int k = 1; k < 64; k <<= 1) {
-                        const uint32_t o = (uint32_t)__shfl_up((int)p, k, 64);
-                        p = lane >= k ? min(p, o) : p;
-                    }
-                    const uint32_t before = (uint32_t)__shfl_up((int)p, 1, 64);
-                    const bool record = lane == 0 ? c < best : __float_as_uint(c) < before;
-                    improved += __popcll(wave_ballot(record));
-                    best = readlane_f(__uint_as_float(p), 63);
-                }
-                cost = readlane_f(c, 63);
-                return;
-            }
+        const float c = add_lanes(cost, pack[lane], lane);
+        if (greedy) {  // optimize_greedy counts every accepted swap
+            improved += n_acc;
+        } else if (wave_ballot(c < best)) {
+            // new bests: below the best before the round and all sums before
+            const float p = wave_scan_min(__builtin_fminf(c, best));
+            const float before = __int_as_float(__builtin_amdgcn_update_dpp(
+                __float_as_int(best), __float_as_int(p), 0x138, 0xF, 0xF, false));  // the lane below's
+            improved += __popcll(wave_ballot(c < before));
+            best = readlane_f(p, 63);
         }
-        const float4* pack4 = reinterpret_cast<const float4*>(pack);
-        uint32_t better = 0;
-        for (int32_t q = 0; q < n_acc; q += 8) {
-            const float4 u0 = pack4[q >> 2], u1 = pack4[(q >> 2) + 1];
-            const float v[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
-            // Adding a +0.0 past the last delta changes nothing.  best =
-            // fminf(best, cost) equals `cost < best ? cost : best` here (no
-            // NaN, no -0.0) and keeps the compare off the dependent chain.
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                cost = cost + v[i];
-                better += cost < best ? 1u : 0u;
-                best = __builtin_fminf(best, cost);
-            }
-        }
-        if (!greedy) improved += better;
     }
 };
 
@@ -698,10 +759,26 @@ __global__ __launch_bounds__(kAnnealThreads) void anneal_kernel(AnnealJob single
         grid = &hbm;
     } else {
         grid = reinterpret_cast<G*>(grid_at);
-        for (int32_t i = tid; i < cells; i += kAnnealThreads) grid[i] = (G)gload(job.grid, i);
+        // (eight loads in flight)
+        for (int32_t i = tid; i < cells; i += 8 * kAnnealThreads) {
+            int32_t m[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                m[k] = gload(job.grid, min(i + k * kAnnealThreads, cells - 1));
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                if (i + k * kAnnealThreads < cells) grid[i + k * kAnnealThreads] = (G)m[k];
+        }
     }
     if (S.labs)
-        for (int32_t i = tid; i < job.n; i += kAnnealThreads) labs[i] = gload4(job.lab4, i);
+        for (int32_t i = tid; i < job.n; i += 4 * kAnnealThreads) {
+            float4 l[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) l[k] = gload4(job.lab4, min(i + k * kAnnealThreads, job.n - 1));
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (i + k * kAnnealThreads < job.n) labs[i + k * kAnnealThreads] = l[k];
+        }
     // the first proposals (coordinates are in the grid past max_iter too)
     if (tid < kRing) {
         S.ring_xy1[tid] = (uint32_t)draw_range(job.seed, tid, 0, job.grid_w) |
@@ -711,11 +788,10 @@ __global__ __launch_bounds__(kAnnealThreads) void anneal_kernel(AnnealJob single
         S.ring_u[tid] = draw_unit(job.seed, tid);
     }
     __syncthreads();
-    float* const scratch = reinterpret_cast<float*>(S.stamp);
-    const int32_t chunk = (words / 2 - 1) & ~1;
     const float initial =
-        S.labs ? total_cost_block(grid, job.grid_w, job.grid_h, TermLds{S.labs}, scratch, chunk)
-               : total_cost_block(grid, job.grid_w, job.grid_h, TermLab{job.lab4}, scratch, chunk);
+        S.labs ? total_cost_block(grid, job.grid_w, job.grid_h, TermLds{S.labs}, S.stamp)
+               : total_cost_block(grid, job.grid_w, job.grid_h, TermLab{job.lab4}, S.stamp);
+    __syncthreads();
     for (int32_t i = tid; i < words; i += kAnnealThreads) S.stamp[i] = 0u;
     if (tid == 0) S.ctrl[kCtrlCost] = __float_as_uint(initial);
     __syncthreads();
@@ -799,20 +875,18 @@ hipError_t anneal_configure(int max_lds) {
 }
 
 // ------------------------------------------------ cost / delta / penalty
-__global__ __launch_bounds__(kAnnealThreads) void total_cost_kernel(const int32_t* __restrict__ grid,
-                                                        int32_t gw, int32_t gh,
-                                                        const float4* __restrict__ lab4,
-                                                        float* __restrict__ scratch, int32_t chunk,
-                                                        float* __restrict__ out) {
-    const float t = total_cost_block(grid, gw, gh, TermLab{lab4}, scratch, chunk);
+__global__ __launch_bounds__(kAnnealThreads) void total_cost_kernel(
+    const int32_t* __restrict__ grid, int32_t gw, int32_t gh, const float4* __restrict__ lab4,
+    float* __restrict__ out) {
+    __shared__ __align__(16) uint32_t lds[kCostWords];
+    const float t = total_cost_block(grid, gw, gh, TermLab{lab4}, lds);
     if (threadIdx.x == 0) *out = t;
 }
 
-void launch_total_cost(const int32_t* grid, int32_t gw, int32_t gh, const float4* lab4,
-                       float* scratch, int32_t chunk, float* out,
+void launch_total_cost(const int32_t* grid, int32_t gw, int32_t gh, const float4* lab4, float* out,
                        hipStream_t stream) {
-    hipLaunchKernelGGL(total_cost_kernel, dim3(1), dim3(kAnnealThreads), 0, stream, grid, gw, gh, lab4,
-                       scratch, chunk, out);
+    hipLaunchKernelGGL(total_cost_kernel, dim3(1), dim3(kAnnealThreads), 0, stream, grid, gw, gh,
+                       lab4, out);
 }
 
 __global__ void swap_delta_kernel(const int32_t* __restrict__ grid, int32_t gw, int32_t gh,

@@ -1281,12 +1281,10 @@ int mh_total_cost(mh_context* ctx, const mh_library* lib, const int32_t* grid, i
     CHK(check_grid_values(grid, cells, lib->n));
     CHK(set_device(ctx));
     int32_t* d_grid;
-    float *d_scratch, *d_out;
-    const int32_t chunk = cells < 65536 ? cells : 65536;
+    float* d_out;
     CHK(upload(ctx, S_GRID, grid, (size_t)cells, &d_grid));
-    CHK(slot(ctx, S_OUT0, (size_t)chunk * 2 + 4, &d_scratch));
     CHK(slot(ctx, S_OUT1, 1, &d_out));
-    launch_total_cost(d_grid, gw, gh, lib->d_lab4, d_scratch, chunk, d_out, ctx->stream);
+    launch_total_cost(d_grid, gw, gh, lib->d_lab4, d_out, ctx->stream);
     HIPCHK(hipGetLastError());
     CHK(download(ctx, out, d_out, 1));
     return sync(ctx);

@@ -195,8 +195,8 @@ size_t anneal_lds_bytes(int32_t cells, int32_t kind, int32_t labs);
 void launch_anneal_single(const AnnealJob& job, int32_t kind, size_t lds_bytes, hipStream_t stream);
 void launch_anneal_batch(const AnnealJob* d_jobs, int32_t n_jobs, int32_t kind, size_t lds_bytes,
                          hipStream_t stream);
-void launch_total_cost(const int32_t* grid, int32_t gw, int32_t gh, const float4* lab4,
-                       float* scratch, int32_t chunk, float* out, hipStream_t stream);
+void launch_total_cost(const int32_t* grid, int32_t gw, int32_t gh, const float4* lab4, float* out,
+                       hipStream_t stream);
 void launch_swap_deltas(const int32_t* grid, int32_t gw, int32_t gh, const float4* lab4,
                         const int32_t* pairs, int32_t p, float* out, hipStream_t stream);
 void launch_penalties(const int32_t* grid, int32_t gw, int32_t gh, const float4* lab4, float weight,
