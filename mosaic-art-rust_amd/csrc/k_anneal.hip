@@ -299,19 +299,19 @@ __device__ float total_cost_block(const G* grid, int32_t gw, int32_t gh, const T
 
 // ---------------------------------------------------------- annealing
 // What bounds it is the latency of a round, and how many proposals a round
-// commits.  A round runs on seven waves of one workgroup, a barrier between
-// its three phases (s: the first proposal of the round; lane l of the first
-// four waves: proposal s + l):
-//   * reads: slot wave w reads the swap's two cells and its two of their
-//     eight neighbour cells (w = 0, 1: Up and Down, Left and Right of the
-//     first cell; 2, 3: of the second), and those materials' Labs;
-//   * terms: the four adjacency terms of its two neighbours with the swap's
-//     two materials, to LDS;
-//   * decisions: wave 0 adds a swap's terms in the reference's order, decides
-//     it, finds how many proposals can be committed, and swaps.
-// Meanwhile three waves, on the SIMDs that wait for wave 0 then, draw later
-// proposals and add the last round's deltas to the running cost.  (The fifth
-// wave would share wave 0's SIMD: it ends after the set-up.)
+// commits.  A round runs on eight waves of one workgroup in two phases, with a
+// barrier after each (s: the first proposal of the round; lane l of the slot
+// waves and the judge: proposal s + l):
+//   * terms: slot wave w makes the adjacency terms of two of the eight
+//     neighbour cells (w = 0, 1: Up and Down, Left and Right of the first
+//     cell; 2, 3: of the second) with the swap's two materials.  The judge
+//     takes in the proposals, and swaps those it expects to be accepted.
+//   * decisions: the judge adds a swap's terms in the reference's order and
+//     decides it.  The slot waves read the next round's cells and Labs, from
+//     the grid as it is expected to be.
+// If a decision was not the expected one, the judge puts the grid right and
+// the next round begins with its reads once more (a third phase).  Meanwhile
+// two waves draw later proposals and one adds the deltas to the running cost.
 //
 // A round's prefix that can be committed, `first`, is found in one of two
 // ways, by which is longer for the share p of proposals that are accepted:
@@ -331,10 +331,11 @@ __device__ float total_cost_block(const G* grid, int32_t gw, int32_t gh, const T
 //
 // Measured against one wave that gathered its terms from a matrix of all pairs
 // and added the initial cost one term after another: 1,000 proposals on 20 x
-// 15 cells 332 -> 150 us (200 rounds -> 97), 2,000 on 80 x 60 340 -> 105 (100
-// -> 54), 2,000 on 206 x 116 600 -> 147, 20,000 on 200 x 120 1,650 -> 701.  A
-// round takes 1.5 us for 3.3: its three phases 0.45 each, and the barriers.
-constexpr int kSlotWaves = 4, kIdleWave = 4, kDraw1Wave = 5, kDraw2Wave = 6, kCostWave = 7;
+// 15 cells 332 -> 127 us (200 rounds -> 97), 2,000 on 80 x 60 340 -> 92 (100 ->
+// 54), 2,000 on 206 x 116 600 -> 132, 20,000 on 200 x 120 1,650 -> 568.  A
+// round takes 1.15 us for 3.3 (1.5 with the reads as a phase of their own):
+// 1,600 cycles of terms, 1,000 of decisions.
+constexpr int kSlotWaves = 4, kJudgeWave = 4, kDraw1Wave = 5, kDraw2Wave = 6, kCostWave = 7;
 static_assert(kAnnealThreads == 64 * (kCostWave + 1), "one wave a role");
 
 // Stamps, tag << 7 | (63 - lane) << 1 | cell (0: the first of the swap): one
@@ -347,7 +348,7 @@ constexpr int32_t kHashStamps = 16384;
 __host__ __device__ __forceinline__ int32_t stamp_words(int32_t cells) {
     return cells > kHashStamps ? kHashStamps : (cells < kCostWords ? kCostWords : (cells + 3) & ~3);
 }
-constexpr uint32_t kTagEnd = (1u << 25) - 1u;  // (odd: pack buffers alternate across the wrap)
+constexpr uint32_t kTagEnd = (1u << 25) - 2u;  // (a round takes at most two)
 // Proposal draws, made ahead into a ring of three words a slot: x1 | y1 << 16,
 // x2 | y2 << 16, u (both sides are below 2^16: a grid in LDS is far smaller,
 // and the HBM variant requires it).
@@ -355,30 +356,34 @@ constexpr int32_t kRing = 256;
 
 // LDS in words, behind the stamps: Labs of the swaps' materials (64 of the
 // first, 64 of the second), the terms (4 waves x 64 x {m1 with a, m2 with a,
-// m1 with b, m2 with b} for the wave's neighbours a, b), the mutual terms,
-// two rounds' accepted deltas, the ring, control words, the grid, the
-// library's Labs (where they fit).
-constexpr int32_t kLabWords = 2 * 64 * 4, kTermWords = kSlotWaves * 64 * 4, kMutualWords = 64,
-                  kPackWords = 2 * 64, kCtrlWords = 8;
+// m1 with b, m2 with b} for the wave's neighbours a, b), the lanes that a and b
+// were taken from, the mutual terms, a round's accepted deltas, the ring,
+// control words, the grid, the library's Labs (where they fit).
+constexpr int32_t kLabWords = 2 * 64 * 4, kTermWords = kSlotWaves * 64 * 4,
+                  kFromWords = kSlotWaves * 64, kMutualWords = 64, kPackWords = 64, kCtrlWords = 8;
 constexpr int32_t kFixedWords =
-    kLabWords + kTermWords + kMutualWords + kPackWords + 3 * kRing + kCtrlWords;
+    kLabWords + kTermWords + kFromWords + kMutualWords + kPackWords + 3 * kRing + kCtrlWords;
 __host__ __device__ __forceinline__ int32_t grid_words(int32_t cells, int32_t kind) {
     return kind == kAnnealHbm ? 0 : (kind == kAnnealNarrow ? (cells + 7) / 8 * 4 : (cells + 3) & ~3);
 }
 
 // The control words: what a round leaves for the next, then a run's results.
 enum { kCtrlRound = 0, kCtrlCost = 2, kCtrlBest = 3, kCtrlImproved = 4 };
-__device__ __forceinline__ uint32_t pack_round(int32_t advance, bool hopeful, int32_t accepted) {
-    return (uint32_t)advance | (hopeful ? 128u : 0u) | (uint32_t)accepted << 8;
+__device__ __forceinline__ uint32_t pack_round(int32_t advance, bool hopeful, bool reread,
+                                               int32_t accepted) {
+    return (uint32_t)advance | (hopeful ? 128u : 0u) | (reread ? 256u : 0u) | (uint32_t)accepted << 9;
 }
+
+constexpr uint32_t kNoLane = 255u;
 
 template <typename G>
 struct AnnealShared {
     uint32_t* stamp;
     float4* lab_m;     // [2][64]
     float4* terms;     // [kSlotWaves][64]
+    uint32_t* from;    // [kSlotWaves][64]: a's lane | b's << 8, kNoLane: none
     float* mutual;     // [64]
-    float* pack;       // [2][64]
+    float* pack;       // [64]
     uint32_t *ring_xy1, *ring_xy2;
     float* ring_u;
     uint32_t* ctrl;
@@ -389,33 +394,6 @@ struct AnnealShared {
     }
 };
 
-// How the waves follow the run, alike in each: the round's first proposal,
-// its number, how its prefix is found, and the deltas the last round left.
-struct Rounds {
-    int64_t s = 0;
-    uint32_t tag = 1;
-    bool hopeful;
-    int32_t pending = 0;
-    __device__ __forceinline__ void next(const uint32_t* ctrl) {
-        const uint32_t v = (uint32_t)__builtin_amdgcn_readfirstlane((int32_t)ctrl[kCtrlRound]);
-        s += v & 127u;
-        hopeful = (v & 128u) != 0u;
-        pending = (int32_t)(v >> 8);
-        ++tag;
-    }
-};
-
-// Stamps of an old round look like this round's once the tags wrap.
-template <typename G>
-__device__ __forceinline__ void wrap_tags(const AnnealShared<G>& S, Rounds& R, int32_t words, int tid) {
-    if (R.tag < kTagEnd) return;
-    __syncthreads();
-    if (tid < 64 * kSlotWaves)
-        for (int32_t i = tid; i < words; i += 64 * kSlotWaves) S.stamp[i] = 0u;
-    R.tag = 1;
-    __syncthreads();
-}
-
 // End of a phase: this wave's LDS operations are complete, then all waves
 // meet.  (__syncthreads would also wait for loads in flight: the temperatures,
 // which are requested a phase before their use.)
@@ -424,6 +402,48 @@ __device__ __forceinline__ void phase_end() {
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 }
+
+// How the waves follow the run, alike in each: the round's first proposal,
+// the tag of its stamps, how its prefix is found, whether its reads must be
+// repeated, and how many deltas the last round left.
+struct Rounds {
+    int64_t s = 0;
+    uint32_t tag = 1;
+    bool hopeful = true, reread = false;
+    int32_t pending = 0;
+
+    // The last round's outcome.
+    __device__ __forceinline__ void next(uint32_t ctrl) {
+        const uint32_t v = (uint32_t)__builtin_amdgcn_readfirstlane((int32_t)ctrl);
+        s += v & 127u;
+        hopeful = (v & 128u) != 0u;
+        reread = (v & 256u) != 0u;
+        pending = (int32_t)(v >> 9);
+    }
+    // Before a round's terms; read: what the slot waves do to repeat the
+    // reads, load: what a wave has to take in again then.  (Stamps of an old round look like this round's once the tags
+    // wrap, so the stamps are cleared then.)
+    template <typename G, typename Read, typename Load>
+    __device__ __forceinline__ void begin(const AnnealShared<G>& S, int32_t words, int tid,
+                                          Read&& read, Load&& load) {
+        if (tag >= kTagEnd) {
+            phase_end();
+            for (int32_t i = tid; i < words; i += kAnnealThreads) S.stamp[i] = 0u;
+            tag = 0;
+            reread = true;
+            phase_end();
+        }
+        if (reread) {
+            ++tag;
+            read();
+            phase_end();
+            load();
+        }
+    }
+};
+struct Nothing {
+    __device__ __forceinline__ void operator()() const {}
+};
 
 // The Labs of two neighbours and (waves 0 and 1) of one of the swap's
 // materials, requested together.
@@ -445,234 +465,372 @@ __device__ __forceinline__ void load_labs(const AnnealJob& job, const AnnealShar
     }
 }
 
-template <typename G, bool kHbm>
-__device__ __forceinline__ void slot_wave(const AnnealJob& job, const AnnealShared<G>& S, G* grid,
-                                          int w, int lane, Rounds R, int32_t words,
-                                          AnnealOut* out) {
-    const int32_t gw = job.grid_w, gh = job.grid_h;
+// Where a slot wave's swap and its two neighbours are.
+struct Place {
+    int32_t p1, p2, qa, qb;
+    bool in_a, in_b, self_a, self_b;  // inside the grid; the swap's other cell
+    bool active;
+};
+
+template <typename G>
+__device__ __forceinline__ Place place_of(const AnnealJob& job, const AnnealShared<G>& S, int w,
+                                          int64_t it) {
+    const int32_t gw = job.grid_w;
     const bool vertical = !(w & 1), second = w >= 2;
-    const int32_t step = vertical ? gw : 1, bound = vertical ? gh : gw;
-    const int64_t max_iter = job.max_iter;
-    int64_t kbase = 0, accepted = 0, evaluated = 0, rounds = 0;  // (wave 0's)
-    while (R.s < max_iter) {
-        wrap_tags(S, R, words, w * 64 + lane);
-        // ---- reads
-        const int64_t it = R.s + lane;
-        const uint32_t slot = (uint32_t)it & (kRing - 1);
-        const uint32_t xy1 = S.ring_xy1[slot], xy2 = S.ring_xy2[slot];
-        const int32_t x1 = (int32_t)(xy1 & 0xffffu), y1 = (int32_t)(xy1 >> 16);
-        const int32_t x2 = (int32_t)(xy2 & 0xffffu), y2 = (int32_t)(xy2 >> 16);
-        const int32_t p1 = y1 * gw + x1, p2 = y2 * gw + x2;
-        const int32_t centre = second ? p2 : p1, partner = second ? p1 : p2;
-        const int32_t along = vertical ? (second ? y2 : y1) : (second ? x2 : x1);
-        const bool in_a = along > 0, in_b = along < bound - 1;
-        // a neighbour outside the grid reads its own cell, always in bounds
-        const int32_t qa = in_a ? centre - step : centre, qb = in_b ? centre + step : centre;
-        const int32_t m1 = gget(grid, p1), m2 = gget(grid, p2);
-        const int32_t a = gget(grid, qa), b = gget(grid, qb);
-        const bool skip = it >= max_iter || p1 == p2 || m1 == kEmpty || m2 == kEmpty;
-        float4 la = make_float4(0, 0, 0, 0), lb = la, lm = la;
-        if (job.n > 0) load_labs(job, S, a, b, w == 0 ? m1 : m2, w < 2, la, lb, lm);
-        uint64_t nonskip = 0;
-        float temp = 1.0f, u = 0.0f;
+    const int32_t step = vertical ? gw : 1, bound = vertical ? job.grid_h : gw;
+    const uint32_t slot = (uint32_t)it & (kRing - 1);
+    const uint32_t xy1 = S.ring_xy1[slot], xy2 = S.ring_xy2[slot];
+    const int32_t x1 = (int32_t)(xy1 & 0xffffu), y1 = (int32_t)(xy1 >> 16);
+    const int32_t x2 = (int32_t)(xy2 & 0xffffu), y2 = (int32_t)(xy2 >> 16);
+    Place p;
+    p.p1 = y1 * gw + x1;
+    p.p2 = y2 * gw + x2;
+    const int32_t centre = second ? p.p2 : p.p1, partner = second ? p.p1 : p.p2;
+    const int32_t along = vertical ? (second ? y2 : y1) : (second ? x2 : x1);
+    p.in_a = along > 0;
+    p.in_b = along < bound - 1;
+    // a neighbour outside the grid reads its own cell, always in bounds
+    p.qa = p.in_a ? centre - step : centre;
+    p.qb = p.in_b ? centre + step : centre;
+    p.self_a = p.in_a && p.qa == partner;
+    p.self_b = p.in_b && p.qb == partner;
+    p.active = it < job.max_iter && p.p1 != p.p2;
+    return p;
+}
+
+// What a slot wave's reads bring: the neighbours' Labs, which of them count,
+// and whether the proposal does.
+struct Reads {
+    float4 la, lb;
+    bool ok_a, ok_b, skip;
+};
+
+template <typename G>
+__device__ __forceinline__ Reads read_swap(const AnnealJob& job, const AnnealShared<G>& S, G* grid,
+                                           int w, int lane, const Place& p, const Rounds& R) {
+    const int32_t m1 = gget(grid, p.p1), m2 = gget(grid, p.p2);
+    const int32_t a = gget(grid, p.qa), b = gget(grid, p.qb);
+    Reads r;
+    r.skip = !p.active || m1 == kEmpty || m2 == kEmpty;
+    r.ok_a = p.in_a && !p.self_a && a != kEmpty;
+    r.ok_b = p.in_b && !p.self_b && b != kEmpty;
+    float4 lm = make_float4(0, 0, 0, 0);
+    r.la = r.lb = lm;
+    if (job.n > 0) load_labs(job, S, a, b, w == 0 ? m1 : m2, w < 2, r.la, r.lb, lm);
+    if (w == 2 && R.hopeful && !r.skip) {
         const uint32_t mine = (R.tag << 7) | ((uint32_t)(63 - lane) << 1);
-        if (w == 0) {
-            nonskip = wave_ballot(!skip);
-            if (!skip) {
-                if (R.hopeful) {
-                    atomicMax(&S.stamp[S.at(p1)], mine);
-                    atomicMax(&S.stamp[S.at(p2)], mine | 1u);
-                }
-                if (!job.greedy) {
-                    temp = gload(job.temps, kbase + lanes_before(nonskip));
-                    u = S.ring_u[slot];
-                }
-            }
-        }
-        if (w < 2) S.lab_m[w * 64 + lane] = lm;
-        phase_end();
+        atomicMax(&S.stamp[S.at(p.p1)], mine);
+        atomicMax(&S.stamp[S.at(p.p2)], mine | 1u);
+    }
+    if (w < 2) S.lab_m[w * 64 + lane] = lm;
+    return r;
+}
+
+// How many of the round's proposals are not blocked by a lower lane's stamp
+// on one of their own cells (v1, v2: those cells' stamps), at most the rest of
+// the run.
+__device__ __forceinline__ int32_t expected_prefix(uint32_t v1, uint32_t v2, uint32_t mine, bool skip,
+                                                   int64_t remain) {
+    const bool taken = !skip && ((v1 >> 1) != (mine >> 1) || (v2 >> 1) != (mine >> 1));
+    const uint64_t t = wave_ballot(taken);
+    const int32_t first = t ? __ffsll((unsigned long long)t) - 1 : 64;
+    return (int64_t)first < remain ? first : (int32_t)remain;
+}
+
+template <typename G>
+__device__ __forceinline__ void slot_wave(const AnnealJob& job, const AnnealShared<G>& S, G* grid,
+                                          int w, int lane, int32_t words) {
+    Rounds R;
+    R.hopeful = !job.greedy;
+    const int64_t max_iter = job.max_iter;
+    Place p = place_of(job, S, w, lane);
+    Reads r = read_swap(job, S, grid, w, lane, p, R);
+    phase_end();
+    for (;;) {
         // ---- terms
-        const float4 l1 = S.lab_m[lane], l2 = S.lab_m[64 + lane];
-        int32_t first = 64;
+        const uint32_t outcome = S.ctrl[kCtrlRound];
+        float4 l1, l2;
+        uint32_t va, vb, v1, v2;
+        // (with the outcome in flight: it is nearly always the expected one)
+        auto load = [&]() __attribute__((always_inline)) {
+            va = S.stamp[S.at(p.qa)];
+            vb = S.stamp[S.at(p.qb)];
+            v1 = S.stamp[S.at(p.p1)];
+            v2 = S.stamp[S.at(p.p2)];
+            l1 = S.lab_m[lane];
+            l2 = S.lab_m[64 + lane];
+        };
+        load();
+        R.next(outcome);
+        if (R.s >= max_iter) return;
+        R.begin(
+            S, words, w * 64 + lane,
+            [&]() __attribute__((always_inline)) {
+                p = place_of(job, S, w, R.s + lane);
+                r = read_swap(job, S, grid, w, lane, p, R);
+            },
+            load);
+        float4 la = r.la, lb = r.lb;
+        const Place q = p;
+        uint32_t from = kNoLane | kNoLane << 8;
         if (R.hopeful) {
-            const uint32_t va = S.stamp[S.at(qa)], vb = S.stamp[S.at(qb)];
-            if (w == 0) {
-                const uint32_t v1 = S.stamp[S.at(p1)], v2 = S.stamp[S.at(p2)];
-                const bool taken = !skip && ((v1 >> 1) != (mine >> 1) || (v2 >> 1) != (mine >> 1));
-                const uint64_t t = wave_ballot(taken);
-                first = t ? __ffsll((unsigned long long)t) - 1 : 64;
-            }
+            const uint32_t mine = (R.tag << 7) | ((uint32_t)(63 - lane) << 1);
+            // the next round's proposals, if all goes as expected
+            const int32_t first = expected_prefix(v1, v2, mine, r.skip, max_iter - R.s);
+            p = place_of(job, S, w, R.s + first + lane);
             // stamped in this round by a lower lane: above this lane's stamps
             bool sub_a = va > (mine | 1u), sub_b = vb > (mine | 1u);
             if (wave_ballot(sub_a || sub_b)) {
-                const int32_t ka = 63 - (int32_t)((va >> 1) & 63u), kb = 63 - (int32_t)((vb >> 1) & 63u);
+                const uint32_t ka = 63u - ((va >> 1) & 63u), kb = 63u - ((vb >> 1) & 63u);
                 uint32_t ca = va & 1u, cb = vb & 1u;  // which of k's cells
                 if (S.hashed) {
-                    auto which = [&](int32_t k, int32_t q, bool& sub) {
+                    auto which = [&](uint32_t k, int32_t cell, bool& sub) {
                         const uint32_t ks = (uint32_t)(R.s + k) & (kRing - 1);
                         const uint32_t k1 = S.ring_xy1[ks], k2 = S.ring_xy2[ks];
-                        const bool is1 = (int32_t)(k1 >> 16) * gw + (int32_t)(k1 & 0xffffu) == q;
-                        const bool is2 = (int32_t)(k2 >> 16) * gw + (int32_t)(k2 & 0xffffu) == q;
+                        const bool is1 =
+                            (int32_t)(k1 >> 16) * job.grid_w + (int32_t)(k1 & 0xffffu) == cell;
+                        const bool is2 =
+                            (int32_t)(k2 >> 16) * job.grid_w + (int32_t)(k2 & 0xffffu) == cell;
                         sub = sub && (is1 || is2);
                         return is1 ? 0u : 1u;
                     };
-                    ca = which(ka, qa, sub_a);
-                    cb = which(kb, qb, sub_b);
+                    ca = which(ka, q.qa, sub_a);
+                    cb = which(kb, q.qb, sub_b);
                 }
                 // k's first cell gets its second material, and the reverse
-                const float4 na = S.lab_m[(ca ? 0 : 64) + ka], nb = S.lab_m[(cb ? 0 : 64) + kb];
+                const float4 na = S.lab_m[(ca ? 0u : 64u) + ka], nb = S.lab_m[(cb ? 0u : 64u) + kb];
                 la = make_float4(sub_a ? na.x : la.x, sub_a ? na.y : la.y, sub_a ? na.z : la.z, 0.0f);
                 lb = make_float4(sub_b ? nb.x : lb.x, sub_b ? nb.y : lb.y, sub_b ? nb.z : lb.z, 0.0f);
+                from = (sub_a ? ka : kNoLane) | (sub_b ? kb : kNoLane) << 8;
             }
+            S.from[w * 64 + lane] = from;
         }
-        const bool self_a = in_a && qa == partner, self_b = in_b && qb == partner;
-        const bool ok_a = in_a && !self_a && a != kEmpty, ok_b = in_b && !self_b && b != kEmpty;
         const float t1a = adj_term(l1, la), t2a = adj_term(l2, la);
         const float t1b = adj_term(l1, lb), t2b = adj_term(l2, lb);
-        S.terms[w * 64 + lane] = make_float4(ok_a ? t1a : 0.0f, ok_a ? t2a : 0.0f,
-                                             ok_b ? t1b : 0.0f, ok_b ? t2b : 0.0f);
+        S.terms[w * 64 + lane] = make_float4(r.ok_a ? t1a : 0.0f, r.ok_a ? t2a : 0.0f,
+                                             r.ok_b ? t1b : 0.0f, r.ok_b ? t2b : 0.0f);
         // the partner as a neighbour of the first cell: the mutual term
-        if (!second && (self_a || self_b)) S.mutual[lane] = self_a ? t1a : t1b;
+        if (w < 2 && (q.self_a || q.self_b)) S.mutual[lane] = q.self_a ? t1a : t1b;
         phase_end();
         // ---- decisions
-        if (w == 0) {
-            const float4 v0 = S.terms[lane], v1 = S.terms[64 + lane], v2 = S.terms[128 + lane],
-                         v3 = S.terms[192 + lane];
-            const bool adjacent = p1 - p2 == gw || p2 - p1 == gw || (y1 == y2 && (x1 - x2 == 1 || x2 - x1 == 1));
-            // the first cell's neighbours: old with m1, new with m2; the second's the reverse
-            float old_cost = v0.x, new_cost = v0.y;
-            old_cost += v0.z;
-            new_cost += v0.w;
-            old_cost += v1.x;
-            new_cost += v1.y;
-            old_cost += v1.z;
-            new_cost += v1.w;
-            old_cost += v2.y;
-            new_cost += v2.x;
-            old_cost += v2.w;
-            new_cost += v2.z;
-            old_cost += v3.y;
-            new_cost += v3.x;
-            old_cost += v3.w;
-            new_cost += v3.z;
-            if (adjacent) {
-                const float t = S.mutual[lane];
-                old_cost += t;
-                new_cost += t;
+        if (R.hopeful) {
+            ++R.tag;
+            r = read_swap(job, S, grid, w, lane, p, R);
+        }
+        phase_end();
+    }
+}
+
+// kHbm: the grid's swaps are complete at agent scope before other waves read
+// it (the barriers order the waves).
+template <typename G, bool kHbm>
+__device__ __forceinline__ void judge_wave(const AnnealJob& job, const AnnealShared<G>& S, G* grid,
+                                           int lane, int32_t words, AnnealOut* out) {
+    Rounds R;
+    R.hopeful = !job.greedy;
+    const int32_t gw = job.grid_w, gh = job.grid_h;
+    const int64_t max_iter = job.max_iter;
+    int64_t kbase = 0, accepted = 0, evaluated = 0, rounds = 0;
+    // the last round's, for the cost wave and the traces
+    float delta = 0.0f;
+    uint64_t accmask = 0;
+    int64_t it = lane;
+    bool acc = false, skip = true;
+    int32_t first = 0;
+    // the round's proposals (the next round's are taken in ahead)
+    uint32_t xy1, xy2;
+    float u;
+    auto take = [&](int64_t from) __attribute__((always_inline)) {
+        const uint32_t slot = (uint32_t)(from + lane) & (kRing - 1);
+        xy1 = S.ring_xy1[slot];
+        xy2 = S.ring_xy2[slot];
+        u = S.ring_u[slot];
+    };
+    take(0);
+    phase_end();
+    for (;;) {
+        // ---- terms
+        const uint32_t outcome = S.ctrl[kCtrlRound];
+        int32_t x1, y1, x2, y2, p1, p2, m1, m2;
+        uint32_t v1, v2;
+        float uniform;
+        auto load = [&]() __attribute__((always_inline)) {
+            x1 = (int32_t)(xy1 & 0xffffu);
+            y1 = (int32_t)(xy1 >> 16);
+            x2 = (int32_t)(xy2 & 0xffffu);
+            y2 = (int32_t)(xy2 >> 16);
+            uniform = u;
+            p1 = y1 * gw + x1;
+            p2 = y2 * gw + x2;
+            m1 = gget(grid, p1);
+            m2 = gget(grid, p2);
+            v1 = S.stamp[S.at(p1)];
+            v2 = S.stamp[S.at(p2)];
+        };
+        load();
+        R.next(outcome);
+        // the accepted deltas in proposal order, +0.0 past the last
+        S.pack[lane] = 0.0f;
+        asm volatile("" ::: "memory");
+        if (lane_in(accmask)) S.pack[lanes_before(accmask)] = delta;
+        if (lane < first) {
+            if (job.trace_delta) gstore(job.trace_delta, it, skip ? __int_as_float(0x7fc00000) : delta);
+            if (job.trace_accept) gstore(job.trace_accept, it, (uint8_t)(acc ? 1 : 0));
+        }
+        if (R.s >= max_iter) break;
+        R.begin(S, words, kJudgeWave * 64 + lane, Nothing{}, [&]() __attribute__((always_inline)) {
+            take(R.s);
+            load();
+        });
+        it = R.s + lane;
+        const uint32_t mine = (R.tag << 7) | ((uint32_t)(63 - lane) << 1);
+        skip = it >= max_iter || p1 == p2 || m1 == kEmpty || m2 == kEmpty;
+        const uint64_t nonskip = wave_ballot(!skip);
+        float temp = 1.0f;
+        if (!skip && !job.greedy) temp = gload(job.temps, kbase + lanes_before(nonskip));
+        const int64_t remain = max_iter - R.s;
+        first = remain < 64 ? (int32_t)remain : 64;
+        if (R.hopeful) {
+            first = expected_prefix(v1, v2, mine, skip, remain);
+            take(R.s + first);
+            if (!skip && lane < first) {  // (all of these cells are different)
+                gput(grid, p1, m2);
+                gput(grid, p2, m1);
             }
-            const float delta = m1 == m2 ? 0.0f : new_cost - old_cost;
-            bool acc = false;
-            if (!skip) {
-                if (delta < 0.0f) {
-                    acc = true;
-                } else if (!job.greedy) {
-                    // Metropolis test u < exp(x), x = -delta/T (src/optimizer.rs:77-84).
-                    // An estimate from the hardware reciprocal and exp2 is within
-                    // 2^-15 of exp(x), relative, down to 2^-126 (below, it may be 0,
-                    // and u is either 0 or at least 2^-24), so it decides alone
-                    // unless u lies within 2^-10 of it (or it is 0 or not finite);
-                    // those lanes compute x and exp exactly.
-                    const float e = __builtin_amdgcn_exp2f(-delta * __builtin_amdgcn_rcpf(temp) *
-                                                           1.44269504f);
-                    if (__builtin_fabsf(u - e) > e * (1.0f / 1024.0f))
-                        acc = u < e;
-                    else
-                        acc = u < exp_f32(-delta / temp);
+            if constexpr (kHbm) __threadfence();
+        }
+        const bool adjacent =
+            p1 - p2 == gw || p2 - p1 == gw || (y1 == y2 && (x1 - x2 == 1 || x2 - x1 == 1));
+        phase_end();
+        // ---- decisions
+        const float4 t0 = S.terms[lane], t1 = S.terms[64 + lane], t2 = S.terms[128 + lane],
+                     t3 = S.terms[192 + lane];
+        // the first cell's neighbours: old with m1, new with m2; the second's the reverse
+        float old_cost = t0.x, new_cost = t0.y;
+        old_cost += t0.z;
+        new_cost += t0.w;
+        old_cost += t1.x;
+        new_cost += t1.y;
+        old_cost += t1.z;
+        new_cost += t1.w;
+        old_cost += t2.y;
+        new_cost += t2.x;
+        old_cost += t2.w;
+        new_cost += t2.z;
+        old_cost += t3.y;
+        new_cost += t3.x;
+        old_cost += t3.w;
+        new_cost += t3.z;
+        if (adjacent) {
+            const float t = S.mutual[lane];
+            old_cost += t;
+            new_cost += t;
+        }
+        delta = m1 == m2 ? 0.0f : new_cost - old_cost;
+        acc = false;
+        if (!skip) {
+            if (delta < 0.0f) {
+                acc = true;
+            } else if (!job.greedy) {
+                // Metropolis test u < exp(x), x = -delta/T (src/optimizer.rs:77-84).
+                // An estimate from the hardware reciprocal and exp2 is within
+                // 2^-15 of exp(x), relative, down to 2^-126 (below, it may be 0,
+                // and u is either 0 or at least 2^-24), so it decides alone
+                // unless u lies within 2^-10 of it (or it is 0 or not finite);
+                // those lanes compute x and exp exactly.
+                const float e = __builtin_amdgcn_exp2f(-delta * __builtin_amdgcn_rcpf(temp) *
+                                                       1.44269504f);
+                if (__builtin_fabsf(uniform - e) > e * (1.0f / 1024.0f))
+                    acc = uniform < e;
+                else
+                    acc = uniform < exp_f32(-delta / temp);
+            }
+        }
+        const uint64_t acc_all = wave_ballot(acc);
+        const uint64_t below = first >= 64 ? ~0ull : (1ull << first) - 1ull;
+        const uint64_t rejected = nonskip & ~acc_all & below;
+        uint64_t commit = below;
+        const bool as_expected = R.hopeful && !rejected;
+        if (!as_expected) {
+            bool conflict = false;
+            if (R.hopeful) {
+                // took a value that a rejected lane would have moved
+#pragma unroll
+                for (int i = 0; i < kSlotWaves; ++i) {
+                    const uint32_t f = S.from[64 * i + lane], ka = f & 255u, kb = f >> 8;
+                    conflict |= ka != kNoLane && ((rejected >> (ka & 63u)) & 1ull) != 0ull;
+                    conflict |= kb != kNoLane && ((rejected >> (kb & 63u)) & 1ull) != 0ull;
                 }
-            }
-            const int64_t remain = max_iter - R.s;
-            if ((int64_t)first > remain) first = (int32_t)remain;
-            const uint64_t acc_all = wave_ballot(acc);
-            const uint64_t below = first >= 64 ? ~0ull : (1ull << first) - 1ull;
-            const uint64_t rejected = nonskip & ~acc_all & below;
-            if (!R.hopeful || rejected) {
-                if (!R.hopeful && acc) {
+            } else {
+                if (acc) {
                     atomicMax(&S.stamp[S.at(p1)], mine);
                     atomicMax(&S.stamp[S.at(p2)], mine);
                 }
                 // (one wave's LDS operations are done in order)
                 asm volatile("" ::: "memory");
-                const int32_t q[8] = {y1 > 0 ? p1 - gw : p1, y1 < gh - 1 ? p1 + gw : p1,
-                                      x1 > 0 ? p1 - 1 : p1,  x1 < gw - 1 ? p1 + 1 : p1,
-                                      y2 > 0 ? p2 - gw : p2, y2 < gh - 1 ? p2 + gw : p2,
-                                      x2 > 0 ? p2 - 1 : p2,  x2 < gw - 1 ? p2 + 1 : p2};
-                bool conflict = false;
+                const int32_t q[10] = {p1, p2,
+                                       y1 > 0 ? p1 - gw : p1, y1 < gh - 1 ? p1 + gw : p1,
+                                       x1 > 0 ? p1 - 1 : p1,  x1 < gw - 1 ? p1 + 1 : p1,
+                                       y2 > 0 ? p2 - gw : p2, y2 < gh - 1 ? p2 + gw : p2,
+                                       x2 > 0 ? p2 - 1 : p2,  x2 < gw - 1 ? p2 + 1 : p2};
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const uint32_t v = S.stamp[S.at(q[i])];
-                    const int32_t k = 63 - (int32_t)((v >> 1) & 63u);
-                    conflict |= v > (mine | 1u) && (!R.hopeful || ((rejected >> k) & 1ull) != 0ull);
-                }
-                if (!R.hopeful)
-                    conflict |= S.stamp[S.at(p1)] > (mine | 1u) || S.stamp[S.at(p2)] > (mine | 1u);
-                const uint64_t c = wave_ballot(conflict && !skip);
-                first = min(first, c ? __ffsll((unsigned long long)c) - 1 : 64);
+                for (int i = 0; i < 10; ++i) conflict |= S.stamp[S.at(q[i])] > (mine | 1u);
             }
-            const uint64_t commit = first >= 64 ? ~0ull : (1ull << first) - 1ull;
-            const uint64_t accmask = acc_all & commit;
-            if (lane_in(accmask)) {
-                // no lower lane of this round wrote p1 or p2
-                gput(grid, p1, m2);
-                gput(grid, p2, m1);
+            const uint64_t c = wave_ballot(conflict && !skip);
+            const int32_t expected = first;
+            first = min(first, c ? __ffsll((unsigned long long)c) - 1 : 64);
+            commit = first >= 64 ? ~0ull : (1ull << first) - 1ull;
+            const bool keep = lane_in(acc_all & commit);
+            if (R.hopeful ? !skip && lane < expected && !keep : keep) {
+                // (hopeful: back; else no lower lane of this round wrote p1 or p2)
+                gput(grid, p1, R.hopeful ? m1 : m2);
+                gput(grid, p2, R.hopeful ? m2 : m1);
             }
-            if (lane < first) {
-                if (job.trace_delta) gstore(job.trace_delta, it, skip ? __int_as_float(0x7fc00000) : delta);
-                if (job.trace_accept) gstore(job.trace_accept, it, (uint8_t)(acc ? 1 : 0));
-            }
-            // an HBM grid's swaps are complete at agent scope before the next
-            // round's reads (the barrier below orders the waves)
             if constexpr (kHbm) __threadfence();
-            // the accepted deltas in proposal order, +0.0 past the last
-            float* const pack = S.pack + (R.tag & 1u) * 64;
-            const int32_t n_acc = __popcll(accmask), n_ev = __popcll(nonskip & commit);
-            pack[lane] = 0.0f;
-            if (lane_in(accmask)) pack[lanes_before(accmask)] = delta;
-            if (lane == 0)
-                S.ctrl[kCtrlRound] = pack_round(first, !job.greedy && 9 * n_acc > 5 * n_ev, n_acc);
-            accepted += n_acc;
-            evaluated += n_ev;
-            kbase += n_ev;
-            ++rounds;
         }
+        accmask = acc_all & commit;
+        const int32_t n_acc = __popcll(accmask), n_ev = __popcll(nonskip & commit);
+        if (lane == 0)
+            S.ctrl[kCtrlRound] =
+                pack_round(first, !job.greedy && 9 * n_acc >= 5 * n_ev, !as_expected, n_acc);
+        accepted += n_acc;
+        evaluated += n_ev;
+        kbase += n_ev;
+        ++rounds;
+        if (R.hopeful) ++R.tag;  // (the slot waves' reads)
         phase_end();
-        R.next(S.ctrl);
     }
-    if (w == 0) {
-        out->accepted = accepted;
-        out->evaluated = evaluated;
-        out->rounds = rounds;
-    }
+    out->accepted = accepted;
+    out->evaluated = evaluated;
+    out->rounds = rounds;
 }
 
-// The draw waves: in a round that starts with proposals up to `filled` drawn,
-// the block of 64 behind them, one draw after the decisions phase has begun
-// and one in the next round's first phase (when this SIMD's slot wave has
-// least to do).  filled >= s + 128 holds in every round when its decisions
-// start (the next window ends there at the latest), and a block is only
-// drawn where it overwrites slots before s (filled <= s + 192).
+// The draw waves, in the decisions phase, whose slot waves leave their SIMDs
+// the most: the 64 proposals behind the `filled` first.  filled >= s + 128
+// holds in every round before its terms (they look at proposals up to there),
+// and a block only overwrites slots before s (filled <= s + 192).
 template <typename G>
 __device__ __forceinline__ void draw_wave(const AnnealJob& job, const AnnealShared<G>& S, int w,
-                                          int lane, Rounds R, int32_t words) {
+                                          int lane, int32_t words) {
+    Rounds R;
+    R.hopeful = !job.greedy;
     const uint32_t k = w == kDraw1Wave ? 0u : 2u;
     uint32_t* const ring = w == kDraw1Wave ? S.ring_xy1 : S.ring_xy2;
     int64_t filled = kRing;
-    bool drawing = false;
-    uint32_t x = 0;
-    while (R.s < job.max_iter) {
-        wrap_tags(S, R, words, w * 64 + lane);
-        if (drawing) {
-            const uint64_t j = (uint64_t)(filled - 64 + lane);
-            ring[j & (kRing - 1)] = x | (uint32_t)draw_range(job.seed, j, k + 1, job.grid_h) << 16;
-        }
+    phase_end();
+    for (;;) {
+        R.next(S.ctrl[kCtrlRound]);
+        if (R.s >= job.max_iter) return;
+        R.begin(S, words, w * 64 + lane, Nothing{}, Nothing{});
         phase_end();
-        phase_end();
-        drawing = filled <= R.s + kRing - 64;
-        if (drawing) {
-            x = (uint32_t)draw_range(job.seed, (uint64_t)(filled + lane), k, job.grid_w);
+        if (filled <= R.s + kRing - 64) {
+            const uint64_t j = (uint64_t)(filled + lane);
+            ring[j & (kRing - 1)] = (uint32_t)draw_range(job.seed, j, k, job.grid_w) |
+                                    (uint32_t)draw_range(job.seed, j, k + 1, job.grid_h) << 16;
             filled += 64;
         }
+        if (R.hopeful) ++R.tag;
         phase_end();
-        R.next(S.ctrl);
     }
 }
 
@@ -699,26 +857,29 @@ struct CostSum {
 // The cost wave; it also draws u for the draw waves' blocks.
 template <typename G>
 __device__ __forceinline__ void cost_wave(const AnnealJob& job, const AnnealShared<G>& S, int lane,
-                                          Rounds R, int32_t words) {
+                                          int32_t words) {
+    Rounds R;
+    R.hopeful = !job.greedy;
     CostSum C;
     C.cost = C.best = __uint_as_float(uniform_copy(S.ctrl[kCtrlCost]));
     int64_t filled = kRing;
-    bool drawing = false;
-    while (R.s < job.max_iter) {
-        wrap_tags(S, R, words, kCostWave * 64 + lane);
-        if (drawing) {
-            const uint64_t j = (uint64_t)(filled - 64 + lane);
+    phase_end();
+    for (;;) {
+        R.next(S.ctrl[kCtrlRound]);
+        if (R.s >= job.max_iter) break;
+        R.begin(S, words, kCostWave * 64 + lane, Nothing{}, Nothing{});
+        phase_end();
+        if (R.pending) C.add(S.pack, R.pending, job.greedy != 0, lane);
+        if (filled <= R.s + kRing - 64) {
+            const uint64_t j = (uint64_t)(filled + lane);
             S.ring_u[j & (kRing - 1)] = draw_unit(job.seed, j);
+            filled += 64;
         }
+        if (R.hopeful) ++R.tag;
         phase_end();
-        if (R.pending) C.add(S.pack + ((R.tag - 1) & 1u) * 64, R.pending, job.greedy != 0, lane);
-        phase_end();
-        drawing = filled <= R.s + kRing - 64;
-        if (drawing) filled += 64;
-        phase_end();
-        R.next(S.ctrl);
     }
-    if (R.pending) C.add(S.pack + ((R.tag - 1) & 1u) * 64, R.pending, job.greedy != 0, lane);
+    phase_end();  // the last round's deltas are there
+    if (R.pending) C.add(S.pack, R.pending, job.greedy != 0, lane);
     if (lane == 0) {
         S.ctrl[kCtrlCost] = __float_as_uint(C.cost);
         S.ctrl[kCtrlBest] = __float_as_uint(C.best);
@@ -742,7 +903,8 @@ __global__ __launch_bounds__(kAnnealThreads) void anneal_kernel(AnnealJob single
     S.stamp = sm;
     S.lab_m = reinterpret_cast<float4*>(sm + words);
     S.terms = S.lab_m + 2 * 64;
-    S.mutual = reinterpret_cast<float*>(S.terms + kSlotWaves * 64);
+    S.from = reinterpret_cast<uint32_t*>(S.terms + kSlotWaves * 64);
+    S.mutual = reinterpret_cast<float*>(S.from + kFromWords);
     S.pack = S.mutual + kMutualWords;
     S.ring_xy1 = reinterpret_cast<uint32_t*>(S.pack + kPackWords);
     S.ring_xy2 = S.ring_xy1 + kRing;
@@ -793,25 +955,26 @@ __global__ __launch_bounds__(kAnnealThreads) void anneal_kernel(AnnealJob single
                : total_cost_block(grid, job.grid_w, job.grid_h, TermLab{job.lab4}, S.stamp);
     __syncthreads();
     for (int32_t i = tid; i < words; i += kAnnealThreads) S.stamp[i] = 0u;
-    if (tid == 0) S.ctrl[kCtrlCost] = __float_as_uint(initial);
+    if (tid == 0) {
+        S.ctrl[kCtrlCost] = __float_as_uint(initial);
+        S.ctrl[kCtrlRound] = pack_round(0, !job.greedy, false, 0);
+    }
     __syncthreads();
 
-    Rounds R;
-    R.hopeful = !job.greedy;
     AnnealOut r{};
     if (w < kSlotWaves)
-        slot_wave<Grid, kHbm>(job, S, grid, w, lane, R, words, &r);
-    else if (w == kDraw1Wave || w == kDraw2Wave)
-        draw_wave(job, S, w, lane, R, words);
-    else if (w == kCostWave)
-        cost_wave(job, S, lane, R, words);
+        slot_wave(job, S, grid, w, lane, words);
+    else if (w == kJudgeWave)
+        judge_wave<Grid, kHbm>(job, S, grid, lane, words, &r);
+    else if (w != kCostWave)
+        draw_wave(job, S, w, lane, words);
     else
-        return;
+        cost_wave(job, S, lane, words);
+    if (w != kCostWave) phase_end();
     __syncthreads();
     if constexpr (!kHbm)
-        if (w < kSlotWaves)
-            for (int32_t i = tid; i < cells; i += 64 * kSlotWaves) gstore(job.grid, i, (int32_t)grid[i]);
-    if (tid == 0 && job.result) {
+        for (int32_t i = tid; i < cells; i += kAnnealThreads) gstore(job.grid, i, (int32_t)grid[i]);
+    if (tid == 64 * kJudgeWave && job.result) {
         r.initial_cost = initial;
         r.final_cost = __uint_as_float(S.ctrl[kCtrlCost]);
         r.best_cost = job.greedy ? r.final_cost : __uint_as_float(S.ctrl[kCtrlBest]);
