@@ -420,14 +420,21 @@ template <typename T>
 int upload(mh_context* ctx, Slot s, const T* host, size_t count, T** dev) {
     int rc = slot(ctx, s, count, dev);
     if (rc) return rc;
-    if (count) HIPCHK(hipMemcpyAsync(*dev, host, sizeof(T) * count, hipMemcpyHostToDevice, ctx->stream));
+    const size_t bytes = sizeof(T) * count;
+    if (staged(host, bytes))
+        return stage_upload(ctx, reinterpret_cast<uint8_t*>(*dev),
+                            {HostSpan{reinterpret_cast<const uint8_t*>(host), bytes}});
+    if (count) HIPCHK(hipMemcpyAsync(*dev, host, bytes, hipMemcpyHostToDevice, ctx->stream));
     return MH_OK;
 }
 
 template <typename T>
 int download(mh_context* ctx, T* host, const T* dev, size_t count) {
-    if (host && count)
-        HIPCHK(hipMemcpyAsync(host, dev, sizeof(T) * count, hipMemcpyDeviceToHost, ctx->stream));
+    const size_t bytes = sizeof(T) * count;
+    if (host && staged(host, bytes))
+        return stage_download(ctx, reinterpret_cast<uint8_t*>(host),
+                              reinterpret_cast<const uint8_t*>(dev), bytes);
+    if (host && count) HIPCHK(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, ctx->stream));
     return MH_OK;
 }
 
@@ -476,15 +483,8 @@ void library_release(mh_library* lib) {
     if (!ctx) return;
     hipSetDevice(ctx->device);
     hipStreamSynchronize(ctx->stream);
-    if (lib->d_lab4) hipFree(lib->d_lab4);
-    if (lib->d_L) hipFree(lib->d_L);
-    if (lib->d_A) hipFree(lib->d_A);
-    if (lib->d_B) hipFree(lib->d_B);
-    if (lib->d_pL) hipFree(lib->d_pL);
-    if (lib->d_pA) hipFree(lib->d_pA);
-    if (lib->d_pB) hipFree(lib->d_pB);
-    if (lib->d_pidx) hipFree(lib->d_pidx);
-    if (lib->d_box) hipFree(lib->d_box);
+    if (lib->d_tables) hipFree(lib->d_tables);
+    lib->d_tables = nullptr;
     lib->d_pL = lib->d_pA = lib->d_pB = nullptr;
     lib->d_pidx = nullptr;
     lib->d_box = nullptr;
@@ -493,10 +493,9 @@ void library_release(mh_library* lib) {
     lib->d_lab4 = nullptr;
     lib->d_L = lib->d_A = lib->d_B = lib->d_sim = nullptr;
     lib->d_pixels = nullptr;
-    for (PixelGroup& g : lib->groups) {
-        if (g.d_index) hipFree(g.d_index);
-        g.d_index = nullptr;
-    }
+    if (lib->d_index) hipFree(lib->d_index);
+    lib->d_index = nullptr;
+    for (PixelGroup& g : lib->groups) g.d_index = nullptr;
     for (auto& kv : lib->tiles) {
         if (kv.second.tiles) hipFree(kv.second.tiles);
         if (kv.second.avg) hipFree(kv.second.avg);
@@ -585,6 +584,7 @@ void mh_context_destroy(mh_context* ctx) {
         for (mh_batch* b : batches) batch_release(b);
         for (mh_library* lib : libs) library_release(lib);
     }
+    stage_release(ctx);
     for (auto& b : ctx->slots)
         if (b.p) hipFree(b.p);
     for (auto& kv : ctx->temps)
@@ -741,12 +741,22 @@ static int library_alloc(mh_context* ctx, int32_t n, mh_library** out) {
     }
     lib->n = n;
     lib->h_lab.assign((size_t)n * 3, 0.0f);
-    const size_t m = n > 0 ? (size_t)n : 1;
-    hipError_t e = hipMalloc(&lib->d_lab4, sizeof(float4) * m);
-    if (e == hipSuccess) e = hipMalloc(&lib->d_L, sizeof(float) * m);
-    if (e == hipSuccess) e = hipMalloc(&lib->d_A, sizeof(float) * m);
-    if (e == hipSuccess) e = hipMalloc(&lib->d_B, sizeof(float) * m);
-    if (e != hipSuccess) {
+    // one allocation: the Lab table, its three columns, and the block layout
+    // (library_upload_lab fills it the same way)
+    const size_t m = n > 0 ? (size_t)n : 1, nb = (m + 63) / 64, slots = nb * 64;
+    const size_t bytes = sizeof(float4) * (m + 2 * nb) + sizeof(float) * (3 * m + 4 * slots);
+    hipError_t e = hipMalloc(&lib->d_tables, bytes);
+    if (e == hipSuccess) {
+        lib->d_lab4 = static_cast<float4*>(lib->d_tables);
+        lib->d_box = lib->d_lab4 + m;
+        lib->d_L = reinterpret_cast<float*>(lib->d_box + 2 * nb);
+        lib->d_A = lib->d_L + m;
+        lib->d_B = lib->d_A + m;
+        lib->d_pL = lib->d_B + m;
+        lib->d_pA = lib->d_pL + slots;
+        lib->d_pB = lib->d_pA + slots;
+        lib->d_pidx = reinterpret_cast<int32_t*>(lib->d_pB + slots);
+    } else {
         mh_library_destroy(lib);
         return fail(e == hipErrorOutOfMemory ? MH_ERR_OUT_OF_MEMORY : MH_ERR_HIP, "library alloc: %s",
                     hipGetErrorString(e));
@@ -760,7 +770,8 @@ static int library_alloc(mh_context* ctx, int32_t n, mh_library** out) {
 // of widest extent, until a range is one block; ties on the axis value go
 // by material index, so the layout is a function of the Labs alone.  Only
 // the last block can be partial.
-static int library_build_blocks(mh_library* lib) {
+static void library_build_blocks(const mh_library* lib, float4* box, float* pl, float* pa, float* pb,
+                                 int32_t* pidx) {
     const int32_t n = lib->n;
     const int32_t nb = (n + 63) / 64;
     const float* lab = lib->h_lab.data();
@@ -791,10 +802,6 @@ static int library_build_blocks(mh_library* lib) {
         todo.push_back({lo, mid});
         todo.push_back({mid, hi});
     }
-    const size_t slots = (size_t)(nb > 0 ? nb : 1) * 64;
-    std::vector<float> pl(slots, 0.0f), pa(slots, 0.0f), pb(slots, 0.0f);
-    std::vector<int32_t> pidx(slots, -1);
-    std::vector<float4> box((size_t)(nb > 0 ? nb : 1) * 2, make_float4(0, 0, 0, 0));
     for (int32_t b = 0; b < nb; ++b) {
         float4 lo4 = make_float4(INFINITY, INFINITY, INFINITY, 0.0f);
         float4 hi4 = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.0f);
@@ -815,49 +822,38 @@ static int library_build_blocks(mh_library* lib) {
         box[2 * (size_t)b] = lo4;
         box[2 * (size_t)b + 1] = hi4;
     }
-    hipError_t e = hipMalloc(&lib->d_pL, sizeof(float) * slots);
-    if (e == hipSuccess) e = hipMalloc(&lib->d_pA, sizeof(float) * slots);
-    if (e == hipSuccess) e = hipMalloc(&lib->d_pB, sizeof(float) * slots);
-    if (e == hipSuccess) e = hipMalloc(&lib->d_pidx, sizeof(int32_t) * slots);
-    if (e == hipSuccess) e = hipMalloc(&lib->d_box, sizeof(float4) * box.size());
-    if (e == hipSuccess) e = hipMemcpy(lib->d_pL, pl.data(), sizeof(float) * slots, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(lib->d_pA, pa.data(), sizeof(float) * slots, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(lib->d_pB, pb.data(), sizeof(float) * slots, hipMemcpyHostToDevice);
-    if (e == hipSuccess)
-        e = hipMemcpy(lib->d_pidx, pidx.data(), sizeof(int32_t) * slots, hipMemcpyHostToDevice);
-    if (e == hipSuccess)
-        e = hipMemcpy(lib->d_box, box.data(), sizeof(float4) * box.size(), hipMemcpyHostToDevice);
-    if (e != hipSuccess)
-        return fail(e == hipErrorOutOfMemory ? MH_ERR_OUT_OF_MEMORY : MH_ERR_HIP,
-                    "material blocks: %s", hipGetErrorString(e));
-    lib->nb = nb;
-    return MH_OK;
 }
 
+// Fills lib->d_tables from the Labs.
 static int library_upload_lab(mh_library* lib) {
     const int32_t n = lib->n;
     if (n == 0) return MH_OK;
-    std::vector<float4> l4((size_t)n);
-    std::vector<float> L((size_t)n), A((size_t)n), B((size_t)n);
+    const size_t nb = ((size_t)n + 63) / 64, slots = nb * 64;
+    std::vector<uint8_t> tables(sizeof(float4) * ((size_t)n + 2 * nb) +
+                                sizeof(float) * (3 * (size_t)n + 4 * slots));
+    float4* l4 = reinterpret_cast<float4*>(tables.data());
+    float4* box = l4 + n;
+    float *L = reinterpret_cast<float*>(box + 2 * nb), *A = L + n, *B = A + n;
+    float *pl = B + n, *pa = pl + slots, *pb = pa + slots;
+    int32_t* pidx = reinterpret_cast<int32_t*>(pb + slots);
     for (int32_t i = 0; i < n; ++i) {
         L[i] = lib->h_lab[3 * i];
         A[i] = lib->h_lab[3 * i + 1];
         B[i] = lib->h_lab[3 * i + 2];
         l4[i] = make_float4(L[i], A[i], B[i], 0.0f);
     }
-    HIPCHK(hipMemcpy(lib->d_lab4, l4.data(), sizeof(float4) * n, hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(lib->d_L, L.data(), sizeof(float) * n, hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(lib->d_A, A.data(), sizeof(float) * n, hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(lib->d_B, B.data(), sizeof(float) * n, hipMemcpyHostToDevice));
-    CHK(library_build_blocks(lib));
+    for (size_t i = n; i < slots; ++i) pidx[i] = -1;  // (padding)
+    library_build_blocks(lib, box, pl, pa, pb, pidx);
+    lib->nb = (int32_t)nb;
+    HIPCHK(hipMemcpyAsync(lib->d_tables, tables.data(), tables.size(), hipMemcpyHostToDevice,
+                          lib->ctx->stream));
     // largest adjacency terms, for the placement's prepared lists (a library
     // that has none in the narrowest grid does not read them)
     if (place_raster_lds_bytes(1, n, kRasterLists) <= lib->ctx->max_lds) {
         launch_near_terms(lib->d_lab4, n, lib->ctx->stream);
         HIPCHK(hipGetLastError());
-        HIPCHK(hipStreamSynchronize(lib->ctx->stream));
     }
-    return MH_OK;
+    return sync(lib->ctx);  // (any stream may read the tables; `tables` is pageable and local)
 }
 
 int mh_library_from_lab(mh_context* ctx, const float* lab, int32_t n, mh_library** out) {
@@ -889,10 +885,16 @@ int mh_library_from_pixels(mh_context* ctx, const uint8_t* rgb, int32_t n, int32
     if (n > 0) lib->groups.push_back(PixelGroup{w, h, n, 0, nullptr});
     int rc = MH_OK;
     hipError_t e = hipMalloc(&lib->d_pixels, bytes ? bytes : 16);
-    if (e == hipSuccess && bytes) e = hipMemcpy(lib->d_pixels, rgb, bytes, hipMemcpyHostToDevice);
-    if (e != hipSuccess) {
+    if (e == hipSuccess && bytes) {
+        if (staged(rgb, bytes))
+            rc = stage_upload(ctx, lib->d_pixels, {HostSpan{rgb, bytes}});
+        else
+            e = hipMemcpyAsync(lib->d_pixels, rgb, bytes, hipMemcpyHostToDevice, ctx->stream);
+    }
+    if (e != hipSuccess) rc = fail(MH_ERR_HIP, "library pixels: %s", hipGetErrorString(e));
+    if (rc) {
         mh_library_destroy(lib);
-        return fail(MH_ERR_HIP, "library pixels: %s", hipGetErrorString(e));
+        return rc;
     }
     if (n > 0) {
         float* d_lab = nullptr;
@@ -963,20 +965,18 @@ static int ragged_plan(const uint8_t* rgb, const int64_t* offsets, const int32_t
     return MH_OK;
 }
 
-// Packs the images in slot order and copies them to d_dst (p.bytes bytes).
+// Copies the images in slot order to d_dst (p.bytes bytes), back to back.
 static int ragged_upload(mh_context* ctx, const uint8_t* rgb, const int64_t* offsets,
                          const RaggedPlan& p, uint8_t* d_dst) {
-    if (p.bytes == 0) return MH_OK;
-    std::vector<uint8_t> pack(p.bytes);
+    std::vector<HostSpan> spans;
+    spans.reserve(p.slot_image.size());
     for (size_t g = 0; g < p.groups.size(); ++g) {
         const PixelGroup& pg = p.groups[g];
         const size_t img = (size_t)pg.w * pg.h * 3;
         for (int32_t k = 0; k < pg.count; ++k)
-            memcpy(pack.data() + pg.offset + k * img, rgb + offsets[p.slot_image[p.group_first[g] + k]],
-                   img);
+            spans.push_back(HostSpan{rgb + offsets[p.slot_image[p.group_first[g] + k]], img});
     }
-    HIPCHK(hipMemcpyAsync(d_dst, pack.data(), p.bytes, hipMemcpyHostToDevice, ctx->stream));
-    return sync(ctx);  // `pack` is pageable and local
+    return stage_upload(ctx, d_dst, spans);
 }
 
 // calculate_average_lab of every packed image (one batched launch, one
@@ -1043,19 +1043,21 @@ int mh_library_from_images(mh_context* ctx, const uint8_t* rgb, const int64_t* o
     if (e != hipSuccess)
         rc = fail(e == hipErrorOutOfMemory ? MH_ERR_OUT_OF_MEMORY : MH_ERR_HIP, "library pixels: %s",
                   hipGetErrorString(e));
+    // the index maps (slot -> image), but for a group that is images 0, 1, ...
+    if (!rc && n > 0) {
+        e = hipMalloc(&lib->d_index, sizeof(int32_t) * (size_t)n);
+        if (e == hipSuccess)
+            e = hipMemcpyAsync(lib->d_index, p.slot_image.data(), sizeof(int32_t) * (size_t)n,
+                               hipMemcpyHostToDevice, ctx->stream);
+        if (e != hipSuccess) rc = fail(MH_ERR_HIP, "library index: %s", hipGetErrorString(e));
+    }
     for (size_t g = 0; g < p.groups.size() && !rc; ++g) {
         PixelGroup pg = p.groups[g];
         const int32_t* idx = p.slot_image.data() + p.group_first[g];
         bool identity = p.group_first[g] == 0;
         for (int32_t k = 0; k < pg.count && identity; ++k) identity = idx[k] == k;
-        if (!identity) {
-            e = hipMalloc(&pg.d_index, sizeof(int32_t) * pg.count);
-            if (e == hipSuccess)
-                e = hipMemcpy(pg.d_index, idx, sizeof(int32_t) * pg.count, hipMemcpyHostToDevice);
-            if (e != hipSuccess)
-                rc = fail(MH_ERR_HIP, "library index: %s", hipGetErrorString(e));
-        }
-        lib->groups.push_back(pg);  // owned by the library even on failure
+        if (!identity) pg.d_index = lib->d_index + p.group_first[g];
+        lib->groups.push_back(pg);
     }
     if (!rc) rc = ragged_upload(ctx, rgb, offsets, p, lib->d_pixels);
     if (!rc) rc = ragged_lab(ctx, lib->d_pixels, p, lib->h_lab.data());

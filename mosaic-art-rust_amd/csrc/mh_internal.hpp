@@ -60,6 +60,18 @@ struct TapsBuf {
     int32_t prec = 0;
 };
 
+// Large host copies (mh_stage.hip): pinned buffers, two for each thread that
+// copies, made on first use and kept by the context (24 MiB in all).
+constexpr int kStageThreads = 3;
+struct StageBuf {
+    uint8_t* p = nullptr;
+    hipEvent_t copied = nullptr;  // the last copy from or to it
+};
+struct HostSpan {
+    const uint8_t* p;
+    size_t bytes;
+};
+
 struct PhaseMark {
     int32_t phase;
     hipEvent_t a, b;
@@ -75,6 +87,8 @@ struct mh_context {
     // them afterwards only frees host memory
     std::vector<mh_library*> libs;
     std::vector<mh_batch*> batches;
+    mh::host::StageBuf stage[2 * mh::host::kStageThreads];
+    std::mutex stage_mu;
     std::mutex dep_mu;
     // per-phase timing (HIP events on `stream`)
     uint32_t timing = 0;  // bit p: phase p is bracketed by events
@@ -120,6 +134,7 @@ struct mh_library {
     mh_context* ctx = nullptr;
     int32_t n = 0;
     std::vector<float> h_lab;  // n x 3
+    void* d_tables = nullptr;  // one allocation for the ten arrays below
     float4* d_lab4 = nullptr;
     float* d_L = nullptr;
     float* d_A = nullptr;
@@ -133,6 +148,7 @@ struct mh_library {
     int32_t nb = 0;
     float* d_sim = nullptr;    // n x n after build_similarities
     uint8_t* d_pixels = nullptr;
+    int32_t* d_index = nullptr;  // the groups' index maps
     std::vector<PixelGroup> groups;  // materials grouped by size (empty: Labs only)
     // lazily built device caches (resized tiles per cell size)
     std::mutex cache_mu;
@@ -152,6 +168,13 @@ int set_device(mh_context* ctx);
 void phase_begin(mh_context* ctx, int phase);
 void phase_end(mh_context* ctx, int phase);
 int ensure(mh_context* ctx, DevBuf& b, size_t bytes);
+// Whether a copy of pageable host memory goes through the pinned buffers.
+bool staged(const void* host, size_t bytes);
+// The spans, back to back, to dst: queued on the stream, the spans read.
+int stage_upload(mh_context* ctx, uint8_t* dst, const std::vector<HostSpan>& spans);
+// After everything queued on the stream: copied, host written.
+int stage_download(mh_context* ctx, uint8_t* host, const uint8_t* src, size_t bytes);
+void stage_release(mh_context* ctx);
 bool finite3(const float* v, int64_t count);
 int get_taps(mh_context* ctx, int32_t in_size, int32_t out_size, ResizeTaps* t);
 // Device memory of a library / batch freed, the handle detached from its

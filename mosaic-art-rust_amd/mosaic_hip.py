@@ -353,9 +353,9 @@ class Context:
 
     def average_lab_many(self, images):
         """calculate_average_lab of each RGB8 image (list of h x w x 3)."""
-        buf, off, w, h = _pack_images(images)
+        keep, base, off, w, h = _image_table(images)
         out = np.zeros((len(images), 3), np.float32)
-        _check(self.lib.mh_average_lab_many(self.h, _ptr(buf), _ptr(off), _ptr(w), _ptr(h),
+        _check(self.lib.mh_average_lab_many(self.h, base, _ptr(off), _ptr(w), _ptr(h),
                                             len(images), _ptr(out)))
         return out
 
@@ -523,17 +523,15 @@ class Context:
         return Server(self, memory_budget, max_batch, streams)
 
 
-def _pack_images(images):
-    """Concatenates RGB8 images into one buffer: (bytes, offsets, widths, heights)."""
+def _image_table(images):
+    """RGB8 images where they lie: (arrays, base address, offsets from it, widths, heights).
+    The arrays must outlive the call that gets the table."""
     arrs = [_c(im, np.uint8) for im in images]
-    off = np.zeros(len(arrs), np.int64)
-    w = np.array([a.shape[1] for a in arrs], np.int32)
+    at = np.array([a.__array_interface__["data"][0] for a in arrs], np.int64)
+    base = int(at.min()) if arrs else 0
     h = np.array([a.shape[0] for a in arrs], np.int32)
-    sizes = np.array([a.size for a in arrs], np.int64)
-    if len(arrs):
-        off[1:] = np.cumsum(sizes)[:-1]
-    buf = np.concatenate([a.reshape(-1) for a in arrs]) if arrs else np.zeros(1, np.uint8)
-    return buf, off, w, h
+    w = np.array([a.shape[1] for a in arrs], np.int32)
+    return arrs, ctypes.c_void_p(base), at - base, w, h
 
 
 class Library:
@@ -544,8 +542,8 @@ class Library:
         self.lib = ctx.lib
         h = ctypes.c_void_p()
         if images is not None:
-            buf, off, w, hh = _pack_images(images)
-            _check(self.lib.mh_library_from_images(ctx.h, _ptr(buf), _ptr(off), _ptr(w), _ptr(hh),
+            keep, base, off, w, hh = _image_table(images)
+            _check(self.lib.mh_library_from_images(ctx.h, base, _ptr(off), _ptr(w), _ptr(hh),
                                                    len(images), ctypes.byref(h)))
         elif pixels is not None:
             px = _c(pixels, np.uint8)
