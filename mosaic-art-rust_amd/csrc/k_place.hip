@@ -237,13 +237,13 @@ __global__ __launch_bounds__(64) void place_chain_kernel(PlaceJob single,
 //
 // Measured, one job at a time, against one wave that did all of it (a step of
 // 450 cycles, a full evaluation in 10% of the cells): 1,500 materials in 80 x
-// 60 cells 905 -> 316 us, 10,000 in 160 x 150 4,957 -> 2,050, 500 in 50 x 28
-// 269 -> 102, 1,000 in 20 x 15 58 -> 32, 777 in 97 x 41 with the GUI score
-// 2,283 -> 525.  A step takes 42-48 ns; 0.6% (1,500 materials) to 16% (GUI
+// 60 cells 905 -> 279 us, 10,000 in 160 x 150 4,957 -> 1,908, 500 in 50 x 28
+// 269 -> 91, 1,000 in 20 x 15 58 -> 31, 777 in 97 x 41 with the GUI score
+// 2,283 -> 495.  A step takes 42-48 ns, and the preparation of two cells 1,450
+// cycles of its wave, about a period; 0.6% (1,500 materials) to 16% (GUI
 // score, whose distances lie closer) of the cells are flagged, at 0.4-1 us.
-// With the device full of other jobs' work the preparation's instructions
-// count: a stream of 5,000 queued jobs is 2% slower for them, one of 512
-// jobs, which is as long as its longest chains, 20% faster.
+// Twelve preparing waves of a cell each: 267 us for the first, and twice the
+// waves beside other jobs' work.
 constexpr int32_t kGroup = 12;       // cells per period
 constexpr int32_t kSlots = 3;        // groups in LDS: worked on, ready, being filled
 constexpr int32_t kPrepWaves = 6;    // two cells each per period
@@ -406,6 +406,23 @@ struct PrepArgs {
     bool penalty;         // weight > 0
 };
 
+// A cell's list has at least this many entries, if its row has them: ranks 64
+// and up are only looked at when fewer of the first 64 are kept (of one of
+// the cells prepared together).  The list's last entry is reached only where
+// the cells since (36 at most) took all before it; the cell then reads its
+// row.  With all ranks in every list 316 us instead of 279 (1,500 materials,
+// 80 x 60 cells).
+constexpr uint32_t kEnough = 8;
+
+// The kept candidates' places in a list in preparation, lanes of `kept` in
+// order from `first`; a 65th place for the others.  (Branch-free: left to
+// itself the compiler puts the counting under an exec mask.)
+__device__ __forceinline__ uint32_t list_place(uint64_t kept, uint32_t first) {
+    uint32_t p = first + lanes_before(kept);
+    asm("" : "+v"(p));
+    return lane_in(kept) ? p : 64u;
+}
+
 // The lists of cells c .. c + kPrepCells - 1, side by side so that their LDS
 // reads are in flight together: a cell's count-limited candidates without the
 // up neighbour up[k] (an entry id, 0: none), the first 64 of them.  An
@@ -415,38 +432,59 @@ struct PrepArgs {
 // fl(2 t w) and its score at most fl(d + fl(2 t w)); a later entry's score is
 // at least its distance.  stage: the candidates kept, by place in the list,
 // {material + 1 | term << 16, distance} (the counts fit LDS, so a material
-// fits 16 bits); those left out go to a 65th place.  Cells past the grid get
-// an empty list.
+// fits 16 bits).  The distances behind a list's end bound those of the row's
+// other candidates from below.  Cells past the grid get an empty list.
 __device__ __forceinline__ void prep_cells(const RawRow (&q)[kPrepCells], int32_t c, int32_t cells,
                                            const uint32_t (&up)[kPrepCells],
                                            const bool (&first)[kPrepCells], const PrepArgs& P,
                                            const ChainShared& S, uint32_t* slot, int32_t k0,
                                            uint32_t* stage, int lane) {
-    uint32_t m0[kPrepCells], m1[kPrepCells], u0[kPrepCells], u1[kPrepCells];
+    uint32_t m0[kPrepCells], u0[kPrepCells];
 #pragma unroll
     for (int k = 0; k < kPrepCells; ++k) {
         m0[k] = (uint32_t)q[k].r0 + 1u;
-        m1[k] = (uint32_t)q[k].r1 + 1u;
         u0[k] = S.counts[m0[k]];
-        u1[k] = S.counts[m1[k]];
     }
-    uint32_t total[kPrepCells];
+    uint64_t b0[kPrepCells];
+    uint32_t total[kPrepCells], n0[kPrepCells];
+    float tail[kPrepCells];
+    bool whole = false;  // the lists hold their rows' every kept candidate, or 64
 #pragma unroll
     for (int k = 0; k < kPrepCells; ++k) {
         // (ranks past the row's end read the guard)
-        const uint32_t um = up[k] >> 2;
-        const uint64_t b0 = lanes_ult(u0[k], P.limit) & lanes_ne((int32_t)m0[k], (int32_t)um);
-        const uint64_t b1 = lanes_ult(u1[k], P.limit) & lanes_ne((int32_t)m1[k], (int32_t)um);
-        const uint32_t n0 = (uint32_t)__popcll(b0);
-        total[k] = c + k < cells ? n0 + (uint32_t)__popcll(b1) : 0u;
-        const uint32_t p0 = lane_in(b0) ? lanes_before(b0) : 64u;
-        const uint32_t p1 = min(lane_in(b1) ? n0 + lanes_before(b1) : 64u, 64u);
-        uint64_t* at = reinterpret_cast<uint64_t*>(stage + k * kStageWords);
-        const uint32_t t0 = P.packed ? u0[k] << 16 : 0x3f800000u;
-        const uint32_t t1 = P.packed ? u1[k] << 16 : 0x3f800000u;
-        at[p0] = (q[k].r0 & 0xffffffff00000000ull) | (t0 | m0[k]);
-        at[p1] = (q[k].r1 & 0xffffffff00000000ull) | (t1 | m1[k]);
+        b0[k] = lanes_ult(u0[k], P.limit) & lanes_ne((int32_t)m0[k], (int32_t)(up[k] >> 2));
+        n0[k] = (uint32_t)__popcll(b0[k]);
+        total[k] = n0[k];
+        whole = whole || n0[k] < kEnough;
     }
+#pragma unroll
+    for (int k = 0; k < kPrepCells; ++k) {
+        const uint32_t t0 = P.packed ? u0[k] << 16 : 0x3f800000u;
+        uint64_t* at = reinterpret_cast<uint64_t*>(stage + k * kStageWords);
+        at[list_place(b0[k], 0u)] = (q[k].r0 & 0xffffffff00000000ull) | (t0 | m0[k]);
+        tail[k] = readlane_f(__uint_as_float((uint32_t)(q[k].r1 >> 32)), 0);
+    }
+    if (whole) {
+        uint32_t m1[kPrepCells], u1[kPrepCells];
+#pragma unroll
+        for (int k = 0; k < kPrepCells; ++k) {
+            m1[k] = (uint32_t)q[k].r1 + 1u;
+            u1[k] = S.counts[m1[k]];
+        }
+#pragma unroll
+        for (int k = 0; k < kPrepCells; ++k) {
+            const uint64_t b1 =
+                lanes_ult(u1[k], P.limit) & lanes_ne((int32_t)m1[k], (int32_t)(up[k] >> 2));
+            const uint32_t t1 = P.packed ? u1[k] << 16 : 0x3f800000u;
+            uint64_t* at = reinterpret_cast<uint64_t*>(stage + k * kStageWords);
+            at[min(list_place(b1, n0[k]), 64u)] =
+                (q[k].r1 & 0xffffffff00000000ull) | (t1 | m1[k]);
+            total[k] = n0[k] + (uint32_t)__popcll(b1);
+            tail[k] = __builtin_inff();
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < kPrepCells; ++k) total[k] = c + k < cells ? total[k] : 0u;
     asm volatile("" ::: "memory");  // (a wave's LDS operations are done in order)
     uint64_t e[kPrepCells];
     float dn[kPrepCells];
@@ -461,18 +499,19 @@ __device__ __forceinline__ void prep_cells(const RawRow (&q)[kPrepCells], int32_
 #pragma unroll
     for (int k = 0; k < kPrepCells; ++k) {
         const uint32_t x = (uint32_t)e[k];
+        const uint64_t in = lanes_ult((uint32_t)lane, total[k]);
         const float d = __uint_as_float((uint32_t)(e[k] >> 32));
         const float reach = d + __uint_as_float(x & 0xffff0000u) * P.w2;
-        const uint64_t in = lanes_ult((uint32_t)lane, total[k]);
-        // safe: the last of the list, or the next beyond reach (with no
-        // penalty, always)
-        uint64_t safe = in & ~(in >> 1);
-        safe |= P.penalty ? in & __builtin_amdgcn_fcmpf(dn[k], reach, 2) : in;  // >
+        // safe: the next beyond reach, or none next (with no penalty, always)
+        const uint64_t next = in >> 1;
+        uint64_t safe = in & next & __builtin_amdgcn_fcmpf(dn[k], reach, 2);  // >
+        safe |= whole ? in & ~next : 0ull;
+        safe = P.penalty ? safe : in;
         safe &= 0x7fffffffffffffffull;
         const uint32_t common = first[k] ? kFlagged | kFirst : 0u;
         const uint32_t a = lane_in(in) ? (x & 0xffffu) << 2 : 0u;
         slot[entry_word(k0 + k, lane)] = a | common | (lane_in(safe) ? 0u : kFlagged | kUnsafe);
-        slot[dist_word(k0 + k, lane)] = __float_as_uint(d);
+        slot[dist_word(k0 + k, lane)] = __float_as_uint(lane_in(in) ? d : tail[k]);
     }
 }
 
@@ -750,8 +789,8 @@ __device__ __forceinline__ bool decide_from_list(const PlaceJob& job, uint32_t a
     if (!(job.weight > 0.0f)) return true;  // scores are the distances
     const float est = score_estimate(d, lab, nb, job.weight);
     const float far = rival_bound(readlane_f(est, f), job.weight);
-    // a full list may go on within reach
-    if (readlane_u(a, 63) != 0u && !(readlane_f(d, 63) > far)) return false;
+    // the row may go on within reach
+    if (!(readlane_f(d, 63) > far)) return false;
     const uint64_t field = usable & wave_ballot(!(est > far));  // f and its rivals
     if (field == (1ull << f)) return true;
     const bool in = lane_in(field | (1ull << f));
