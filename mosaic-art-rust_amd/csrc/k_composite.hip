@@ -254,37 +254,67 @@ void launch_cell_adjust(const int32_t* grid, int32_t cells, const uint8_t* tile_
 // each channel value (contrast1_entry); blocks copy it to LDS.
 __device__ const Contrast1Table kContrast1 = make_contrast1_table();
 
-// Pixels per thread: a block of bs threads covers kPx * bs pixels of one
-// output row, pixel X = X0 + k * bs (k < kPx), so the row's setup is shared
-// by kPx pixels per thread and every k-step stores a contiguous run.  One
-// job's launch (a few Mpx) takes 4, so that its blocks fill the device; the
-// batched launch, with many jobs' rows, takes 8, which halves the per-thread
-// share of the setup (segment search, row and column divisions, the table
-// copy): the served stream 57.3k -> 59.0k jobs/s, against 16.9 us instead
-// of 14.9 us for a medium job's own launch.  12 and 16 pixels per thread
-// lose more to idle lanes at the ends of short rows than they save (57.0k
-// and 54.5-55.0k jobs/s).
-constexpr int32_t kCompPxJob = 4;
-constexpr int32_t kCompPxBatch = 8;
+// The composite goes by quads: up to four neighbouring pixels of one cell's row
+// of the output, by one thread.  They share the cell's material and adjustment,
+// and their 12 bytes are one load from the tile and one store, where a thread
+// to a pixel had two loads of each and three stores (the address unit takes a
+// wave's 64 scattered lanes one after another, whatever their size).  A row of
+// a cell is (tw + 3) / 4 quads, the last of them short where tw is no multiple
+// of 4.  Bound by VALU issue (the colour adjustment).
+// Measured, a thread to a pixel before: 1,920 x 1,080 with 24 x 24 cells 14.4 ->
+// 11.7 us, 4,000 x 2,400 with 20 x 20 cells 40.7 -> 31.9, 3,914 x 2,204 with 19 x
+// 19 cells (a twentieth of the lanes idle) 38.2 -> 34.8, all with 4 us of
+// launch; a stream of 5,000 queued jobs, whose composites were a third of its
+// instructions, 60.0k -> 66.0k jobs/s.
+//
+// A thread does kQuads quads, bs apart (a block of bs threads): one job's
+// launch (a few Mpx) takes 1, so that its blocks fill the device; the batched
+// launch, with many jobs' rows, 2, which halves the per-thread share of the
+// setup (segment search, row division, the table copy).
+constexpr int32_t kQuadsJob = 1;
+constexpr int32_t kQuadsBatch = 2;
 
-static int32_t composite_row_blocks(int32_t ow, int32_t oh, int32_t threads, int32_t px) {
-    return ow > 0 && oh > 0 ? ((ow + threads * px - 1) / (threads * px)) * oh : 0;
+__host__ __device__ __forceinline__ int32_t cell_quads(int32_t tw) { return (tw + 3) / 4; }
+
+static int32_t composite_row_blocks(int32_t gw, int32_t tw, int32_t oh, int32_t threads,
+                                    int32_t quads) {
+    const int32_t row = gw * cell_quads(tw);
+    return row > 0 && oh > 0 ? ((row + threads * quads - 1) / (threads * quads)) * oh : 0;
 }
 
-// Block b of segment s: row Y = b / per_row of the gw*tw x gh*th mosaic,
-// pixels X0 + k * bs with X0 = (b % per_row) * bs * kCompPx + thread and
-// per_row = ceil(ow / (bs * kCompPx)), ow = gw * tw.  Everything about the
-// row is uniform: its cell row's grid entries and adjustments, the tiles'
-// pixel row dy = Y % th, the output row.  A thread divides once for its
-// first pixel's cell column cx and byte column dx3 = 3 (X0 - cx tw) and steps
-// the others by bs = q tw + r.  kNarrow: every material index and the tile
-// size th tw 3 are below 2^24 and n th tw 3 < 2^32 (composite_narrow), so a
-// tile byte offset is one 24-bit multiply-add; otherwise 64-bit.
-template <bool kNarrow, int32_t kCompPx>
+// Twelve bytes at any address (a tile's last row is readable to the end of
+// its last quad).
+struct Quad {
+    uint32_t w[3];
+};
+__device__ __forceinline__ Quad load_quad(const uint8_t* p) {
+    typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
+    typedef u32x3 u32x3_any __attribute__((aligned(1)));
+    const u32x3 v = *(const MH_GAS u32x3_any*)p;
+    return Quad{{v.x, v.y, v.z}};
+}
+__device__ __forceinline__ void store_quad(uint8_t* p, const Quad& q) {
+    typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
+    typedef u32x3 u32x3_any __attribute__((aligned(1)));
+    *(MH_GAS u32x3_any*)p = u32x3{q.w[0], q.w[1], q.w[2]};
+}
+__device__ __forceinline__ uint32_t quad_byte(const Quad& q, int i) {
+    return q.w[i >> 2] >> (8 * (i & 3)) & 0xffu;
+}
+
+// Block b of segment s: row Y = b / per_row of the gw*tw x gh*th mosaic, quads
+// Q0 + k * bs with Q0 = (b % per_row) * bs * kQuads + thread and per_row =
+// ceil(row quads / (bs * kQuads)).  Everything about the row is uniform: its
+// cell row's grid entries and adjustments, the tiles' pixel row dy = Y % th,
+// the output row.  kNarrow: every material index and the tile size th tw 3 are
+// below 2^24 and n th tw 3 < 2^32 (composite_narrow), so a tile byte offset is
+// one 24-bit multiply-add; otherwise 64-bit.
+template <bool kNarrow, int32_t kQuads>
 __device__ __forceinline__ void composite_block(const CompSeg& s, int32_t b, float* ctab) {
-    const int32_t tw = s.tw, th = s.th, ow = s.gw * tw;
+    const int32_t tw = s.tw, th = s.th;
+    const int32_t qpc = cell_quads(tw), row = s.gw * qpc;
     const int32_t bs = (int32_t)blockDim.x;
-    const int32_t per_row = (ow + bs * kCompPx - 1) / (bs * kCompPx);
+    const int32_t per_row = (row + bs * kQuads - 1) / (bs * kQuads);
     const int32_t Y = b / per_row;
     const int32_t cy = Y / th, dy = Y - cy * th;
     const int64_t row_cell = (int64_t)cy * s.gw;
@@ -292,7 +322,7 @@ __device__ __forceinline__ void composite_block(const CompSeg& s, int32_t b, flo
     const float4* __restrict__ adj = s.adjust ? s.adj + row_cell : nullptr;
     const uint32_t tile_bytes = (uint32_t)th * (uint32_t)tw * 3u;
     const uint8_t* __restrict__ tiles = s.tiles + (int64_t)dy * tw * 3;
-    uint8_t* __restrict__ out = s.out + (int64_t)Y * ow * 3;
+    uint8_t* __restrict__ out = s.out + (int64_t)Y * s.gw * tw * 3;
     if (s.adjust) {
         // blockDim.x >= 64: one float4 of the table per thread of the first 64
         if (threadIdx.x < 64)
@@ -300,98 +330,92 @@ __device__ __forceinline__ void composite_block(const CompSeg& s, int32_t b, flo
                 gload4(reinterpret_cast<const float4*>(kContrast1.v), threadIdx.x);
         __syncthreads();
     }
-    const int32_t X0 = (b - Y * per_row) * bs * kCompPx + (int32_t)threadIdx.x;
-    // the pixels go through in stages, so that each stage's loads are in
-    // flight together: cells, then tile pixels and adjustments, then the
+    const int32_t Q0 = (b - Y * per_row) * bs * kQuads + (int32_t)threadIdx.x;
+    // Q / qpc as umulhi(Q, floor((2^32 - 1) / qpc) + 1), exact while
+    // Q * qpc < 2^32 (then Q m / 2^32 exceeds Q / qpc by less than 1 / qpc)
+    const uint32_t magic = 0xffffffffu / (uint32_t)qpc + 1u;
+    const bool magic_ok = ((uint64_t)(uint32_t)row + (uint32_t)(bs * kQuads)) * (uint32_t)qpc < (1ull << 32);
+    // the quads go through in stages, so that each stage's loads are in
+    // flight together: cells, then tile bytes and adjustments, then the
     // arithmetic and stores
-    int32_t m[kCompPx], cxk[kCompPx];
-    uint32_t dxk[kCompPx];
-    {
-        // X0 / tw as umulhi(X0, floor((2^32 - 1) / tw) + 1), exact while
-        // X0 * tw < 2^32 (then X0 m / 2^32 exceeds X0 / tw by less than 1 / tw)
-        const uint32_t tw_magic = 0xffffffffu / (uint32_t)tw + 1u;
-        const bool magic_ok =
-            (uint64_t)((uint32_t)ow + (uint32_t)(bs * kCompPx)) * (uint32_t)tw < (1ull << 32);
-        int32_t cx = magic_ok ? (int32_t)__umulhi((uint32_t)X0, tw_magic)
-                              : (int32_t)((uint32_t)X0 / (uint32_t)tw);
-        uint32_t dx3 = (uint32_t)(X0 - cx * tw) * 3u;
-        const int32_t q = bs / tw;
-        const uint32_t r3 = (uint32_t)(bs - q * tw) * 3u, tw3 = (uint32_t)tw * 3u;
+    int32_t m[kQuads], cx[kQuads], px[kQuads];
 #pragma unroll
-        for (int32_t k = 0; k < kCompPx; ++k) {
-            cxk[k] = cx;
-            dxk[k] = dx3;
-            m[k] = X0 + k * bs < ow ? gload_at(grid, (uint32_t)cx * 4u) : kEmpty;
-            cx += q;
-            dx3 += r3;
-            if (dx3 >= tw3) {
-                dx3 -= tw3;
-                ++cx;
-            }
-        }
+    for (int32_t k = 0; k < kQuads; ++k) {
+        const int32_t q = Q0 + k * bs;
+        // (one quad to a cell: the magic number would be 2^32)
+        cx[k] = qpc == 1 ? q
+                         : (magic_ok ? (int32_t)__umulhi((uint32_t)q, magic)
+                                     : (int32_t)((uint32_t)q / (uint32_t)qpc));
+        px[k] = 4 * (q - cx[k] * qpc);
+        m[k] = q < row ? gload_at(grid, (uint32_t)cx[k] * 4u) : kEmpty;
     }
-    // a pixel's red and green bytes as one (unaligned) 16-bit load, blue
-    // alone; the raw loaded values are kept until the last stage, so no
-    // wait is needed before the next pixel's loads
-    typedef uint16_t u16_any __attribute__((aligned(1)));
-    uint32_t rg[kCompPx], bk[kCompPx];
-    v4f_t av[kCompPx];
+    Quad in[kQuads];
+    v4f_t av[kQuads];
 #pragma unroll
-    for (int32_t k = 0; k < kCompPx; ++k) {
-        rg[k] = 0u;
-        bk[k] = 0u;
+    for (int32_t k = 0; k < kQuads; ++k) {
+        in[k] = Quad{{0u, 0u, 0u}};
         av[k] = v4f_t{0.0f, 1.0f, 0.0f, 1.0f};
         if (m[k] != kEmpty) {
-            const MH_GAS uint8_t* p =
-                kNarrow ? (const MH_GAS uint8_t*)tiles + (__umul24((uint32_t)m[k], tile_bytes) + dxk[k])
-                        : (const MH_GAS uint8_t*)tiles + ((int64_t)m[k] * tile_bytes + (int64_t)dxk[k]);
-            rg[k] = *(const MH_GAS u16_any*)p;
-            bk[k] = p[2];
-            if (s.adjust) av[k] = gload_at(reinterpret_cast<const v4f_t*>(adj), (uint32_t)cxk[k] * 16u);
+            const uint32_t at = (uint32_t)px[k] * 3u;
+            in[k] = load_quad(kNarrow ? tiles + (__umul24((uint32_t)m[k], tile_bytes) + at)
+                                      : tiles + ((int64_t)m[k] * tile_bytes + (int64_t)at));
+            if (s.adjust) av[k] = gload_at(reinterpret_cast<const v4f_t*>(adj), (uint32_t)cx[k] * 16u);
         }
     }
 #pragma unroll
-    for (int32_t k = 0; k < kCompPx; ++k) {
-        const int32_t X = X0 + k * bs;
-        if (X < ow) {
-            uint32_t r = rg[k] & 0xffu, g = rg[k] >> 8, bl = bk[k];
-            // per-cell adjustments come from calculate_optimal_adjustment and
-            // ColorAdjustment::new's clamps (cell_adjust_one), whose contrast
-            // is always 1
-            if (m[k] != kEmpty && s.adjust) {
-                const float4 a = make_float4(av[k].x, av[k].y, av[k].z, av[k].w);
-                float br, bg, bb;
-                if (a.y == 1.0f) {
-                    br = clamp_unit(ctab[r] + a.x);
-                    bg = clamp_unit(ctab[g] + a.x);
-                    bb = clamp_unit(ctab[bl] + a.x);
-                } else {
-                    br = bright_contrast<true>(u8_unit(r), a.x, a.y);
-                    bg = bright_contrast<true>(u8_unit(g), a.x, a.y);
-                    bb = bright_contrast<true>(u8_unit(bl), a.x, a.y);
+    for (int32_t k = 0; k < kQuads; ++k) {
+        if (Q0 + k * bs >= row) continue;
+        Quad o = in[k];
+        // per-cell adjustments come from calculate_optimal_adjustment and
+        // ColorAdjustment::new's clamps (cell_adjust_one), whose contrast
+        // is always 1
+        if (m[k] != kEmpty && s.adjust) {
+            const float4 a = make_float4(av[k].x, av[k].y, av[k].z, av[k].w);
+            float r[4], g[4], bl[4];
+            uint32_t c[12];
+            if (a.y == 1.0f) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    r[i] = clamp_unit(ctab[quad_byte(in[k], 3 * i)] + a.x);
+                    g[i] = clamp_unit(ctab[quad_byte(in[k], 3 * i + 1)] + a.x);
+                    bl[i] = clamp_unit(ctab[quad_byte(in[k], 3 * i + 2)] + a.x);
                 }
-                adjust_tail<true>(a, br, bg, bb, r, g, bl);
+            } else {
+                for (int i = 0; i < 4; ++i) {
+                    r[i] = bright_contrast<true>(u8_unit(quad_byte(in[k], 3 * i)), a.x, a.y);
+                    g[i] = bright_contrast<true>(u8_unit(quad_byte(in[k], 3 * i + 1)), a.x, a.y);
+                    bl[i] = bright_contrast<true>(u8_unit(quad_byte(in[k], 3 * i + 2)), a.x, a.y);
+                }
             }
-            MH_GAS uint8_t* d = (MH_GAS uint8_t*)out + (uint32_t)X * 3u;
-            d[0] = (uint8_t)r;
-            d[1] = (uint8_t)g;
-            d[2] = (uint8_t)bl;
+            adjust_four(a, r, g, bl, c);
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+                o.w[i] = c[4 * i] | c[4 * i + 1] << 8 | c[4 * i + 2] << 16 | c[4 * i + 3] << 24;
+        }
+        uint8_t* d = out + (int64_t)((uint32_t)cx[k] * (uint32_t)tw + (uint32_t)px[k]) * 3;
+        const int32_t count = tw - px[k];
+        if (count >= 4) {
+            store_quad(d, o);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 9; ++i)
+                if (i < 3 * count) ((MH_GAS uint8_t*)d)[i] = (uint8_t)quad_byte(o, i);
         }
     }
 }
 
-template <int32_t kPx>
+template <int32_t kQuads>
 __device__ __forceinline__ void composite_run(const CompSeg& s, int32_t b) {
     __shared__ __align__(16) float ctab[256];
     if (s.narrow)
-        composite_block<true, kPx>(s, b, ctab);
+        composite_block<true, kQuads>(s, b, ctab);
     else
-        composite_block<false, kPx>(s, b, ctab);
+        composite_block<false, kQuads>(s, b, ctab);
 }
 
 // One job: blocks of 256 threads.
 __global__ __launch_bounds__(256) void composite_kernel(CompSeg s) {
-    composite_run<kCompPxJob>(s, (int32_t)blockIdx.x);
+    composite_run<kQuadsJob>(s, (int32_t)blockIdx.x);
 }
 
 int32_t composite_narrow(int32_t n_tiles, int32_t tw, int32_t th) {
@@ -405,7 +429,7 @@ int32_t composite_narrow(int32_t n_tiles, int32_t tw, int32_t th) {
 void launch_composite(const int32_t* grid, int32_t gw, int32_t gh, int32_t tw, int32_t th,
                       const uint8_t* tiles, int32_t n_tiles, const float4* adj, int32_t adjust,
                       uint8_t* out, hipStream_t stream) {
-    const int32_t blocks = composite_row_blocks(gw * tw, gh * th, 256, kCompPxJob);
+    const int32_t blocks = composite_row_blocks(gw, tw, gh * th, 256, kQuadsJob);
     if (blocks <= 0) return;
     CompSeg s{};
     s.grid = grid;
@@ -422,7 +446,7 @@ void launch_composite(const int32_t* grid, int32_t gw, int32_t gh, int32_t tw, i
 }
 
 // Batched finish of many jobs: per-cell adjustments (a thread per cell), then
-// compositing (a thread per output pixel).  Block b of a launch belongs to
+// compositing (a thread per quad of output pixels).  Block b of a launch belongs to
 // segment j with starts[j] <= b < starts[j+1]; the host sizes each
 // segment's block count from its cells (adjust) or output pixels (composite).
 __global__ __launch_bounds__(256) void cell_adjust_batch_kernel(const CompSeg* __restrict__ segs,
@@ -435,19 +459,19 @@ __global__ __launch_bounds__(256) void cell_adjust_batch_kernel(const CompSeg* _
     cell_adjust_one(s.grid, c, s.tile_avg, s.target_avg, s.strength, s.adj);
 }
 
-// A block of blockDim.x (64, 128 or 256) threads covers kCompPxBatch pixels
+// A block of blockDim.x (64, 128 or 256) threads covers kQuadsBatch quads
 // per thread of one output row (composite_block).
 __global__ __launch_bounds__(256) void composite_batch_kernel(const CompSeg* __restrict__ segs,
                                                               const int32_t* __restrict__ starts,
                                                               int32_t n_segs) {
     const int32_t j = find_segment(starts, n_segs, blockIdx.x);
-    composite_run<kCompPxBatch>(segs[j], (int32_t)blockIdx.x - starts[j]);
+    composite_run<kQuadsBatch>(segs[j], (int32_t)blockIdx.x - starts[j]);
 }
 
 int32_t cell_adjust_blocks(int32_t cells) { return cells > 0 ? (cells + 255) / 256 : 0; }
 
-int32_t composite_blocks(int32_t ow, int32_t oh, int32_t threads) {
-    return composite_row_blocks(ow, oh, threads, kCompPxBatch);
+int32_t composite_blocks(int32_t gw, int32_t tw, int32_t oh, int32_t threads) {
+    return composite_row_blocks(gw, tw, oh, threads, kQuadsBatch);
 }
 
 void launch_cell_adjust_batch(const CompSeg* d_segs, const int32_t* d_starts, int32_t n_segs,

@@ -283,7 +283,8 @@ int library_tiles(const mh_library* clib, int32_t tw, int32_t th, hipStream_t st
         const size_t n = (size_t)(lib->n > 0 ? lib->n : 1);
         TileSet ts;
         uint8_t* tmp = nullptr;
-        hipError_t e = hipMalloc(&ts.tiles, n * th * tw * 3);
+        // (the composite reads a tile row's last pixels 12 bytes at a time)
+        hipError_t e = hipMalloc(&ts.tiles, n * th * tw * 3 + 16);
         if (e == hipSuccess) e = hipMalloc(&ts.avg, n * 3);
         if (e == hipSuccess) e = hipMalloc(&tmp, tmp_bytes);
         if (e == hipSuccess && lib->n > 0) {

@@ -308,7 +308,7 @@ int build_plan(const std::vector<JobSpec>& specs, const std::vector<uint8_t*>& j
                                   s.adjust ? 1 : 0, adj, image, composite_narrow(s.n, s.tw, s.th)};
         ++p->n_comp;
         adj_blocks += s.adjust ? cell_adjust_blocks(s.cells) : 0;
-        comp_blocks += composite_blocks(s.gw * s.tw, s.gh * s.th, p->comp_threads);
+        comp_blocks += composite_blocks(s.gw, s.tw, s.gh * s.th, p->comp_threads);
     }
     for (size_t h = 0; h < hbm_place.size(); ++h) place[p->n_place_lds + h] = hbm_place[h];
     p->n_anneal = 0;

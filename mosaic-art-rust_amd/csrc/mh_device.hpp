@@ -267,6 +267,21 @@ __device__ __forceinline__ float draw_unit(uint64_t seed, uint64_t it) {
 // (v, 0, 1) is then the same value (+0 below, 1 above, v between).
 __device__ __forceinline__ float clamp_unit(float v) { return __builtin_amdgcn_fmed3f(v, 0.0f, 1.0f); }
 
+// a / b, correctly rounded, for |a| <= b, 2^-60 < b <= 1 and a = 0 or
+// |a| > 2^-90: the hardware's reciprocal corrected by its fused residual is the
+// correctly rounded one (compared for every mantissa, as part of adj_term),
+// and a product with that, corrected once by its exact residual, the quotient
+// (Markstein).  6 instructions; the general division scales for ranges that do
+// not occur here, 12.  (rgb_to_hsv divides differences of values in [0, 1]
+// that are sums with a u8 / 255 table or with 0.5: no nonzero one is below
+// 2^-60.)
+__device__ __forceinline__ float div_unit(float a, float b) {
+    float y = __builtin_amdgcn_rcpf(b);
+    y = __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
+    const float q = a * y;
+    return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+}
+
 // palette Hsv::from_color(Srgb<f32>) (src/color_adjustment.rs:70, :122).
 // kUnit: r, g, b lie in [0, 1] and none is -0 (see adjust_pixel), so the
 // max(., 0) are identities and s, v are clamps of non-negative values.
@@ -302,7 +317,12 @@ __device__ __forceinline__ void rgb_to_hsv(float r, float g, float b, float& h, 
         }
     }
     float hh = 0.0f, ss = 0.0f;
-    if (mx != mn) {
+    if (kUnit) {  // (computed for grey too, and dropped)
+        const bool grey = mx == mn;
+        const float d = mx - mn;
+        hh = grey ? 0.0f : (div_unit(sep, d) + coeff) * 60.0f;
+        ss = grey ? 0.0f : div_unit(d, mx);
+    } else if (mx != mn) {
         float d = mx - mn;
         hh = (sep / d + coeff) * 60.0f;
         ss = d / mx;
@@ -323,9 +343,12 @@ __device__ __forceinline__ float div60_fast(float x) {
     return __builtin_fmaf(r, c, q);
 }
 
+// Hues that div60_fast is not for.
+__device__ __forceinline__ bool tiny_hue(float h) { return h != 0.0f && h < 0x1p-124f; }
+
 // palette Srgb::from_color(Hsv) (src/color_adjustment.rs:76).
 // kUnit: v in [0, 1] and not -0, s in [0, 1], hdeg in [0, 360] and not -0
-// (see adjust_pixel).
+// (see adjust_pixel), and not tiny_hue(hdeg).
 template <bool kUnit = false>
 __device__ __forceinline__ void hsv_to_rgb(float hdeg, float s, float v, float& r, float& g,
                                            float& b) {
@@ -342,7 +365,8 @@ __device__ __forceinline__ void hsv_to_rgb(float hdeg, float s, float v, float& 
         hp = hdeg - floorf(hdeg / 360.0f) * 360.0f;
     }
     float h = div60_fast(hp);
-    if (__builtin_expect(!(hp == 0.0f || (hp >= 0x1p-124f && hp < 360.0f)), 0)) h = hp / 60.0f;
+    if (!kUnit && __builtin_expect(!(hp == 0.0f || (hp >= 0x1p-124f && hp < 360.0f)), 0))
+        h = hp / 60.0f;
     float hm2 = h - 2.0f * floorf(h * 0.5f);
     float x = c * (1.0f - fabsf(hm2 - 1.0f));
     float m = v - c;
@@ -413,11 +437,9 @@ __device__ __forceinline__ float u8_unit(uint32_t x) {
 
 // fmodf(a, 360.0f).  For 360 <= |a| < 720 the remainder is a -/+ 360,
 // exact by Sterbenz's lemma; a zero remainder keeps the sign of a.
-// kUnit: |a| < 720 is known (see adjust_pixel), so no other case is tested.
-template <bool kUnit = false>
 __device__ __forceinline__ float fmod_360(float a) {
     const float m = __builtin_fabsf(a);
-    if (!kUnit && !(m < 720.0f)) return fmodf(a, 360.0f);  // NaN and infinities too
+    if (!(m < 720.0f)) return fmodf(a, 360.0f);  // NaN and infinities too
     const float r = m >= 360.0f ? m - 360.0f : m;
     return __builtin_copysignf(r, a);
 }
@@ -442,37 +464,68 @@ __device__ __forceinline__ float fmod_360(float a) {
 //     in [-60, 300]; it is never -0 (sep is a difference of distinct values
 //     or +0, and h starts at +0).  With hue_shift in [-180, 180],
 //     h + hue_shift lies in [-240, 480] and is not -0 (a -0 sum needs two
-//     -0 operands), so fmod_360 needs no range test, and rem_euclid gives
+//     -0 operands), so one or two selects make rem_euclid, which gives
 //     a value in [0, 360] that is not -0 (360 when a tiny negative
 //     remainder rounds up);
 // and every channel that reaches to_u8 lies in [0, 1].  The saturation
 // product s * adj.w may be -0 (adj.w = -0) and keeps the general clamp.
 //
-// adjust_tail is everything after brightness/contrast: the HSV hue and
-// saturation step and the conversion back to u8.
-template <bool kUnit>
+// The HSV hue and saturation step, and the conversion back to u8, are
+// adjust_tail for one pixel in general form, and adjust_four for four pixels
+// of one adjustment in the kUnit form: without branches but for one around the
+// step, so that the four pixels' instructions fill each other's waits.
 __device__ __forceinline__ void adjust_tail(float4 adj, float br, float bg, float bb,
                                             uint32_t& ro, uint32_t& go, uint32_t& bo) {
     if (adj.z != 0.0f || adj.w != 1.0f) {
         float h, s, v;
-        rgb_to_hsv<kUnit>(br, bg, bb, h, s, v);
-        float hr = fmod_360<kUnit>(h + adj.z);  // rem_euclid(360.0)
+        rgb_to_hsv(br, bg, bb, h, s, v);
+        float hr = fmod_360(h + adj.z);  // rem_euclid(360.0)
         if (hr < 0.0f) hr = hr + 360.0f;
         float s2 = clampf(s * adj.w, 0.0f, 1.0f);
-        hsv_to_rgb<kUnit>(hr, s2, v, br, bg, bb);
+        hsv_to_rgb(hr, s2, v, br, bg, bb);
     }
-    ro = to_u8<kUnit>(br);
-    go = to_u8<kUnit>(bg);
-    bo = to_u8<kUnit>(bb);
+    ro = to_u8(br);
+    go = to_u8(bg);
+    bo = to_u8(bb);
 }
 
-template <bool kUnit = false>
+// (s * adj.w may be -0 where the general form keeps the sign: c = v s is then
+// -0, x too, m = v - c = v, and every sum with m >= +0 the same as with +0.)
+__device__ __forceinline__ void adjust_four(float4 adj, float (&r)[4], float (&g)[4], float (&b)[4],
+                                            uint32_t (&out)[12]) {
+    if (adj.z != 0.0f || adj.w != 1.0f) {
+        float h[4], s[4], v[4];
+        bool tiny = false;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            rgb_to_hsv<true>(r[i], g[i], b[i], h[i], s[i], v[i]);
+            // rem_euclid(360.0) of a value in [-240, 480] (fmodf's remainder is
+            // a - 360, exact, from 360 on, else a itself)
+            const float a = h[i] + adj.z;
+            h[i] = a >= 360.0f ? a - 360.0f : (a < 0.0f ? a + 360.0f : a);
+            s[i] = clamp_unit(s[i] * adj.w);
+            tiny = tiny || tiny_hue(h[i]);
+        }
+        if (__builtin_expect(tiny, 0)) {
+            for (int i = 0; i < 4; ++i) hsv_to_rgb(h[i], s[i], v[i], r[i], g[i], b[i]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) hsv_to_rgb<true>(h[i], s[i], v[i], r[i], g[i], b[i]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        out[3 * i] = to_u8<true>(r[i]);
+        out[3 * i + 1] = to_u8<true>(g[i]);
+        out[3 * i + 2] = to_u8<true>(b[i]);
+    }
+}
+
 __device__ __forceinline__ void adjust_pixel(float4 adj, uint32_t r8, uint32_t g8, uint32_t b8,
                                              uint32_t& ro, uint32_t& go, uint32_t& bo) {
     float r = u8_unit(r8), g = u8_unit(g8), b = u8_unit(b8);
-    adjust_tail<kUnit>(adj, bright_contrast<kUnit>(r, adj.x, adj.y),
-                       bright_contrast<kUnit>(g, adj.x, adj.y),
-                       bright_contrast<kUnit>(b, adj.x, adj.y), ro, go, bo);
+    adjust_tail(adj, bright_contrast(r, adj.x, adj.y), bright_contrast(g, adj.x, adj.y),
+                bright_contrast(b, adj.x, adj.y), ro, go, bo);
 }
 
 // The contrast stage at contrast 1 for channel value x in 0..255:
