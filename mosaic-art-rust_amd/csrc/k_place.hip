@@ -237,9 +237,9 @@ __global__ __launch_bounds__(64) void place_chain_kernel(PlaceJob single,
 //
 // Measured, one job at a time, against one wave that did all of it (a step of
 // 450 cycles, a full evaluation in 10% of the cells): 1,500 materials in 80 x
-// 60 cells 905 -> 279 us, 10,000 in 160 x 150 4,957 -> 1,908, 500 in 50 x 28
-// 269 -> 91, 1,000 in 20 x 15 58 -> 31, 777 in 97 x 41 with the GUI score
-// 2,283 -> 495.  A step takes 42-48 ns, and the preparation of two cells 1,450
+// 60 cells 905 -> 271 us, 10,000 in 160 x 150 4,957 -> 1,867, 500 in 50 x 28
+// 269 -> 89, 1,000 in 20 x 15 58 -> 30, 777 in 97 x 41 with the GUI score
+// 2,283 -> 482.  A step takes 42-48 ns, and the preparation of two cells 1,350
 // cycles of its wave, about a period; 0.6% (1,500 materials) to 16% (GUI
 // score, whose distances lie closer) of the cells are flagged, at 0.4-1 us.
 // Twelve preparing waves of a cell each: 267 us for the first, and twice the
@@ -389,6 +389,21 @@ __device__ __forceinline__ RawRow load_row(const PlaceJob& job, int32_t cell, in
     return RawRow{gload(rec, lane), gload(rec, lane + 64)};
 }
 
+// The rows of cells c .. c + kPrepCells - 1, from one address (at the grid's end
+// those of its last cells: a cell inside reads its own).
+__device__ __forceinline__ void load_rows(const PlaceJob& job, int32_t c, int32_t cells, int lane,
+                                          RawRow (&q)[kPrepCells]) {
+    if (c + kPrepCells <= cells) {
+        const uint64_t* rec = reinterpret_cast<const uint64_t*>(job.cand) + (int64_t)c * kCandStride;
+#pragma unroll
+        for (int k = 0; k < kPrepCells; ++k)
+            q[k] = RawRow{gload(rec, k * kCandStride + lane), gload(rec, k * kCandStride + lane + 64)};
+    } else {
+#pragma unroll
+        for (int k = 0; k < kPrepCells; ++k) q[k] = load_row(job, c + k, cells, lane);
+    }
+}
+
 // Whether the lists leave out exhausted candidates.  Those of a library of at
 // most 64 materials hold every candidate without that, and stay valid across
 // resets (one every n * limit cells at the least); with a limit of 0 every
@@ -402,8 +417,8 @@ __device__ __forceinline__ bool filters(const PlaceJob& job) {
 struct PrepArgs {
     uint32_t limit;       // candidates whose count word is below it are kept
     bool packed;          // count words hold terms
-    float w2;             // 2 * weight (doubling is exact: t * w2 is 2 t * w)
-    bool penalty;         // weight > 0
+    float w2;             // 2 * weight (doubling is exact: t * w2 is 2 t * w);
+                          // -inf without a penalty: no entry has any reach
 };
 
 // A cell's list has at least this many entries, if its row has them: ranks 64
@@ -446,25 +461,28 @@ __device__ __forceinline__ void prep_cells(const RawRow (&q)[kPrepCells], int32_
         u0[k] = S.counts[m0[k]];
     }
     uint64_t b0[kPrepCells];
-    uint32_t total[kPrepCells], n0[kPrepCells];
-    float tail[kPrepCells];
+    uint32_t total[kPrepCells];
     bool whole = false;  // the lists hold their rows' every kept candidate, or 64
 #pragma unroll
     for (int k = 0; k < kPrepCells; ++k) {
         // (ranks past the row's end read the guard)
         b0[k] = lanes_ult(u0[k], P.limit) & lanes_ne((int32_t)m0[k], (int32_t)(up[k] >> 2));
-        n0[k] = (uint32_t)__popcll(b0[k]);
-        total[k] = n0[k];
-        whole = whole || n0[k] < kEnough;
+        total[k] = (uint32_t)__popcll(b0[k]);
+        whole = whole || total[k] < kEnough;
     }
 #pragma unroll
     for (int k = 0; k < kPrepCells; ++k) {
-        const uint32_t t0 = P.packed ? u0[k] << 16 : 0x3f800000u;
         uint64_t* at = reinterpret_cast<uint64_t*>(stage + k * kStageWords);
-        at[list_place(b0[k], 0u)] = (q[k].r0 & 0xffffffff00000000ull) | (t0 | m0[k]);
-        tail[k] = readlane_f(__uint_as_float((uint32_t)(q[k].r1 >> 32)), 0);
+        at[list_place(b0[k], 0u)] =
+            (q[k].r0 & 0xffffffff00000000ull) | ((P.packed ? u0[k] : 0x3f80u) << 16 | m0[k]);
     }
+    float tail[kPrepCells];  // behind the list: rank 64, or nothing
+#pragma unroll
+    for (int k = 0; k < kPrepCells; ++k)
+        tail[k] = readlane_f(__uint_as_float((uint32_t)(q[k].r1 >> 32)), 0);
+    uint64_t end = 0ull;  // the lanes whose list may end there
     if (whole) {
+        end = ~0ull;
         uint32_t m1[kPrepCells], u1[kPrepCells];
 #pragma unroll
         for (int k = 0; k < kPrepCells; ++k) {
@@ -475,24 +493,23 @@ __device__ __forceinline__ void prep_cells(const RawRow (&q)[kPrepCells], int32_
         for (int k = 0; k < kPrepCells; ++k) {
             const uint64_t b1 =
                 lanes_ult(u1[k], P.limit) & lanes_ne((int32_t)m1[k], (int32_t)(up[k] >> 2));
-            const uint32_t t1 = P.packed ? u1[k] << 16 : 0x3f800000u;
             uint64_t* at = reinterpret_cast<uint64_t*>(stage + k * kStageWords);
-            at[min(list_place(b1, n0[k]), 64u)] =
-                (q[k].r1 & 0xffffffff00000000ull) | (t1 | m1[k]);
-            total[k] = n0[k] + (uint32_t)__popcll(b1);
+            at[min(list_place(b1, total[k]), 64u)] =
+                (q[k].r1 & 0xffffffff00000000ull) | ((P.packed ? u1[k] : 0x3f80u) << 16 | m1[k]);
+            total[k] += (uint32_t)__popcll(b1);
             tail[k] = __builtin_inff();
         }
     }
+    if (c + kPrepCells > cells)
 #pragma unroll
-    for (int k = 0; k < kPrepCells; ++k) total[k] = c + k < cells ? total[k] : 0u;
+        for (int k = 0; k < kPrepCells; ++k) total[k] = c + k < cells ? total[k] : 0u;
     asm volatile("" ::: "memory");  // (a wave's LDS operations are done in order)
-    uint64_t e[kPrepCells];
-    float dn[kPrepCells];
+    uint64_t e[kPrepCells], en[kPrepCells];
 #pragma unroll
     for (int k = 0; k < kPrepCells; ++k) {
         const uint64_t* at = reinterpret_cast<const uint64_t*>(stage + k * kStageWords) + lane;
-        e[k] = *at;
-        dn[k] = reinterpret_cast<const float*>(at)[3];
+        e[k] = at[0];
+        en[k] = at[1];
     }
     // flag the entries that a later one could beat; the last place stands
     // for everything beyond it
@@ -501,16 +518,15 @@ __device__ __forceinline__ void prep_cells(const RawRow (&q)[kPrepCells], int32_
         const uint32_t x = (uint32_t)e[k];
         const uint64_t in = lanes_ult((uint32_t)lane, total[k]);
         const float d = __uint_as_float((uint32_t)(e[k] >> 32));
+        const float dn = __uint_as_float((uint32_t)(en[k] >> 32));
         const float reach = d + __uint_as_float(x & 0xffff0000u) * P.w2;
-        // safe: the next beyond reach, or none next (with no penalty, always)
-        const uint64_t next = in >> 1;
-        uint64_t safe = in & next & __builtin_amdgcn_fcmpf(dn[k], reach, 2);  // >
-        safe |= whole ? in & ~next : 0ull;
-        safe = P.penalty ? safe : in;
+        // safe: the next beyond reach, or none next
+        uint64_t safe = in >> 1 & __builtin_amdgcn_fcmpf(dn, reach, 2);  // >
+        safe |= in & ~(in >> 1) & end;
         safe &= 0x7fffffffffffffffull;
-        const uint32_t common = first[k] ? kFlagged | kFirst : 0u;
+        const uint32_t flags = first[k] ? kFlagged | kFirst : 0u;
         const uint32_t a = lane_in(in) ? (x & 0xffffu) << 2 : 0u;
-        slot[entry_word(k0 + k, lane)] = a | common | (lane_in(safe) ? 0u : kFlagged | kUnsafe);
+        slot[entry_word(k0 + k, lane)] = a | flags | (lane_in(safe) ? 0u : kFlagged | kUnsafe);
         slot[dist_word(k0 + k, lane)] = __float_as_uint(lane_in(in) ? d : tail[k]);
     }
 }
@@ -522,8 +538,7 @@ __device__ __forceinline__ void prep_waves(const PlaceJob& job, const ChainShare
     PrepArgs P;
     P.packed = packs(job);
     P.limit = filters(job) ? (uint32_t)job.max_usage << (P.packed ? 16 : 0) : kGuard;
-    P.penalty = job.weight > 0.0f;
-    P.w2 = 2.0f * job.weight;
+    P.w2 = job.weight > 0.0f ? 2.0f * job.weight : -__builtin_inff();
     uint32_t* const stage = S.stage + v * kPrepCells * kStageWords;
     const uint32_t cap = cycle_cap(cells);
     uint32_t cycle = 0;
@@ -533,10 +548,7 @@ __device__ __forceinline__ void prep_waves(const PlaceJob& job, const ChainShare
         RawRow q[kSlots][kPrepCells];
         int32_t c = start + v * kPrepCells;  // this wave's first cell of the group
 #pragma unroll
-        for (int s = 0; s < kSlots; ++s)
-#pragma unroll
-            for (int k = 0; k < kPrepCells; ++k)
-                q[s][k] = load_row(job, c + s * kGroup + k, cells, lane);
+        for (int s = 0; s < kSlots; ++s) load_rows(job, c + s * kGroup, cells, lane, q[s]);
         // Everything landed (vmcnt 0): with nothing pending on the way in, the
         // compiler's wait counts inside the loop are those of its own loads,
         // and the rows in flight are not waited for.
@@ -557,13 +569,11 @@ __device__ __forceinline__ void prep_waves(const PlaceJob& job, const ChainShare
                     up[k] = 0u;
                     if (kUp == kUpPrep)
                         up[k] = S.ring[rp + k < S.ring_n ? rp + k : rp + k - S.ring_n];
-                    first[k] = x + k == 0 || x + k == gw;
+                    first[k] = x + k == (k == 0 ? 0 : gw);  // (x < gw)
                 }
                 prep_cells(q[s], c, cells, up, first, P, S, S.rows + s * kSlotWords, v * kPrepCells,
                            stage, lane);
-#pragma unroll
-                for (int k = 0; k < kPrepCells; ++k)
-                    q[s][k] = load_row(job, c + kSlots * kGroup + k, cells, lane);
+                load_rows(job, c + kSlots * kGroup, cells, lane, q[s]);
                 c += kGroup;
                 x = kUp == kUpPrep ? (x + kGroup < gw ? x + kGroup : x + kGroup - gw)
                                    : (x + kGroup) % gw;
@@ -898,6 +908,7 @@ __device__ __forceinline__ void leave_cycle(const ChainShared& S, uint32_t event
 // follows a vector compare or lane read waits about 16 more, a branch takes
 // 12 and an LDS instruction among vector ones 8 (measured); the order below
 // is the best of some 300 measured, 88 cycles a step (128 for the plain one).
+// The steps begin on a 256-byte boundary: 1-2% for their instruction fetch.
 //
 // Flags of an entry: kFlagged any of the others; kFirst the row's first
 // cell, which has no left neighbour -- the step is right for it all the same
@@ -991,6 +1002,7 @@ __device__ __forceinline__ void leave_cycle(const ChainShared& S, uint32_t event
         MH_ENTER(3, 4, 5)                                                                       \
         "L_in0_%=:\n"                                                                           \
         MH_ENTER(0, 1, 2)                                                                       \
+        ".p2align 8\n"                                                                          \
         MH_STEP(0, 0, 1, 2, v65, v66, 1, 0, 0, "", BAN, KEEP, UP)                               \
         MH_STEP(1, 1, 2, 0, v66, v68, 0, 1, 1, MH_READ("v[64:67]", rc, 2), BAN, KEEP, UP)       \
         MH_STEP(2, 2, 0, 1, v68, v69, 1, 0, 0, "", BAN, KEEP, UP)                               \
