@@ -209,7 +209,7 @@ __device__ __forceinline__ float sum_lanes(float s, float t) {
 // run: mostly the binades of the first few hundred terms.)  24,000 cells:
 // 50 us, 450 us one by one.  lds: kCostWords words, 16-byte aligned.
 // The result is returned to every wave.
-constexpr int32_t kCostWaves = 8, kCostWords = 256 + 2 * kCostWaves + 4;
+constexpr int32_t kCostWaves = 12, kCostWords = 256 + 2 * kCostWaves + 4;
 constexpr int32_t kAnnealThreads = 64 * kCostWaves;
 
 template <typename G, typename TS>
@@ -279,7 +279,7 @@ __device__ float total_cost_block(const G* grid, int32_t gw, int32_t gh, const T
                     done = k + 1;
                 }
             }
-            buffer ^= kCostWaves;
+            buffer = kCostWaves - buffer;
             s = U.value(m);
             if (done == kCostWaves) break;
             if (w == done) {
@@ -299,13 +299,12 @@ __device__ float total_cost_block(const G* grid, int32_t gw, int32_t gh, const T
 
 // ---------------------------------------------------------- annealing
 // What bounds it is the latency of a round, and how many proposals a round
-// commits.  A round runs on eight waves of one workgroup in two phases, with a
+// commits.  A round runs on twelve waves of one workgroup in two phases, with a
 // barrier after each (s: the first proposal of the round; lane l of the slot
 // waves and the judge: proposal s + l):
-//   * terms: slot wave w makes the adjacency terms of two of the eight
-//     neighbour cells (w = 0, 1: Up and Down, Left and Right of the first
-//     cell; 2, 3: of the second) with the swap's two materials.  The judge
-//     takes in the proposals, and swaps those it expects to be accepted.
+//   * terms: slot wave w makes the adjacency terms of one of the eight
+//     neighbour cells with the swap's two materials.  The judge takes in the
+//     proposals, and swaps those it expects to be accepted.
 //   * decisions: the judge adds a swap's terms in the reference's order and
 //     decides it.  The slot waves read the next round's cells and Labs, from
 //     the grid as it is expected to be.
@@ -331,11 +330,12 @@ __device__ float total_cost_block(const G* grid, int32_t gw, int32_t gh, const T
 //
 // Measured against one wave that gathered its terms from a matrix of all pairs
 // and added the initial cost one term after another: 1,000 proposals on 20 x
-// 15 cells 332 -> 127 us (200 rounds -> 97), 2,000 on 80 x 60 340 -> 92 (100 ->
-// 54), 2,000 on 206 x 116 600 -> 132, 20,000 on 200 x 120 1,650 -> 568.  A
-// round takes 1.15 us for 3.3 (1.5 with the reads as a phase of their own):
-// 1,600 cycles of terms, 1,000 of decisions.
-constexpr int kSlotWaves = 4, kJudgeWave = 4, kDraw1Wave = 5, kDraw2Wave = 6, kCostWave = 7;
+// 15 cells 332 -> 112 us (200 rounds -> 97), 2,000 on 80 x 60 340 -> 84 (100 ->
+// 54), 2,000 on 206 x 116 600 -> 120, 20,000 on 200 x 120 1,650 -> 488.  A
+// round takes 1.0 us for 3.3 (1.5 with the reads as a phase of their own, 1.15
+// with two neighbours to each of four slot waves): 1,450 cycles of terms (the
+// judge's taking in), 1,150 of decisions.
+constexpr int kSlotWaves = 8, kJudgeWave = 8, kDraw1Wave = 9, kDraw2Wave = 10, kCostWave = 11;
 static_assert(kAnnealThreads == 64 * (kCostWave + 1), "one wave a role");
 
 // Stamps, tag << 7 | (63 - lane) << 1 | cell (0: the first of the swap): one
@@ -355,11 +355,11 @@ constexpr uint32_t kTagEnd = (1u << 25) - 2u;  // (a round takes at most two)
 constexpr int32_t kRing = 256;
 
 // LDS in words, behind the stamps: Labs of the swaps' materials (64 of the
-// first, 64 of the second), the terms (4 waves x 64 x {m1 with a, m2 with a,
-// m1 with b, m2 with b} for the wave's neighbours a, b), the lanes that a and b
-// were taken from, the mutual terms, a round's accepted deltas, the ring,
-// control words, the grid, the library's Labs (where they fit).
-constexpr int32_t kLabWords = 2 * 64 * 4, kTermWords = kSlotWaves * 64 * 4,
+// first, 64 of the second), the terms (4 pairs of waves x 64 x {m1 with a, m2
+// with a, m1 with b, m2 with b} for the pair's neighbours a, b), the lanes that
+// the neighbours were taken from, the mutual terms, a round's accepted deltas,
+// the ring, control words, the grid, the library's Labs (where they fit).
+constexpr int32_t kLabWords = 2 * 64 * 4, kTermWords = kSlotWaves * 64 * 2,
                   kFromWords = kSlotWaves * 64, kMutualWords = 64, kPackWords = 64, kCtrlWords = 8;
 constexpr int32_t kFixedWords =
     kLabWords + kTermWords + kFromWords + kMutualWords + kPackWords + 3 * kRing + kCtrlWords;
@@ -380,8 +380,8 @@ template <typename G>
 struct AnnealShared {
     uint32_t* stamp;
     float4* lab_m;     // [2][64]
-    float4* terms;     // [kSlotWaves][64]
-    uint32_t* from;    // [kSlotWaves][64]: a's lane | b's << 8, kNoLane: none
+    float4* terms;     // [kSlotWaves / 2][64]
+    uint32_t* from;    // [kSlotWaves][64], kNoLane: none
     float* mutual;     // [64]
     float* pack;       // [64]
     uint32_t *ring_xy1, *ring_xy2;
@@ -445,30 +445,11 @@ struct Nothing {
     __device__ __forceinline__ void operator()() const {}
 };
 
-// The Labs of two neighbours and (waves 0 and 1) of one of the swap's
-// materials, requested together.
-template <typename G>
-__device__ __forceinline__ void load_labs(const AnnealJob& job, const AnnealShared<G>& S, int32_t a,
-                                          int32_t b, int32_t m, bool want_m, float4& la, float4& lb,
-                                          float4& lm) {
-    a = max(a, 0);
-    b = max(b, 0);
-    m = max(m, 0);
-    if (S.labs) {
-        la = S.labs[a];
-        lb = S.labs[b];
-        if (want_m) lm = S.labs[m];
-    } else {
-        la = gload4(job.lab4, a);
-        lb = gload4(job.lab4, b);
-        if (want_m) lm = gload4(job.lab4, m);
-    }
-}
-
-// Where a slot wave's swap and its two neighbours are.
+// Where a slot wave's swap and its neighbour are (wave w & 3: Up, Down, Left,
+// Right; w >> 2: of the swap's first, second cell).
 struct Place {
-    int32_t p1, p2, qa, qb;
-    bool in_a, in_b, self_a, self_b;  // inside the grid; the swap's other cell
+    int32_t p1, p2, q;
+    bool in, self;  // inside the grid; the swap's other cell
     bool active;
 };
 
@@ -476,53 +457,58 @@ template <typename G>
 __device__ __forceinline__ Place place_of(const AnnealJob& job, const AnnealShared<G>& S, int w,
                                           int64_t it) {
     const int32_t gw = job.grid_w;
-    const bool vertical = !(w & 1), second = w >= 2;
-    const int32_t step = vertical ? gw : 1, bound = vertical ? job.grid_h : gw;
+    const bool vertical = !(w & 2), second = w >= 4, onward = w & 1;
+    const int32_t step = vertical ? gw : 1, last = (vertical ? job.grid_h : gw) - 1;
     const uint32_t slot = (uint32_t)it & (kRing - 1);
     const uint32_t xy1 = S.ring_xy1[slot], xy2 = S.ring_xy2[slot];
-    const int32_t x1 = (int32_t)(xy1 & 0xffffu), y1 = (int32_t)(xy1 >> 16);
-    const int32_t x2 = (int32_t)(xy2 & 0xffffu), y2 = (int32_t)(xy2 >> 16);
     Place p;
-    p.p1 = y1 * gw + x1;
-    p.p2 = y2 * gw + x2;
+    p.p1 = (int32_t)(xy1 >> 16) * gw + (int32_t)(xy1 & 0xffffu);
+    p.p2 = (int32_t)(xy2 >> 16) * gw + (int32_t)(xy2 & 0xffffu);
     const int32_t centre = second ? p.p2 : p.p1, partner = second ? p.p1 : p.p2;
-    const int32_t along = vertical ? (second ? y2 : y1) : (second ? x2 : x1);
-    p.in_a = along > 0;
-    p.in_b = along < bound - 1;
+    const uint32_t xy = second ? xy2 : xy1;
+    const int32_t along = (int32_t)(vertical ? xy >> 16 : xy & 0xffffu);
+    p.in = along != (onward ? last : 0);
     // a neighbour outside the grid reads its own cell, always in bounds
-    p.qa = p.in_a ? centre - step : centre;
-    p.qb = p.in_b ? centre + step : centre;
-    p.self_a = p.in_a && p.qa == partner;
-    p.self_b = p.in_b && p.qb == partner;
+    p.q = p.in ? centre + (onward ? step : -step) : centre;
+    p.self = p.q == partner;  // (an outside one only where the proposal is skipped)
     p.active = it < job.max_iter && p.p1 != p.p2;
     return p;
 }
 
-// What a slot wave's reads bring: the neighbours' Labs, which of them count,
-// and whether the proposal does.
+// What a slot wave's reads bring: the neighbour's Lab, whether it counts, and
+// whether the proposal does.
 struct Reads {
-    float4 la, lb;
-    bool ok_a, ok_b, skip;
+    float4 lab;
+    bool ok, skip;
 };
 
 template <typename G>
 __device__ __forceinline__ Reads read_swap(const AnnealJob& job, const AnnealShared<G>& S, G* grid,
                                            int w, int lane, const Place& p, const Rounds& R) {
-    const int32_t m1 = gget(grid, p.p1), m2 = gget(grid, p.p2);
-    const int32_t a = gget(grid, p.qa), b = gget(grid, p.qb);
+    const int32_t m1 = gget(grid, p.p1), m2 = gget(grid, p.p2), a = gget(grid, p.q);
     Reads r;
     r.skip = !p.active || m1 == kEmpty || m2 == kEmpty;
-    r.ok_a = p.in_a && !p.self_a && a != kEmpty;
-    r.ok_b = p.in_b && !p.self_b && b != kEmpty;
+    r.ok = p.in && !p.self && a != kEmpty;
+    // waves 0 and 4 read the swap's materials' Labs too
+    const bool own = (w & 3) == 0;
     float4 lm = make_float4(0, 0, 0, 0);
-    r.la = r.lb = lm;
-    if (job.n > 0) load_labs(job, S, a, b, w == 0 ? m1 : m2, w < 2, r.la, r.lb, lm);
+    r.lab = lm;
+    if (job.n > 0) {
+        const int32_t i = max(a, 0), k = max(w == 0 ? m1 : m2, 0);
+        if (S.labs) {
+            r.lab = S.labs[i];
+            if (own) lm = S.labs[k];
+        } else {
+            r.lab = gload4(job.lab4, i);
+            if (own) lm = gload4(job.lab4, k);
+        }
+    }
     if (w == 2 && R.hopeful && !r.skip) {
         const uint32_t mine = (R.tag << 7) | ((uint32_t)(63 - lane) << 1);
         atomicMax(&S.stamp[S.at(p.p1)], mine);
         atomicMax(&S.stamp[S.at(p.p2)], mine | 1u);
     }
-    if (w < 2) S.lab_m[w * 64 + lane] = lm;
+    if (own) S.lab_m[w * 16 + lane] = lm;
     return r;
 }
 
@@ -550,15 +536,14 @@ __device__ __forceinline__ void slot_wave(const AnnealJob& job, const AnnealShar
         // ---- terms
         const uint32_t outcome = S.ctrl[kCtrlRound];
         float4 l1, l2;
-        uint32_t va, vb, v1, v2;
+        uint32_t va, v1, v2;
         // (with the outcome in flight: it is nearly always the expected one)
         auto load = [&]() __attribute__((always_inline)) {
-            va = S.stamp[S.at(p.qa)];
-            vb = S.stamp[S.at(p.qb)];
-            v1 = S.stamp[S.at(p.p1)];
-            v2 = S.stamp[S.at(p.p2)];
+            va = S.stamp[S.at(p.q)];
             l1 = S.lab_m[lane];
             l2 = S.lab_m[64 + lane];
+            v1 = S.stamp[S.at(p.p1)];
+            v2 = S.stamp[S.at(p.p2)];
         };
         load();
         R.next(outcome);
@@ -570,50 +555,40 @@ __device__ __forceinline__ void slot_wave(const AnnealJob& job, const AnnealShar
                 r = read_swap(job, S, grid, w, lane, p, R);
             },
             load);
-        float4 la = r.la, lb = r.lb;
-        const Place q = p;
-        uint32_t from = kNoLane | kNoLane << 8;
+        const uint32_t mine = (R.tag << 7) | ((uint32_t)(63 - lane) << 1);
+        float4 la = r.lab;
         if (R.hopeful) {
-            const uint32_t mine = (R.tag << 7) | ((uint32_t)(63 - lane) << 1);
-            // the next round's proposals, if all goes as expected
-            const int32_t first = expected_prefix(v1, v2, mine, r.skip, max_iter - R.s);
-            p = place_of(job, S, w, R.s + first + lane);
             // stamped in this round by a lower lane: above this lane's stamps
-            bool sub_a = va > (mine | 1u), sub_b = vb > (mine | 1u);
-            if (wave_ballot(sub_a || sub_b)) {
-                const uint32_t ka = 63u - ((va >> 1) & 63u), kb = 63u - ((vb >> 1) & 63u);
-                uint32_t ca = va & 1u, cb = vb & 1u;  // which of k's cells
+            bool sub = va > (mine | 1u);
+            uint32_t from = kNoLane;
+            if (wave_ballot(sub)) {
+                const uint32_t k = 63u - ((va >> 1) & 63u);
+                bool first_cell = !(va & 1u);  // which of k's cells
                 if (S.hashed) {
-                    auto which = [&](uint32_t k, int32_t cell, bool& sub) {
-                        const uint32_t ks = (uint32_t)(R.s + k) & (kRing - 1);
-                        const uint32_t k1 = S.ring_xy1[ks], k2 = S.ring_xy2[ks];
-                        const bool is1 =
-                            (int32_t)(k1 >> 16) * job.grid_w + (int32_t)(k1 & 0xffffu) == cell;
-                        const bool is2 =
-                            (int32_t)(k2 >> 16) * job.grid_w + (int32_t)(k2 & 0xffffu) == cell;
-                        sub = sub && (is1 || is2);
-                        return is1 ? 0u : 1u;
-                    };
-                    ca = which(ka, q.qa, sub_a);
-                    cb = which(kb, q.qb, sub_b);
+                    const uint32_t ks = (uint32_t)(R.s + k) & (kRing - 1);
+                    const uint32_t k1 = S.ring_xy1[ks], k2 = S.ring_xy2[ks];
+                    first_cell = (int32_t)(k1 >> 16) * job.grid_w + (int32_t)(k1 & 0xffffu) == p.q;
+                    sub = sub && (first_cell || (int32_t)(k2 >> 16) * job.grid_w +
+                                                        (int32_t)(k2 & 0xffffu) == p.q);
                 }
                 // k's first cell gets its second material, and the reverse
-                const float4 na = S.lab_m[(ca ? 0u : 64u) + ka], nb = S.lab_m[(cb ? 0u : 64u) + kb];
-                la = make_float4(sub_a ? na.x : la.x, sub_a ? na.y : la.y, sub_a ? na.z : la.z, 0.0f);
-                lb = make_float4(sub_b ? nb.x : lb.x, sub_b ? nb.y : lb.y, sub_b ? nb.z : lb.z, 0.0f);
-                from = (sub_a ? ka : kNoLane) | (sub_b ? kb : kNoLane) << 8;
+                const float4 other = S.lab_m[(first_cell ? 64u : 0u) + k];
+                la = make_float4(sub ? other.x : la.x, sub ? other.y : la.y, sub ? other.z : la.z, 0.0f);
+                from = sub ? k : kNoLane;
             }
             S.from[w * 64 + lane] = from;
         }
-        const float t1a = adj_term(l1, la), t2a = adj_term(l2, la);
-        const float t1b = adj_term(l1, lb), t2b = adj_term(l2, lb);
-        S.terms[w * 64 + lane] = make_float4(r.ok_a ? t1a : 0.0f, r.ok_a ? t2a : 0.0f,
-                                             r.ok_b ? t1b : 0.0f, r.ok_b ? t2b : 0.0f);
+        const float t1 = adj_term(l1, la), t2 = adj_term(l2, la);
+        reinterpret_cast<float2*>(S.terms)[((w >> 1) * 64 + lane) * 2 + (w & 1)] =
+            make_float2(r.ok ? t1 : 0.0f, r.ok ? t2 : 0.0f);
         // the partner as a neighbour of the first cell: the mutual term
-        if (w < 2 && (q.self_a || q.self_b)) S.mutual[lane] = q.self_a ? t1a : t1b;
+        if (w < 4 && p.self) S.mutual[lane] = t1;
         phase_end();
         // ---- decisions
         if (R.hopeful) {
+            // the next round's proposals, if all goes as expected
+            const int32_t first = expected_prefix(v1, v2, mine, r.skip, max_iter - R.s);
+            p = place_of(job, S, w, R.s + first + lane);
             ++R.tag;
             r = read_swap(job, S, grid, w, lane, p, R);
         }
@@ -631,9 +606,9 @@ __device__ __forceinline__ void judge_wave(const AnnealJob& job, const AnnealSha
     const int32_t gw = job.grid_w, gh = job.grid_h;
     const int64_t max_iter = job.max_iter;
     int64_t kbase = 0, accepted = 0, evaluated = 0, rounds = 0;
-    // the last round's, for the cost wave and the traces
+    // the last round's, for the traces
+    const bool traced = job.trace_delta || job.trace_accept;
     float delta = 0.0f;
-    uint64_t accmask = 0;
     int64_t it = lane;
     bool acc = false, skip = true;
     int32_t first = 0;
@@ -669,11 +644,7 @@ __device__ __forceinline__ void judge_wave(const AnnealJob& job, const AnnealSha
         };
         load();
         R.next(outcome);
-        // the accepted deltas in proposal order, +0.0 past the last
-        S.pack[lane] = 0.0f;
-        asm volatile("" ::: "memory");
-        if (lane_in(accmask)) S.pack[lanes_before(accmask)] = delta;
-        if (lane < first) {
+        if (traced && lane < first) {  // (the last round's)
             if (job.trace_delta) gstore(job.trace_delta, it, skip ? __int_as_float(0x7fc00000) : delta);
             if (job.trace_accept) gstore(job.trace_accept, it, (uint8_t)(acc ? 1 : 0));
         }
@@ -692,11 +663,11 @@ __device__ __forceinline__ void judge_wave(const AnnealJob& job, const AnnealSha
         first = remain < 64 ? (int32_t)remain : 64;
         if (R.hopeful) {
             first = expected_prefix(v1, v2, mine, skip, remain);
-            take(R.s + first);
             if (!skip && lane < first) {  // (all of these cells are different)
                 gput(grid, p1, m2);
                 gput(grid, p2, m1);
             }
+            take(R.s + first);
             if constexpr (kHbm) __threadfence();
         }
         const bool adjacent =
@@ -757,9 +728,8 @@ __device__ __forceinline__ void judge_wave(const AnnealJob& job, const AnnealSha
                 // took a value that a rejected lane would have moved
 #pragma unroll
                 for (int i = 0; i < kSlotWaves; ++i) {
-                    const uint32_t f = S.from[64 * i + lane], ka = f & 255u, kb = f >> 8;
-                    conflict |= ka != kNoLane && ((rejected >> (ka & 63u)) & 1ull) != 0ull;
-                    conflict |= kb != kNoLane && ((rejected >> (kb & 63u)) & 1ull) != 0ull;
+                    const uint32_t k = S.from[64 * i + lane];
+                    conflict |= k != kNoLane && ((rejected >> (k & 63u)) & 1ull) != 0ull;
                 }
             } else {
                 if (acc) {
@@ -788,7 +758,9 @@ __device__ __forceinline__ void judge_wave(const AnnealJob& job, const AnnealSha
             }
             if constexpr (kHbm) __threadfence();
         }
-        accmask = acc_all & commit;
+        const uint64_t accmask = acc_all & commit;
+        // the accepted deltas for the cost wave (adding +0.0 changes no sum)
+        S.pack[lane] = lane_in(accmask) ? delta : 0.0f;
         const int32_t n_acc = __popcll(accmask), n_ev = __popcll(nonskip & commit);
         if (lane == 0)
             S.ctrl[kCtrlRound] =
@@ -834,13 +806,16 @@ __device__ __forceinline__ void draw_wave(const AnnealJob& job, const AnnealShar
     }
 }
 
-// The running cost: the accepted deltas of a round, packed in proposal order,
-// added in the next round (+0.0 past the last changes nothing).
+// The running cost: a round's deltas in proposal order, +0.0 for those not
+// accepted.
 struct CostSum {
     float cost, best;
     int64_t improved = 0;
-    __device__ __forceinline__ void add(const float* pack, int32_t n_acc, bool greedy, int lane) {
-        const float c = add_lanes(cost, pack[lane], lane);
+    float c;  // each lane's sum in the round being added
+    __device__ __forceinline__ void add(const float* pack, int lane) {
+        c = add_lanes(cost, pack[lane], lane);
+    }
+    __device__ __forceinline__ void count(int32_t n_acc, bool greedy) {
         if (greedy) {  // optimize_greedy counts every accepted swap
             improved += n_acc;
         } else if (wave_ballot(c < best)) {
@@ -868,8 +843,9 @@ __device__ __forceinline__ void cost_wave(const AnnealJob& job, const AnnealShar
         R.next(S.ctrl[kCtrlRound]);
         if (R.s >= job.max_iter) break;
         R.begin(S, words, kCostWave * 64 + lane, Nothing{}, Nothing{});
+        if (R.pending) C.add(S.pack, lane);
         phase_end();
-        if (R.pending) C.add(S.pack, R.pending, job.greedy != 0, lane);
+        if (R.pending) C.count(R.pending, job.greedy != 0);
         if (filled <= R.s + kRing - 64) {
             const uint64_t j = (uint64_t)(filled + lane);
             S.ring_u[j & (kRing - 1)] = draw_unit(job.seed, j);
@@ -878,8 +854,10 @@ __device__ __forceinline__ void cost_wave(const AnnealJob& job, const AnnealShar
         if (R.hopeful) ++R.tag;
         phase_end();
     }
-    phase_end();  // the last round's deltas are there
-    if (R.pending) C.add(S.pack, R.pending, job.greedy != 0, lane);
+    if (R.pending) {
+        C.add(S.pack, lane);
+        C.count(R.pending, job.greedy != 0);
+    }
     if (lane == 0) {
         S.ctrl[kCtrlCost] = __float_as_uint(C.cost);
         S.ctrl[kCtrlBest] = __float_as_uint(C.best);
@@ -903,7 +881,7 @@ __global__ __launch_bounds__(kAnnealThreads) void anneal_kernel(AnnealJob single
     S.stamp = sm;
     S.lab_m = reinterpret_cast<float4*>(sm + words);
     S.terms = S.lab_m + 2 * 64;
-    S.from = reinterpret_cast<uint32_t*>(S.terms + kSlotWaves * 64);
+    S.from = reinterpret_cast<uint32_t*>(S.terms + kSlotWaves / 2 * 64);
     S.mutual = reinterpret_cast<float*>(S.from + kFromWords);
     S.pack = S.mutual + kMutualWords;
     S.ring_xy1 = reinterpret_cast<uint32_t*>(S.pack + kPackWords);
@@ -970,7 +948,6 @@ __global__ __launch_bounds__(kAnnealThreads) void anneal_kernel(AnnealJob single
         draw_wave(job, S, w, lane, words);
     else
         cost_wave(job, S, lane, words);
-    if (w != kCostWave) phase_end();
     __syncthreads();
     if constexpr (!kHbm)
         for (int32_t i = tid; i < cells; i += kAnnealThreads) gstore(job.grid, i, (int32_t)grid[i]);
