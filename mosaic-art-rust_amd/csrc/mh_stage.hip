@@ -30,11 +30,9 @@ size_t chunk_of(size_t total) {
     return std::min(kBuffer, std::max(kLeast / 2, share));
 }
 
-int stage_ready(mh_context* ctx, StageBuf& b) {
-    if (b.p) return MH_OK;
-    HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&b.p), kBuffer, hipHostMallocDefault));
-    HIPCHK(hipEventCreateWithFlags(&b.copied, hipEventDisableTiming));
-    (void)ctx;
+int stage_ready(StageBuf& b) {
+    if (!b.copied) HIPCHK(hipEventCreateWithFlags(&b.copied, hipEventDisableTiming));
+    if (!b.p) HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&b.p), kBuffer, hipHostMallocDefault));
     return MH_OK;
 }
 
@@ -85,12 +83,12 @@ int stage_upload(mh_context* ctx, uint8_t* dst, const std::vector<HostSpan>& spa
     const size_t total = at.back(), chunk = chunk_of(total), chunks = (total + chunk - 1) / chunk;
     std::lock_guard<std::mutex> g(ctx->stage_mu);
     std::atomic<size_t> next{0};
-    return on_threads(ctx, chunks, [&](int t) -> int {
+    const int rc = on_threads(ctx, chunks, [&](int t) -> int {
         for (int k = 0;; k ^= 1) {
             const size_t c = next.fetch_add(1);
             if (c >= chunks) return MH_OK;
             StageBuf& b = ctx->stage[2 * t + k];
-            CHK(stage_ready(ctx, b));
+            CHK(stage_ready(b));
             HIPCHK(hipEventSynchronize(b.copied));  // (its last copy; none: returns at once)
             const size_t lo = c * chunk, hi = std::min(total, lo + chunk);
             size_t i = (size_t)(std::upper_bound(at.begin(), at.end(), lo) - at.begin()) - 1;
@@ -103,13 +101,22 @@ int stage_upload(mh_context* ctx, uint8_t* dst, const std::vector<HostSpan>& spa
             HIPCHK(hipEventRecord(b.copied, ctx->stream));
         }
     });
+    if (!rc) return MH_OK;
+    // no pinned memory to be had, perhaps: all of it by the runtime
+    (void)hipGetLastError();
+    for (size_t i = 0; i < spans.size(); ++i)
+        if (spans[i].bytes)
+            HIPCHK(hipMemcpyAsync(dst + at[i], spans[i].p, spans[i].bytes, hipMemcpyHostToDevice,
+                                  ctx->stream));
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    return MH_OK;
 }
 
 int stage_download(mh_context* ctx, uint8_t* host, const uint8_t* src, size_t total) {
     const size_t chunk = chunk_of(total), chunks = (total + chunk - 1) / chunk;
     std::lock_guard<std::mutex> g(ctx->stage_mu);
     std::atomic<size_t> next{0};
-    return on_threads(ctx, chunks, [&](int t) -> int {
+    const int rc = on_threads(ctx, chunks, [&](int t) -> int {
         size_t mine[2];
         bool busy[2] = {false, false};
         for (int k = 0;; k ^= 1) {
@@ -125,7 +132,7 @@ int stage_download(mh_context* ctx, uint8_t* host, const uint8_t* src, size_t to
                 if (!busy[k ^ 1]) return MH_OK;
                 continue;
             }
-            CHK(stage_ready(ctx, b));
+            CHK(stage_ready(b));
             HIPCHK(hipEventSynchronize(b.copied));
             const size_t lo = c * chunk;
             HIPCHK(hipMemcpyAsync(b.p, src + lo, std::min(total, lo + chunk) - lo,
@@ -135,6 +142,11 @@ int stage_download(mh_context* ctx, uint8_t* host, const uint8_t* src, size_t to
             busy[k] = true;
         }
     });
+    if (!rc) return MH_OK;
+    (void)hipGetLastError();
+    HIPCHK(hipMemcpyAsync(host, src, total, hipMemcpyDeviceToHost, ctx->stream));
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    return MH_OK;
 }
 
 void stage_release(mh_context* ctx) {
