@@ -198,7 +198,7 @@ def run_batched(mh, synth, ctx, steps, warmup):
             if lat is not None:
                 lat.append(1000.0 * (time.perf_counter() - t0))
 
-    plain_pass()  # warm: library caches (resized tiles, term matrices)
+    plain_pass()  # warm: library caches (resized tiles, terms)
     plain_lat = []
     t0 = time.perf_counter()
     plain_pass(plain_lat)
@@ -252,7 +252,7 @@ def run_batched(mh, synth, ctx, steps, warmup):
 def stream_setup(mh, synth, ctx, n_jobs, rate):
     """The Poisson stream's libraries and canvases made resident, each job's
     target a contiguous device crop of its canvas, and the libraries'
-    caches (resized tiles, term matrices) warmed by one plain job each."""
+    caches (resized tiles, terms) warmed by one plain job each."""
     st = synth.make_stream(n_jobs, rate)
     jobs = st["jobs"]
     W = st["canvas_size"][0]
