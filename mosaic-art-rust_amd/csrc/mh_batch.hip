@@ -1023,8 +1023,8 @@ namespace {
 // so the last batches hold the shortest chains, unless the oldest job has
 // already been passed over kWindowBatches times.  The rest of the batch are
 // the window's jobs nearest to the anchor in cell count (by ratio), in queue
-// order.  A placement launch lasts as long as its longest chain (one wave
-// walks a job's cells in order), so batches of like-sized jobs keep each
+// order.  A placement launch lasts as long as its longest chain (its
+// cells are decided in order), so batches of like-sized jobs keep each
 // chain stream from waiting on one long job per batch.  Which jobs share a
 // batch changes no job's result.  With at most max_batch jobs queued this is
 // first-come first-served.
