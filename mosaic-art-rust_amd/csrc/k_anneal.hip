@@ -299,7 +299,8 @@ __device__ float total_cost_block(const G* grid, int32_t gw, int32_t gh, const T
 
 // ---------------------------------------------------------- annealing
 // What bounds it is the latency of a round, and how many proposals a round
-// commits.  A round runs on twelve waves of one workgroup in two phases, with a
+// commits.  Small grids begin in whole blocks (follow_blocks, below), which commit
+// more; what follows is the general form.  A round runs on twelve waves of one workgroup in two phases, with a
 // barrier after each (s: the first proposal of the round; lane l of the slot
 // waves and the judge: proposal s + l):
 //   * terms: slot wave w makes the adjacency terms of one of the eight
@@ -330,11 +331,12 @@ __device__ float total_cost_block(const G* grid, int32_t gw, int32_t gh, const T
 //
 // Measured against one wave that gathered its terms from a matrix of all pairs
 // and added the initial cost one term after another: 1,000 proposals on 20 x
-// 15 cells 332 -> 112 us (200 rounds -> 97), 2,000 on 80 x 60 340 -> 84 (100 ->
-// 54), 2,000 on 206 x 116 600 -> 120, 20,000 on 200 x 120 1,650 -> 488.  A
-// round takes 1.0 us for 3.3 (1.5 with the reads as a phase of their own, 1.15
-// with two neighbours to each of four slot waves): 1,450 cycles of terms (the
-// judge's taking in), 1,150 of decisions.
+// 15 cells 332 -> 112 us (200 rounds -> 97; in 17 blocks 44 us), 2,000 on 80 x 60
+// 340 -> 84 (100 -> 54; 32 blocks 81), 2,000 on 206 x 116 600 -> 120, 20,000 on
+// 200 x 120 1,650 -> 488.  A round takes 1.0 us for 3.3 (1.5 with the reads as a
+// phase of their own, 1.15 with two neighbours to each of four slot waves):
+// 1,450 cycles of terms (the judge's taking in), 1,150 of decisions.
+constexpr int kMarkWave = 9;  // in whole blocks; wave 10 draws
 constexpr int kSlotWaves = 8, kJudgeWave = 8, kDraw1Wave = 9, kDraw2Wave = 10, kCostWave = 11;
 static_assert(kAnnealThreads == 64 * (kCostWave + 1), "one wave a role");
 
@@ -345,8 +347,12 @@ static_assert(kAnnealThreads == 64 * (kCostWave + 1), "one wave a role");
 // comparing the cells (substituted neighbours).  The words double as the
 // initial cost's.
 constexpr int32_t kHashStamps = 16384;
-__host__ __device__ __forceinline__ int32_t stamp_words(int32_t cells) {
-    return cells > kHashStamps ? kHashStamps : (cells < kCostWords ? kCostWords : (cells + 3) & ~3);
+// A run that begins in whole blocks (follow_blocks) has two tables of 8 bytes a
+// cell in the same place.
+__host__ __device__ __forceinline__ int32_t stamp_words(int32_t cells, bool blocks) {
+    if (cells > kHashStamps) return kHashStamps;
+    const int32_t w = blocks ? 4 * cells : (cells + 3) & ~3;
+    return w < kCostWords ? kCostWords : w;
 }
 constexpr uint32_t kTagEnd = (1u << 25) - 2u;  // (a round takes at most two)
 // Proposal draws, made ahead into a ring of three words a slot: x1 | y1 << 16,
@@ -360,7 +366,7 @@ constexpr int32_t kRing = 256;
 // the neighbours were taken from, the mutual terms, a round's accepted deltas,
 // the ring, control words, the grid, the library's Labs (where they fit).
 constexpr int32_t kLabWords = 2 * 64 * 4, kTermWords = kSlotWaves * 64 * 2,
-                  kFromWords = kSlotWaves * 64, kMutualWords = 64, kPackWords = 64, kCtrlWords = 8;
+                  kFromWords = kSlotWaves * 64, kMutualWords = 64, kPackWords = 2 * 64, kCtrlWords = 8;
 constexpr int32_t kFixedWords =
     kLabWords + kTermWords + kFromWords + kMutualWords + kPackWords + 3 * kRing + kCtrlWords;
 __host__ __device__ __forceinline__ int32_t grid_words(int32_t cells, int32_t kind) {
@@ -376,6 +382,11 @@ __device__ __forceinline__ uint32_t pack_round(int32_t advance, bool hopeful, bo
 
 constexpr uint32_t kNoLane = 255u;
 
+// How far a run has come.
+struct Progress {
+    int64_t s = 0, accepted = 0, evaluated = 0, rounds = 0;
+};
+
 template <typename G>
 struct AnnealShared {
     uint32_t* stamp;
@@ -383,7 +394,7 @@ struct AnnealShared {
     float4* terms;     // [kSlotWaves / 2][64]
     uint32_t* from;    // [kSlotWaves][64], kNoLane: none
     float* mutual;     // [64]
-    float* pack;       // [64]
+    float* pack;       // [2][64], the rounds use the first
     uint32_t *ring_xy1, *ring_xy2;
     float* ring_u;
     uint32_t* ctrl;
@@ -407,7 +418,7 @@ __device__ __forceinline__ void phase_end() {
 // the tag of its stamps, how its prefix is found, whether its reads must be
 // repeated, and how many deltas the last round left.
 struct Rounds {
-    int64_t s = 0;
+    int64_t s;
     uint32_t tag = 1;
     bool hopeful = true, reread = false;
     int32_t pending = 0;
@@ -525,11 +536,13 @@ __device__ __forceinline__ int32_t expected_prefix(uint32_t v1, uint32_t v2, uin
 
 template <typename G>
 __device__ __forceinline__ void slot_wave(const AnnealJob& job, const AnnealShared<G>& S, G* grid,
-                                          int w, int lane, int32_t words) {
+                                          int w, int lane, int32_t words,
+                                          const Progress& P) {
     Rounds R;
+    R.s = P.s;
     R.hopeful = !job.greedy;
     const int64_t max_iter = job.max_iter;
-    Place p = place_of(job, S, w, lane);
+    Place p = place_of(job, S, w, P.s + lane);
     Reads r = read_swap(job, S, grid, w, lane, p, R);
     phase_end();
     for (;;) {
@@ -596,20 +609,65 @@ __device__ __forceinline__ void slot_wave(const AnnealJob& job, const AnnealShar
     }
 }
 
+// What a swap adds to the cost, from its terms in the reference's order.
+template <typename G>
+__device__ __forceinline__ float added_terms(const AnnealShared<G>& S, int lane, bool adjacent) {
+    const float4 t0 = S.terms[lane], t1 = S.terms[64 + lane], t2 = S.terms[128 + lane],
+                 t3 = S.terms[192 + lane];
+    // the first cell's neighbours: old with m1, new with m2; the second's the reverse
+    float old_cost = t0.x, new_cost = t0.y;
+    old_cost += t0.z;
+    new_cost += t0.w;
+    old_cost += t1.x;
+    new_cost += t1.y;
+    old_cost += t1.z;
+    new_cost += t1.w;
+    old_cost += t2.y;
+    new_cost += t2.x;
+    old_cost += t2.w;
+    new_cost += t2.z;
+    old_cost += t3.y;
+    new_cost += t3.x;
+    old_cost += t3.w;
+    new_cost += t3.z;
+    if (adjacent) {
+        const float t = S.mutual[lane];
+        old_cost += t;
+        new_cost += t;
+    }
+    return new_cost - old_cost;
+}
+
+// Metropolis test u < exp(x), x = -delta/T (src/optimizer.rs:77-84).  An
+// estimate from the hardware reciprocal and exp2 is within 2^-15 of exp(x),
+// relative, down to 2^-126 (below, it may be 0, and u is either 0 or at least
+// 2^-24), so it decides alone unless u lies within 2^-10 of it (or it is 0 or
+// not finite); those lanes compute x and exp exactly.
+__device__ __forceinline__ bool accepts(const AnnealJob& job, float delta, float temp, float u) {
+    if (delta < 0.0f) return true;
+    if (job.greedy) return false;
+    const float e =
+        __builtin_amdgcn_exp2f(-delta * __builtin_amdgcn_rcpf(temp) * 1.44269504f);
+    if (__builtin_fabsf(u - e) > e * (1.0f / 1024.0f)) return u < e;
+    return u < exp_f32(-delta / temp);
+}
+
 // kHbm: the grid's swaps are complete at agent scope before other waves read
 // it (the barriers order the waves).
 template <typename G, bool kHbm>
 __device__ __forceinline__ void judge_wave(const AnnealJob& job, const AnnealShared<G>& S, G* grid,
-                                           int lane, int32_t words, AnnealOut* out) {
+                                           int lane, int32_t words, const Progress& P,
+                                           AnnealOut* out) {
     Rounds R;
+    R.s = P.s;
     R.hopeful = !job.greedy;
     const int32_t gw = job.grid_w, gh = job.grid_h;
     const int64_t max_iter = job.max_iter;
-    int64_t kbase = 0, accepted = 0, evaluated = 0, rounds = 0;
+    int64_t kbase = P.evaluated, accepted = P.accepted, evaluated = P.evaluated, rounds = P.rounds;
     // the last round's, for the traces
     const bool traced = job.trace_delta || job.trace_accept;
     float delta = 0.0f;
-    int64_t it = lane;
+    int64_t it = P.s + lane;
     bool acc = false, skip = true;
     int32_t first = 0;
     // the round's proposals (the next round's are taken in ahead)
@@ -621,7 +679,7 @@ __device__ __forceinline__ void judge_wave(const AnnealJob& job, const AnnealSha
         xy2 = S.ring_xy2[slot];
         u = S.ring_u[slot];
     };
-    take(0);
+    take(P.s);
     phase_end();
     for (;;) {
         // ---- terms
@@ -674,49 +732,8 @@ __device__ __forceinline__ void judge_wave(const AnnealJob& job, const AnnealSha
             p1 - p2 == gw || p2 - p1 == gw || (y1 == y2 && (x1 - x2 == 1 || x2 - x1 == 1));
         phase_end();
         // ---- decisions
-        const float4 t0 = S.terms[lane], t1 = S.terms[64 + lane], t2 = S.terms[128 + lane],
-                     t3 = S.terms[192 + lane];
-        // the first cell's neighbours: old with m1, new with m2; the second's the reverse
-        float old_cost = t0.x, new_cost = t0.y;
-        old_cost += t0.z;
-        new_cost += t0.w;
-        old_cost += t1.x;
-        new_cost += t1.y;
-        old_cost += t1.z;
-        new_cost += t1.w;
-        old_cost += t2.y;
-        new_cost += t2.x;
-        old_cost += t2.w;
-        new_cost += t2.z;
-        old_cost += t3.y;
-        new_cost += t3.x;
-        old_cost += t3.w;
-        new_cost += t3.z;
-        if (adjacent) {
-            const float t = S.mutual[lane];
-            old_cost += t;
-            new_cost += t;
-        }
-        delta = m1 == m2 ? 0.0f : new_cost - old_cost;
-        acc = false;
-        if (!skip) {
-            if (delta < 0.0f) {
-                acc = true;
-            } else if (!job.greedy) {
-                // Metropolis test u < exp(x), x = -delta/T (src/optimizer.rs:77-84).
-                // An estimate from the hardware reciprocal and exp2 is within
-                // 2^-15 of exp(x), relative, down to 2^-126 (below, it may be 0,
-                // and u is either 0 or at least 2^-24), so it decides alone
-                // unless u lies within 2^-10 of it (or it is 0 or not finite);
-                // those lanes compute x and exp exactly.
-                const float e = __builtin_amdgcn_exp2f(-delta * __builtin_amdgcn_rcpf(temp) *
-                                                       1.44269504f);
-                if (__builtin_fabsf(uniform - e) > e * (1.0f / 1024.0f))
-                    acc = uniform < e;
-                else
-                    acc = uniform < exp_f32(-delta / temp);
-            }
-        }
+        delta = m1 == m2 ? 0.0f : added_terms(S, lane, adjacent);
+        acc = !skip && accepts(job, delta, temp, uniform);
         const uint64_t acc_all = wave_ballot(acc);
         const uint64_t below = first >= 64 ? ~0ull : (1ull << first) - 1ull;
         const uint64_t rejected = nonskip & ~acc_all & below;
@@ -783,12 +800,13 @@ __device__ __forceinline__ void judge_wave(const AnnealJob& job, const AnnealSha
 // and a block only overwrites slots before s (filled <= s + 192).
 template <typename G>
 __device__ __forceinline__ void draw_wave(const AnnealJob& job, const AnnealShared<G>& S, int w,
-                                          int lane, int32_t words) {
+                                          int lane, int32_t words, const Progress& P) {
     Rounds R;
+    R.s = P.s;
     R.hopeful = !job.greedy;
     const uint32_t k = w == kDraw1Wave ? 0u : 2u;
     uint32_t* const ring = w == kDraw1Wave ? S.ring_xy1 : S.ring_xy2;
-    int64_t filled = kRing;
+    int64_t filled = P.s + kRing;
     phase_end();
     for (;;) {
         R.next(S.ctrl[kCtrlRound]);
@@ -810,8 +828,20 @@ __device__ __forceinline__ void draw_wave(const AnnealJob& job, const AnnealShar
 // accepted.
 struct CostSum {
     float cost, best;
-    int64_t improved = 0;
+    int64_t improved;
     float c;  // each lane's sum in the round being added
+    template <typename G>
+    __device__ __forceinline__ void load(const AnnealShared<G>& S) {
+        cost = __uint_as_float(uniform_copy(S.ctrl[kCtrlCost]));
+        best = __uint_as_float(uniform_copy(S.ctrl[kCtrlBest]));
+        improved = uniform_copy(reinterpret_cast<const int64_t*>(S.ctrl)[kCtrlImproved / 2]);
+    }
+    template <typename G>
+    __device__ __forceinline__ void store(const AnnealShared<G>& S) const {
+        S.ctrl[kCtrlCost] = __float_as_uint(cost);
+        S.ctrl[kCtrlBest] = __float_as_uint(best);
+        reinterpret_cast<int64_t*>(S.ctrl)[kCtrlImproved / 2] = improved;
+    }
     __device__ __forceinline__ void add(const float* pack, int lane) {
         c = add_lanes(cost, pack[lane], lane);
     }
@@ -832,12 +862,13 @@ struct CostSum {
 // The cost wave; it also draws u for the draw waves' blocks.
 template <typename G>
 __device__ __forceinline__ void cost_wave(const AnnealJob& job, const AnnealShared<G>& S, int lane,
-                                          int32_t words) {
+                                          int32_t words, const Progress& P) {
     Rounds R;
+    R.s = P.s;
     R.hopeful = !job.greedy;
     CostSum C;
-    C.cost = C.best = __uint_as_float(uniform_copy(S.ctrl[kCtrlCost]));
-    int64_t filled = kRing;
+    C.load(S);
+    int64_t filled = P.s + kRing;
     phase_end();
     for (;;) {
         R.next(S.ctrl[kCtrlRound]);
@@ -858,10 +889,297 @@ __device__ __forceinline__ void cost_wave(const AnnealJob& job, const AnnealShar
         C.add(S.pack, lane);
         C.count(R.pending, job.greedy != 0);
     }
-    if (lane == 0) {
-        S.ctrl[kCtrlCost] = __float_as_uint(C.cost);
-        S.ctrl[kCtrlBest] = __float_as_uint(C.best);
-        reinterpret_cast<int64_t*>(S.ctrl)[kCtrlImproved / 2] = C.improved;
+    if (lane == 0) C.store(S);
+}
+
+// ----------------------------------------------------------- whole blocks
+// While nearly all proposals are accepted (annealing starts hot), a block of
+// 64 need not end at the first swap that meets an earlier one's cell: if all
+// of them are taken to be accepted, what a lane's cells hold before its swap
+// follows from the swaps below it.  Every lane sets its bit in both its
+// cells' words.  The highest bit below a lane's own in a cell's word is the lane
+// k that wrote it last, and what k wrote is what k's other cell held before: a
+// pointer to one of 128 nodes (a lane, and 64 for its second cell).  The
+// pointers lead to ever lower lanes and end at a node whose cell nobody wrote,
+// so doubling them finds every node's origin, the cell of the grid that holds
+// its material, in log2 of the longest chain steps (two or three).  A block
+// commits the lanes before its first rejected one, and that one.
+//
+// Two phases a block: in the first the slot waves read the grid at the origins
+// and make terms, while a marking wave sets the bits of the next block; in the
+// second the judge decides and commits, while the marking wave finds the next
+// block's origins (which no commit changes).  After a rejection the judge sets
+// the bits anew, and a third phase finds the origins.
+//
+// A block takes 1.8 us: 1,600 cycles of terms, 2,100 of decisions (the judge
+// alone: sums, test, commit), 400 of reading the outcome.  With every slot wave
+// finding all origins for itself 1.9; with one table, set and read in the decisions,
+// 1.8 and no better at 300 cells, but 2.0 at 4,800; with tables that cells share,
+// for grids of any size, 2.1 (20,000 proposals on 200 x 120 cells 782 us).
+struct Touch {
+    uint64_t* words;  // [2][cells]
+    int32_t cells;
+    __device__ __forceinline__ uint64_t* of(int32_t block, int32_t p) const {
+        return &words[(block & 1) * cells + p];
+    }
+};
+// (every lane takes part: it has another lane's value)
+__device__ __forceinline__ int32_t from_lane(int32_t v, uint32_t k) {
+    return __builtin_amdgcn_ds_bpermute((int32_t)(k << 2), v);
+}
+// The origins of a block's nodes, and its materials, in `from`'s place.
+constexpr int32_t kOrigins = 128;
+
+// A block's proposals: what they are, and their bits.
+struct Proposals {
+    uint32_t xy1, xy2;
+    float u;
+    int32_t p1, p2;
+    bool skip;
+    template <typename G>
+    __device__ __forceinline__ void take(const AnnealJob& job, const AnnealShared<G>& S, G* grid,
+                                         int64_t it) {
+        const uint32_t slot = (uint32_t)it & (kRing - 1);
+        xy1 = S.ring_xy1[slot];
+        xy2 = S.ring_xy2[slot];
+        u = S.ring_u[slot];
+        p1 = (int32_t)(xy1 >> 16) * job.grid_w + (int32_t)(xy1 & 0xffffu);
+        p2 = (int32_t)(xy2 >> 16) * job.grid_w + (int32_t)(xy2 & 0xffffu);
+        // (which cells are empty never changes)
+        const int32_t m1 = gget(grid, p1), m2 = gget(grid, p2);
+        skip = (it >= job.max_iter) | (p1 == p2) | (m1 == kEmpty) | (m2 == kEmpty);
+    }
+    __device__ __forceinline__ void mark(const Touch& T, int32_t block, int lane) const {
+        if (!skip) {
+            atomicOr((unsigned long long*)T.of(block, p1), 1ull << lane);
+            atomicOr((unsigned long long*)T.of(block, p2), 1ull << lane);
+        }
+    }
+    __device__ __forceinline__ void clear(const Touch& T, int32_t block) const {
+        if (!skip) {
+            *T.of(block, p1) = 0ull;
+            *T.of(block, p2) = 0ull;
+        }
+    }
+    // Finds where the materials of all 128 nodes are.
+    template <typename G>
+    __device__ __forceinline__ void origins(const AnnealShared<G>& S, const Touch& T, int32_t block,
+                                            int lane) const {
+        const uint64_t below = (1ull << lane) - 1ull;
+        const uint64_t t1 = *T.of(block, p1) & below, t2 = *T.of(block, p2) & below;
+        int32_t c1 = p1, c2 = p2;
+        if (wave_ballot((t1 | t2) != 0)) {
+            // who wrote the cells last (nobody: this lane, for the reads), and
+            // whether as its first: then it left there what its second held
+            const uint32_t k1 = t1 ? 63u - (uint32_t)__builtin_clzll(t1) : (uint32_t)lane;
+            const uint32_t k2 = t2 ? 63u - (uint32_t)__builtin_clzll(t2) : (uint32_t)lane;
+            const int32_t f1 = from_lane(p1, k1), f2 = from_lane(p1, k2);
+            uint32_t n1 = t1 ? k1 | (f1 == p1 ? 64u : 0u) : (uint32_t)lane;
+            uint32_t n2 = t2 ? k2 | (f2 == p2 ? 64u : 0u) : (uint32_t)lane | 64u;
+            for (uint32_t both = n1 | n2 << 8;;) {
+                const uint32_t a1 = (uint32_t)from_lane((int32_t)both, n1 & 63u);
+                const uint32_t a2 = (uint32_t)from_lane((int32_t)both, n2 & 63u);
+                n1 = (n1 & 64u ? a1 >> 8 : a1) & 127u;
+                n2 = (n2 & 64u ? a2 >> 8 : a2) & 127u;
+                const uint32_t next = n1 | n2 << 8;
+                if (!wave_ballot(next != both)) break;
+                both = next;
+            }
+            const int32_t x1 = from_lane(p1, n1 & 63u), y1 = from_lane(p2, n1 & 63u);
+            const int32_t x2 = from_lane(p1, n2 & 63u), y2 = from_lane(p2, n2 & 63u);
+            c1 = n1 & 64u ? y1 : x1;
+            c2 = n2 & 64u ? y2 : x2;
+        }
+        S.from[kOrigins + lane] = (uint32_t)c1;
+        S.from[kOrigins + 64 + lane] = (uint32_t)c2;
+    }
+};
+
+// The node that a slot wave's neighbour comes from, -1: its own cell.
+__device__ __forceinline__ int32_t neighbour_node(const Touch& T, int32_t block, const Place& p,
+                                                  int lane) {
+    const uint64_t t = *T.of(block, p.q) & ((1ull << lane) - 1ull);
+    const uint32_t k = t ? 63u - (uint32_t)__builtin_clzll(t) : (uint32_t)lane;
+    const int32_t first = from_lane(p.p1, k);
+    return t ? (int32_t)(k | (first == p.q ? 64u : 0u)) : -1;
+}
+
+// The rounds take over for good when the blocks, over the last sixteen or so,
+// commit less than a round would, sqrt(pi / 8 cells) if all is accepted.
+template <typename G>
+__device__ __forceinline__ void follow_blocks(const AnnealJob& job, const AnnealShared<G>& S, G* grid,
+                                              const Touch& T, int w, int lane, Progress& P) {
+    const int32_t gw = job.grid_w;
+    const int64_t max_iter = job.max_iter;
+    const int32_t least =
+        16 * min(48, (int32_t)(0.6267f * __builtin_sqrtf((float)(job.grid_w * job.grid_h))));
+    int64_t filled = kRing;
+    int32_t block = 0, pending = 0, added_last = 0, mean = 16 * 64;
+    const bool traced = job.trace_delta || job.trace_accept;
+    bool again = true;
+    CostSum C;
+    Place p;
+    int32_t node;
+    Proposals now, next;
+    if (w == kJudgeWave) {
+        now.take(job, S, grid, lane);
+        now.mark(T, 0, lane);
+    }
+    if (w == kCostWave) C.load(S);
+    phase_end();
+    for (;;) {
+        // ---- terms
+        if (again) {
+            if (w < kSlotWaves) {
+                p = place_of(job, S, w, P.s + lane);
+                node = neighbour_node(T, block, p, lane);
+            } else if (w == kMarkWave) {
+                next.take(job, S, grid, P.s + lane);
+                next.origins(S, T, block, lane);
+            }
+            phase_end();
+        }
+        uint64_t t1, t2, nonskip;
+        float temp;
+        if (w < kSlotWaves) {
+            const int32_t o1 = (int32_t)S.from[kOrigins + lane],
+                          o2 = (int32_t)S.from[kOrigins + 64 + lane],
+                          on = (int32_t)S.from[kOrigins + max(node, 0)];
+            const int32_t oa = node < 0 ? p.q : on;
+            const int32_t m1 = gget(grid, o1), m2 = gget(grid, o2), a = gget(grid, oa);
+            if (w == 0) {
+                S.from[lane] = (uint32_t)m1;
+                S.from[64 + lane] = (uint32_t)m2;
+            }
+            float4 l1 = make_float4(0, 0, 0, 0), l2 = l1, la = l1;
+            if (S.labs) {
+                if (job.n > 0) {
+                    l1 = S.labs[max(m1, 0)];
+                    l2 = S.labs[max(m2, 0)];
+                    la = S.labs[max(a, 0)];
+                }
+            } else {
+                // (a gather from memory takes the address unit 64 cycles: each
+                // Lab once)
+                if (job.n > 0) {
+                    la = gload4(job.lab4, max(a, 0));
+                    if ((w & 3) == 0) S.lab_m[w * 16 + lane] = gload4(job.lab4, max(w == 0 ? m1 : m2, 0));
+                }
+                phase_end();
+                l1 = S.lab_m[lane];
+                l2 = S.lab_m[64 + lane];
+            }
+            const bool ok = p.in && !p.self && a != kEmpty;
+            const float c1 = adj_term(l1, la), c2 = adj_term(l2, la);
+            reinterpret_cast<float2*>(S.terms)[((w >> 1) * 64 + lane) * 2 + (w & 1)] =
+                make_float2(ok ? c1 : 0.0f, ok ? c2 : 0.0f);
+            // the partner as a neighbour of the first cell: the mutual term
+            if (w < 4 && p.self) S.mutual[lane] = c1;
+        } else {
+            if (w == kJudgeWave) {
+                nonskip = wave_ballot(!now.skip);
+                temp = 1.0f;
+                if (!now.skip) temp = gload(job.temps, P.evaluated + lanes_before(nonskip));
+                // the lanes above this one that write its cells
+                const uint64_t above = ~((2ull << lane) - 1ull);
+                t1 = *T.of(block, now.p1) & above;
+                t2 = *T.of(block, now.p2) & above;
+                next.take(job, S, grid, P.s + 64 + lane);
+            } else if (w == kMarkWave) {
+                next.take(job, S, grid, P.s + 64 + lane);
+                next.mark(T, block + 1, lane);
+            } else if (w == kCostWave && added_last) {
+                C.count(added_last, false);
+                added_last = 0;
+            }
+            if (!S.labs) phase_end();
+        }
+        phase_end();
+        // ---- decisions
+        if (w < kSlotWaves) {
+            p = place_of(job, S, w, P.s + 64 + lane);
+            node = neighbour_node(T, block + 1, p, lane);
+        } else if (w == kMarkWave) {
+            next.origins(S, T, block + 1, lane);
+        } else if (w == kJudgeWave) {
+            const int32_t m1 = (int32_t)S.from[lane], m2 = (int32_t)S.from[64 + lane];
+            const bool adjacent =
+                now.p1 - now.p2 == gw || now.p2 - now.p1 == gw ||
+                ((now.xy1 >> 16) == (now.xy2 >> 16) &&
+                 (now.p1 - now.p2 == 1 || now.p2 - now.p1 == 1));
+            const float added = added_terms(S, lane, adjacent);
+            const float delta = m1 == m2 ? 0.0f : added;
+            const bool acc = !now.skip && accepts(job, delta, temp, now.u);
+            const uint64_t rejected = nonskip & ~wave_ballot(acc);
+            const int32_t r = rejected ? __ffsll((unsigned long long)rejected) - 1 : 64;
+            const int64_t remain = max_iter - P.s;
+            const int32_t end = remain < 64 ? (int32_t)remain : 64, advance = min(r + 1, end);
+            const uint64_t commit = r >= 64 ? ~0ull : (1ull << r) - 1ull;
+            const uint64_t done = advance >= 64 ? ~0ull : (1ull << advance) - 1ull;
+            // of the committed lanes that write a cell, the last
+            const bool keep = lane_in(nonskip & commit);
+            if (keep && !(t1 & commit)) gput(grid, now.p1, m2);
+            if (keep && !(t2 & commit)) gput(grid, now.p2, m1);
+            now.clear(T, block);
+            S.pack[64 * (block & 1) + lane] = keep ? delta : 0.0f;
+            if (traced && lane < advance) {
+                const int64_t it = P.s + lane;
+                if (job.trace_delta)
+                    gstore(job.trace_delta, it, now.skip ? __int_as_float(0x7fc00000) : delta);
+                if (job.trace_accept) gstore(job.trace_accept, it, (uint8_t)(acc ? 1 : 0));
+            }
+            mean += advance - mean / 16;
+            const bool stop = P.s + advance >= max_iter || mean < least;
+            if (lane == 0)
+                S.ctrl[kCtrlRound] = (uint32_t)advance | (stop ? 128u : 0u) |
+                                     (uint32_t)__popcll(nonskip & commit) << 8 |
+                                     (uint32_t)__popcll(nonskip & done) << 16;
+            if (advance != 64 && !stop) {
+                // (one wave's LDS operations are done in order)
+                next.clear(T, block + 1);
+                asm volatile("" ::: "memory");
+                next.take(job, S, grid, P.s + advance + lane);
+                next.mark(T, block + 1, lane);
+            }
+            now = next;
+        } else {
+            if (w == kCostWave && pending) {
+                C.add(S.pack + 64 * ((block - 1) & 1), lane);
+                added_last = pending;
+            }
+            if (filled <= P.s + kRing - 64) {
+                const uint64_t j = (uint64_t)(filled + lane);
+                const uint32_t slot = (uint32_t)j & (kRing - 1);
+                if (w == kCostWave) {
+                    S.ring_u[slot] = draw_unit(job.seed, j);
+                } else {
+                    S.ring_xy1[slot] = (uint32_t)draw_range(job.seed, j, 0, job.grid_w) |
+                                       (uint32_t)draw_range(job.seed, j, 1, job.grid_h) << 16;
+                    S.ring_xy2[slot] = (uint32_t)draw_range(job.seed, j, 2, job.grid_w) |
+                                       (uint32_t)draw_range(job.seed, j, 3, job.grid_h) << 16;
+                }
+                filled += 64;
+            }
+        }
+        phase_end();
+        const uint32_t v = (uint32_t)__builtin_amdgcn_readfirstlane((int32_t)S.ctrl[kCtrlRound]);
+        const int32_t advance = (int32_t)(v & 127u);
+        P.s += advance;
+        pending = (int32_t)(v >> 8 & 127u);
+        P.accepted += pending;
+        P.evaluated += (int64_t)(v >> 16);
+        ++P.rounds;
+        ++block;
+        again = advance != 64;
+        if (v & 128u) break;
+    }
+    if (w == kCostWave) {
+        if (added_last) C.count(added_last, false);
+        if (pending) {
+            C.add(S.pack + 64 * ((block - 1) & 1), lane);
+            C.count(pending, false);
+        }
+        if (lane == 0) C.store(S);
     }
 }
 
@@ -875,7 +1193,7 @@ __global__ __launch_bounds__(kAnnealThreads) void anneal_kernel(AnnealJob single
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int32_t cells = job.grid_w * job.grid_h;
-    const int32_t words = stamp_words(cells);
+    const int32_t words = stamp_words(cells, job.blocks != 0);
     typedef typename std::conditional<kHbm, HbmGrid, G>::type Grid;
     AnnealShared<Grid> S;
     S.stamp = sm;
@@ -919,14 +1237,18 @@ __global__ __launch_bounds__(kAnnealThreads) void anneal_kernel(AnnealJob single
             for (int k = 0; k < 4; ++k)
                 if (i + k * kAnnealThreads < job.n) labs[i + k * kAnnealThreads] = l[k];
         }
-    // the first proposals (coordinates are in the grid past max_iter too)
-    if (tid < kRing) {
-        S.ring_xy1[tid] = (uint32_t)draw_range(job.seed, tid, 0, job.grid_w) |
-                          (uint32_t)draw_range(job.seed, tid, 1, job.grid_h) << 16;
-        S.ring_xy2[tid] = (uint32_t)draw_range(job.seed, tid, 2, job.grid_w) |
-                          (uint32_t)draw_range(job.seed, tid, 3, job.grid_h) << 16;
-        S.ring_u[tid] = draw_unit(job.seed, tid);
-    }
+    // the next proposals (coordinates are in the grid past max_iter too)
+    auto draw_ring = [&](int64_t from) {
+        if (tid >= kRing) return;
+        const uint64_t d = (uint64_t)(from + tid);
+        const uint32_t slot = (uint32_t)d & (kRing - 1);
+        S.ring_xy1[slot] = (uint32_t)draw_range(job.seed, d, 0, job.grid_w) |
+                           (uint32_t)draw_range(job.seed, d, 1, job.grid_h) << 16;
+        S.ring_xy2[slot] = (uint32_t)draw_range(job.seed, d, 2, job.grid_w) |
+                           (uint32_t)draw_range(job.seed, d, 3, job.grid_h) << 16;
+        S.ring_u[slot] = draw_unit(job.seed, d);
+    };
+    draw_ring(0);
     __syncthreads();
     const float initial =
         S.labs ? total_cost_block(grid, job.grid_w, job.grid_h, TermLds{S.labs}, S.stamp)
@@ -934,20 +1256,35 @@ __global__ __launch_bounds__(kAnnealThreads) void anneal_kernel(AnnealJob single
     __syncthreads();
     for (int32_t i = tid; i < words; i += kAnnealThreads) S.stamp[i] = 0u;
     if (tid == 0) {
-        S.ctrl[kCtrlCost] = __float_as_uint(initial);
-        S.ctrl[kCtrlRound] = pack_round(0, !job.greedy, false, 0);
+        S.ctrl[kCtrlCost] = S.ctrl[kCtrlBest] = __float_as_uint(initial);
+        reinterpret_cast<int64_t*>(S.ctrl)[kCtrlImproved / 2] = 0;
     }
+    __syncthreads();
+    Progress P;
+    if constexpr (!kHbm) {
+        if (job.blocks && job.max_iter > 0) {
+            const Touch T{reinterpret_cast<uint64_t*>(sm), cells};
+            follow_blocks(job, S, grid, T, w, lane, P);
+            if (P.s < job.max_iter) {
+                __syncthreads();
+                draw_ring(P.s);
+                for (int32_t i = tid; i < words; i += kAnnealThreads) S.stamp[i] = 0u;
+            }
+            __syncthreads();
+        }
+    }
+    if (tid == 0) S.ctrl[kCtrlRound] = pack_round(0, !job.greedy, false, 0);
     __syncthreads();
 
     AnnealOut r{};
     if (w < kSlotWaves)
-        slot_wave(job, S, grid, w, lane, words);
+        slot_wave(job, S, grid, w, lane, words, P);
     else if (w == kJudgeWave)
-        judge_wave<Grid, kHbm>(job, S, grid, lane, words, &r);
+        judge_wave<Grid, kHbm>(job, S, grid, lane, words, P, &r);
     else if (w != kCostWave)
-        draw_wave(job, S, w, lane, words);
+        draw_wave(job, S, w, lane, words, P);
     else
-        cost_wave(job, S, lane, words);
+        cost_wave(job, S, lane, words, P);
     __syncthreads();
     if constexpr (!kHbm)
         for (int32_t i = tid; i < cells; i += kAnnealThreads) gstore(job.grid, i, (int32_t)grid[i]);
@@ -961,17 +1298,36 @@ __global__ __launch_bounds__(kAnnealThreads) void anneal_kernel(AnnealJob single
     }
 }
 
+namespace {
+size_t anneal_lds_bytes(int32_t cells, int32_t kind, int32_t labs, bool blocks) {
+    return sizeof(uint32_t) *
+               ((size_t)stamp_words(cells, blocks) + kFixedWords + grid_words(cells, kind)) +
+           sizeof(float4) * (size_t)labs;
+}
+// Whole blocks commit up to 64 proposals in 1.8 us, a round about sqrt(pi / 8
+// cells) in 1.0.  Measured (anneal, us, rounds alone and with blocks): 300
+// cells 112 and 44, 1,400 61 and 47, 4,800 84 and 81; from about 5,000 on the
+// rounds are as good.
+constexpr int32_t kFollowCells = 5120;
+}  // namespace
+
 int32_t anneal_kind(int32_t cells, int32_t n, int32_t gw, int32_t gh, size_t max_lds) {
-    if (n < 32768 && anneal_lds_bytes(cells, kAnnealNarrow, 0) <= max_lds) return kAnnealNarrow;
-    if (anneal_lds_bytes(cells, kAnnealWide, 0) <= max_lds) return kAnnealWide;
-    if (gw < 65536 && gh < 65536 && anneal_lds_bytes(cells, kAnnealHbm, 0) <= max_lds)
-        return kAnnealHbm;
+    auto fits = [&](int32_t kind) { return anneal_lds_bytes(cells, kind, 0, false) <= max_lds; };
+    if (n < 32768 && fits(kAnnealNarrow)) return kAnnealNarrow;
+    if (fits(kAnnealWide)) return kAnnealWide;
+    if (gw < 65536 && gh < 65536 && fits(kAnnealHbm)) return kAnnealHbm;
     return -1;
 }
 
-size_t anneal_lds_bytes(int32_t cells, int32_t kind, int32_t labs) {
-    return sizeof(uint32_t) * ((size_t)stamp_words(cells) + kFixedWords + grid_words(cells, kind)) +
-           sizeof(float4) * (size_t)labs;
+// The Labs have the first claim on LDS, then the blocks' tables.
+AnnealLayout anneal_layout(int32_t cells, int32_t kind, int32_t n, bool greedy, bool want_labs,
+                           size_t max_lds) {
+    AnnealLayout l;
+    l.labs = want_labs && anneal_lds_bytes(cells, kind, n, false) <= max_lds;
+    l.blocks = !greedy && kind != kAnnealHbm && cells <= kFollowCells &&
+               anneal_lds_bytes(cells, kind, l.labs ? n : 0, true) <= max_lds;
+    l.lds = anneal_lds_bytes(cells, kind, l.labs ? n : 0, l.blocks);
+    return l;
 }
 
 namespace {

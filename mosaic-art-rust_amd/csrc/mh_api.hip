@@ -343,8 +343,8 @@ int run_anneal(mh_context* ctx, const mh_library* lib, int32_t* d_grid, int32_t 
     if (kind < 0)
         return fail(MH_ERR_UNSUPPORTED, "annealing a %d x %d grid: a side of 65,536 or more", gw,
                     gh);
-    const bool labs = anneal_lds_bytes(cells, kind, lib->n) <= ctx->max_lds;
-    const size_t lds = anneal_lds_bytes(cells, kind, labs ? lib->n : 0);
+    const AnnealLayout lay =
+        anneal_layout(cells, kind, lib->n, p->greedy != 0, true, ctx->max_lds);
     const float* temps = temps_ready;
     int rc;
     if (!p->greedy && !temps && !noalloc) {
@@ -357,7 +357,8 @@ int run_anneal(mh_context* ctx, const mh_library* lib, int32_t* d_grid, int32_t 
     AnnealJob job;
     job.lab4 = lib->d_lab4;
     job.n = lib->n;
-    job.labs_in_lds = labs ? 1 : 0;
+    job.labs_in_lds = lay.labs ? 1 : 0;
+    job.blocks = lay.blocks ? 1 : 0;
     job.grid = d_grid;
     job.grid_w = gw;
     job.grid_h = gh;
@@ -369,7 +370,7 @@ int run_anneal(mh_context* ctx, const mh_library* lib, int32_t* d_grid, int32_t 
     job.trace_accept = d_trace_accept;
     job.result = d_out;
     phase_begin(ctx, MH_PHASE_ANNEAL);
-    launch_anneal_single(job, kind, lds, ctx->stream);
+    launch_anneal_single(job, kind, lay.lds, ctx->stream);
     phase_end(ctx, MH_PHASE_ANNEAL);
     HIPCHK(hipGetLastError());
     return MH_OK;

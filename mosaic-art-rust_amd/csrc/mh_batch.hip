@@ -286,7 +286,10 @@ int build_plan(const std::vector<JobSpec>& specs, const std::vector<uint8_t*>& j
             aj.lab4 = lib->d_lab4;
             aj.n = s.n;
             const int32_t kind = s.anneal_kind;
-            aj.labs_in_lds = labs && anneal_lds_bytes(s.cells, kind, s.n) <= lib->ctx->max_lds ? 1 : 0;
+            const AnnealLayout lay =
+                anneal_layout(s.cells, kind, s.n, false, labs, lib->ctx->max_lds);
+            aj.labs_in_lds = lay.labs ? 1 : 0;
+            aj.blocks = lay.blocks ? 1 : 0;
             aj.grid = grid;
             aj.grid_w = s.gw;
             aj.grid_h = s.gh;
@@ -297,8 +300,7 @@ int build_plan(const std::vector<JobSpec>& specs, const std::vector<uint8_t*>& j
             aj.result = d_aout + i;
             by_kind[kind].push_back(aj);
             job_of_kind[kind].push_back(i);
-            const size_t al = anneal_lds_bytes(s.cells, kind, aj.labs_in_lds ? s.n : 0);
-            if (al > p->anneal_lds[kind]) p->anneal_lds[kind] = al;
+            if (lay.lds > p->anneal_lds[kind]) p->anneal_lds[kind] = lay.lds;
         }
         // a13-a16: adjustments, composite
         float4* adj = s.adjust ? at<float4>(m, s.o_adj) : nullptr;

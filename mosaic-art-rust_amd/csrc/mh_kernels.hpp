@@ -60,6 +60,7 @@ struct AnnealJob {
     uint64_t seed;
     int32_t greedy;
     int32_t labs_in_lds;      // LDS holds the library's Labs too
+    int32_t blocks;           // the run begins in whole blocks of proposals
     float* trace_delta;       // optional, max_iter entries
     uint8_t* trace_accept;
     AnnealOut* result;
@@ -190,8 +191,14 @@ void launch_place_batch(const PlaceJob* d_jobs, int32_t n_jobs, bool raster, siz
 enum : int32_t { kAnnealNarrow = 0, kAnnealWide = 1, kAnnealHbm = 2 };
 // The first variant that holds the job in max_lds bytes of LDS, -1 if none.
 int32_t anneal_kind(int32_t cells, int32_t n, int32_t gw, int32_t gh, size_t max_lds);
-// labs: the Labs that LDS holds too (the library's, or 0).
-size_t anneal_lds_bytes(int32_t cells, int32_t kind, int32_t labs);
+// What else of a job of that variant LDS holds, and how many bytes: the
+// library's Labs (if wanted), the tables of whole blocks.
+struct AnnealLayout {
+    bool labs, blocks;
+    size_t lds;
+};
+AnnealLayout anneal_layout(int32_t cells, int32_t kind, int32_t n, bool greedy, bool want_labs,
+                           size_t max_lds);
 void launch_anneal_single(const AnnealJob& job, int32_t kind, size_t lds_bytes, hipStream_t stream);
 void launch_anneal_batch(const AnnealJob* d_jobs, int32_t n_jobs, int32_t kind, size_t lds_bytes,
                          hipStream_t stream);
