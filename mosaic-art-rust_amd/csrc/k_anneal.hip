@@ -332,8 +332,8 @@ __device__ float total_cost_block(const G* grid, int32_t gw, int32_t gh, const T
 // Measured against one wave that gathered its terms from a matrix of all pairs
 // and added the initial cost one term after another: 1,000 proposals on 20 x
 // 15 cells 332 -> 112 us (200 rounds -> 97; in 17 blocks 44 us), 2,000 on 80 x 60
-// 340 -> 84 (100 -> 54; 32 blocks 81), 2,000 on 206 x 116 600 -> 120, 20,000 on
-// 200 x 120 1,650 -> 488.  A round takes 1.0 us for 3.3 (1.5 with the reads as a
+// 340 -> 84 (100 -> 54), 2,000 on 206 x 116 600 -> 120, 20,000 on 200 x 120 1,650
+// -> 488.  A round takes 1.0 us for 3.3 (1.5 with the reads as a
 // phase of their own, 1.15 with two neighbours to each of four slot waves):
 // 1,450 cycles of terms (the judge's taking in), 1,150 of decisions.
 constexpr int kMarkWave = 9;  // in whole blocks; wave 10 draws
@@ -1005,14 +1005,15 @@ __device__ __forceinline__ int32_t neighbour_node(const Touch& T, int32_t block,
 }
 
 // The rounds take over for good when the blocks, over the last sixteen or so,
-// commit less than a round would, sqrt(pi / 8 cells) if all is accepted.
+// commit less than rounds do in a block's time: a round commits some 0.55
+// sqrt(cells) if all is accepted, and a block takes 1.6 to 1.8 times as long.
 template <typename G>
 __device__ __forceinline__ void follow_blocks(const AnnealJob& job, const AnnealShared<G>& S, G* grid,
                                               const Touch& T, int w, int lane, Progress& P) {
     const int32_t gw = job.grid_w;
     const int64_t max_iter = job.max_iter;
     const int32_t least =
-        16 * min(48, (int32_t)(0.6267f * __builtin_sqrtf((float)(job.grid_w * job.grid_h))));
+        (int32_t)(16.0f * 0.88f * __builtin_sqrtf((float)(job.grid_w * job.grid_h)));
     int64_t filled = kRing;
     int32_t block = 0, pending = 0, added_last = 0, mean = 16 * 64;
     const bool traced = job.trace_delta || job.trace_accept;
@@ -1304,11 +1305,11 @@ size_t anneal_lds_bytes(int32_t cells, int32_t kind, int32_t labs, bool blocks) 
                ((size_t)stamp_words(cells, blocks) + kFixedWords + grid_words(cells, kind)) +
            sizeof(float4) * (size_t)labs;
 }
-// Whole blocks commit up to 64 proposals in 1.8 us, a round about sqrt(pi / 8
-// cells) in 1.0.  Measured (anneal, us, rounds alone and with blocks): 300
-// cells 112 and 44, 1,400 61 and 47, 4,800 84 and 81; from about 5,000 on the
-// rounds are as good.
-constexpr int32_t kFollowCells = 5120;
+// Whole blocks commit up to 64 proposals in 1.6-1.8 us, a round some 0.55
+// sqrt(cells) in 1.0.  Measured (anneal, us, rounds alone and with blocks): 300
+// cells 112 and 44, 1,400 61 and 47, 4,800 84 and 81 on one picture, 79 and 82
+// on another.
+constexpr int32_t kFollowCells = 4096;
 }  // namespace
 
 int32_t anneal_kind(int32_t cells, int32_t n, int32_t gw, int32_t gh, size_t max_lds) {

@@ -3,7 +3,7 @@
 The cases stand where a block's chain of cells, its end or the change to rounds
 can go wrong: proposal counts around one and two blocks and the ring of 256
 draws, grids of so few cells that every swap meets the ones before (the longest
-chains) and of one row or column, the largest grid taken (5,120 cells) and the
+chains) and of one row or column, the largest grid taken (4,096 cells) and the
 next, Labs in LDS and in memory, and too many for both them and the blocks'
 tables, ids of 16 and 32 bits, empty cells, equal materials, and temperatures
 that reject one proposal in a few blocks, one in a few proposals, and most.
@@ -27,10 +27,10 @@ CASES = [
     (24, 18, 10500, 10500, 0.0, 1200, 20.0, 0.9995),
     (24, 18, 33000, 33000, 0.05, 900, 50.0, 0.999),
     (50, 28, 500, 500, 0.0, 3000, 100.0, 0.998),
-    (80, 60, 5500, 5500, 0.0, 700, 100.0, 0.99995),
-    (80, 64, 1500, 1500, 0.0, 2500, 30.0, 0.9995),
-    (80, 64, 1500, 1500, 0.01, 63, 100.0, 0.99995),
-    (3, 1707, 200, 200, 0.0, 1300, 100.0, 0.99995),
+    (63, 65, 7500, 7500, 0.0, 700, 100.0, 0.99995),
+    (64, 64, 1500, 1500, 0.0, 2500, 30.0, 0.9995),
+    (64, 64, 1500, 1500, 0.01, 63, 100.0, 0.99995),
+    (17, 241, 200, 200, 0.0, 1300, 100.0, 0.99995),
 ]
 
 
