@@ -303,6 +303,9 @@ static_assert(kUpPrepColumns + 6 * kGroup < kUpRing,
 __host__ __device__ __forceinline__ int32_t ring_words(int32_t grid_w) {
     return grid_w >= kUpPrepColumns ? grid_w + 5 * kGroup : kUpRing;
 }
+// (not monotone in the width: kUpPrepColumns wide grids have the shortest)
+constexpr int32_t kLeastRingColumns = kUpPrepColumns;
+static_assert(kUpPrepColumns + 5 * kGroup <= kUpRing, "kLeastRingColumns");
 
 // LDS of the chain, in words: events, guard and counts, lane scratch, winner
 // ring, prepared rows, lists in preparation, material Labs (where they fit).
@@ -1324,9 +1327,16 @@ size_t place_raster_lds_bytes(int32_t grid_w, int32_t n, int32_t form) {
 // cell's Labs come from LDS in 0.4 us, from memory in 0.7-1 us.  Without room
 // for the lists (33,700 to 40,700 materials) a cell costs 0.67 us plain; one
 // wave that read ahead in registers took 0.59 there.
-int32_t raster_form(int32_t grid_w, int32_t n, bool outputs, bool labs, size_t max_lds) {
-    for (int32_t form = grid_w < 3 || outputs ? kRasterPlain : labs ? kRasterLabs : kRasterLists;
-         form >= 0; --form)
+//
+// Without the materials' largest terms a list's entries would all look safe,
+// so such a library's runs are plain; lists_taken says which libraries need
+// the terms (33,828 to 33,847 materials: in grids of 48 to 67 columns only).
+bool lists_taken(int32_t n, size_t max_lds) {
+    return place_raster_lds_bytes(kLeastRingColumns, n, kRasterLists) <= max_lds;
+}
+int32_t raster_form(int32_t grid_w, int32_t n, bool outputs, bool labs, bool terms, size_t max_lds) {
+    const bool plain = grid_w < 3 || outputs || !terms;
+    for (int32_t form = plain ? kRasterPlain : labs ? kRasterLabs : kRasterLists; form >= 0; --form)
         if (place_raster_lds_bytes(grid_w, n, form) <= max_lds) return form;
     return -1;
 }

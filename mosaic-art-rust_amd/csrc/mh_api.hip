@@ -217,7 +217,9 @@ int run_place(mh_context* ctx, const mh_library* lib, const float* d_cell_lab, i
               uint8_t* d_stage, float* d_dist, float* d_score, int32_t* d_stats,
               CandRec* cand_buf = nullptr) {
     const int32_t cells = gw * gh;
-    const int32_t form = raster ? raster_form(gw, lib->n, d_stage || d_dist || d_score, true, ctx->max_lds) : -1;
+    const int32_t form = raster ? raster_form(gw, lib->n, d_stage || d_dist || d_score, true,
+                                                   lib->has_terms, ctx->max_lds)
+                                     : -1;
     size_t lds =
         form >= 0 ? place_raster_lds_bytes(gw, lib->n, form) : place_lds_bytes(cells, lib->n);
     // state beyond LDS: the general chain with grid and counts in HBM (it
@@ -849,11 +851,11 @@ static int library_upload_lab(mh_library* lib) {
     lib->nb = (int32_t)nb;
     HIPCHK(hipMemcpyAsync(lib->d_tables, tables.data(), tables.size(), hipMemcpyHostToDevice,
                           lib->ctx->stream));
-    // largest adjacency terms, for the placement's prepared lists (a library
-    // that has none in the narrowest grid does not read them)
-    if (place_raster_lds_bytes(1, n, kRasterLists) <= lib->ctx->max_lds) {
+    // largest adjacency terms, for the placement's prepared lists
+    if (lists_taken(n, lib->ctx->max_lds)) {
         launch_near_terms(lib->d_lab4, n, lib->ctx->stream);
         HIPCHK(hipGetLastError());
+        lib->has_terms = true;
     }
     return sync(lib->ctx);  // (any stream may read the tables; `tables` is pageable and local)
 }

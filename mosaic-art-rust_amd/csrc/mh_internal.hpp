@@ -136,6 +136,7 @@ struct mh_library {
     std::vector<float> h_lab;  // n x 3
     void* d_tables = nullptr;  // one allocation for the ten arrays below
     float4* d_lab4 = nullptr;
+    bool has_terms = false;  // d_lab4 holds the largest adjacency terms
     float* d_L = nullptr;
     float* d_A = nullptr;
     float* d_B = nullptr;

@@ -175,10 +175,13 @@ size_t place_lds_bytes(int32_t cells, int32_t n);
 // also the prepared candidate lists (kRasterLists), also the material Labs
 // (kRasterLabs; read from memory otherwise).  raster_form: the first of
 // kRasterLabs (if labs), kRasterLists, kRasterPlain that fits max_lds bytes,
-// the grid and the run (outputs: it wants every cell's stage, distance or
-// score), -1 if none does.
+// the grid, the run (outputs: it wants every cell's stage, distance or score)
+// and the library (terms: lab4 holds its largest terms), -1 if none does.
+// lists_taken: whether any grid's run takes a library of n materials in lists,
+// so that it needs its terms.
 constexpr int32_t kRasterPlain = 0, kRasterLists = 1, kRasterLabs = 2;
-int32_t raster_form(int32_t grid_w, int32_t n, bool outputs, bool labs, size_t max_lds);
+int32_t raster_form(int32_t grid_w, int32_t n, bool outputs, bool labs, bool terms, size_t max_lds);
+bool lists_taken(int32_t n, size_t max_lds);
 size_t place_raster_lds_bytes(int32_t grid_w, int32_t n, int32_t form);
 // One job passed by value (kernel argument), or n_jobs jobs from a device
 // array; lds_bytes 0 (general chain): grid and counts in the job's buffers.
