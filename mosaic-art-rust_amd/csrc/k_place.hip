@@ -690,7 +690,6 @@ struct Decision {
     uint32_t w;      // the winner's entry id
     int32_t rank;
     int32_t stage;   // 0 scored scan, 1 fallback first-placeable, 2 nearest_one
-    float dist, score;
     bool reset;
 };
 
@@ -719,12 +718,12 @@ __device__ __forceinline__ RowLabs load_labs(const PlaceJob& job, const RawRow& 
 
 // The evaluation of a cell from its whole row, and the usage-reset fallback
 // (src/main.rs:385-475).  Estimates rule out all but the few candidates that
-// can win; with score_wanted, or when those are several, exact scores decide.
+// can win; when those are several, exact scores decide.
 __device__ __forceinline__ Decision decide_from_row(const PlaceJob& job, uint32_t* counts,
                                                     uint32_t limit, const RawRow& row,
                                                     const RowLabs& labs, uint32_t up, uint32_t left,
-                                                    const Neighbours& nb, bool score_wanted,
-                                                    bool may_reset, int lane) {
+                                                    const Neighbours& nb, bool may_reset,
+                                                    int lane) {
     const uint32_t kNone = 0xffffffffu;
     const uint32_t a0 = entry_id((int32_t)(uint32_t)row.r0), a1 = entry_id((int32_t)(uint32_t)row.r1);
     const float d0 = __uint_as_float((uint32_t)(row.r0 >> 32));
@@ -738,7 +737,6 @@ __device__ __forceinline__ Decision decide_from_row(const PlaceJob& job, uint32_
     Decision r;
     r.stage = 0;
     r.reset = false;
-    uint32_t score = 0;
     if (b0 | b1) {
         // keys: the scores' bits (no score is negative)
         uint32_t k0 = lane_in(b0) ? __float_as_uint(d0) : kNone;
@@ -752,7 +750,7 @@ __device__ __forceinline__ Decision decide_from_row(const PlaceJob& job, uint32_
             const float far = rival_bound(__uint_as_float(wave_min_u32(k0 < k1 ? k0 : k1)), job.weight);
             b0 &= wave_ballot(!(e0 > far));
             b1 &= wave_ballot(!(e1 > far));
-            alone = !score_wanted && __popcll(b0) + __popcll(b1) == 1;
+            alone = __popcll(b0) + __popcll(b1) == 1;
         }
         if (!alone && job.weight > 0.0f) {
             // one evaluation does for both candidates of a lane unless both are in
@@ -765,7 +763,7 @@ __device__ __forceinline__ Decision decide_from_row(const PlaceJob& job, uint32_
                 k1 = lane_in(b1) ? __float_as_uint(exact_score(d1, labs.l1, nb, job.weight)) : kNone;
         }
         if (!alone) {
-            score = wave_min_u32(k0 < k1 ? k0 : k1);
+            const uint32_t score = wave_min_u32(k0 < k1 ? k0 : k1);
             b0 &= wave_ballot(k0 == score);
             b1 &= wave_ballot(k1 == score);
         }
@@ -782,8 +780,6 @@ __device__ __forceinline__ Decision decide_from_row(const PlaceJob& job, uint32_
     }
     r.rank = b0 ? __ffsll((unsigned long long)b0) - 1 : 63 + __ffsll((unsigned long long)b1);
     r.w = r.rank < 64 ? readlane_u(a0, r.rank & 63) : readlane_u(a1, r.rank & 63);
-    r.dist = r.rank < 64 ? readlane_f(d0, r.rank & 63) : readlane_f(d1, r.rank & 63);
-    r.score = r.stage == 0 ? __uint_as_float(score) : r.dist;
     return r;
 }
 
@@ -867,12 +863,13 @@ __device__ __forceinline__ uint32_t decide_flagged(const PlaceJob& job, const Ch
     if (!decide_from_list(job, a, d, usable, lab, nb, &w)) {
         const RawRow row = load_row(job, c, A.cells, lane);
         const Decision r = decide_from_row(job, S.counts, A.limit, row, load_labs(job, row), up, left,
-                                           nb, false, true, lane);
+                                           nb, true, lane);
         w = r.w;
         if (r.reset) {
             ++st.resets;
             st.ban += r.stage == 1;
             st.near += r.stage == 2;
+            if (job.stage && lane == 0) gstore(job.stage, c, (uint8_t)r.stage);
             *reset = true;
         }
     }
@@ -1172,9 +1169,8 @@ __device__ __forceinline__ ChainStats chain_wave(const PlaceJob& job, const Chai
 
 // kRasterPlain: one cell at a time from the whole row, the row above in
 // S.ring.  For grids of one or two columns, where the lists would be prepared
-// after their cells are decided, for runs that want every cell's stage,
-// distance or score, and for libraries whose counts leave LDS no place for
-// lists.  Bound by the latency of a scored row; the next cell's Labs and
+// after their cells are decided, and for libraries whose counts leave LDS no
+// place for lists.  Bound by the latency of a scored row; the next cell's Labs and
 // the rows of the four after this one are in flight meanwhile (four cells an
 // iteration and no branch around the loads, so that the compiler's waits are
 // for the Labs alone: cells past the grid are evaluated and dropped).
@@ -1182,11 +1178,8 @@ __device__ __forceinline__ ChainStats raster_plain(const PlaceJob& job, const Ch
     constexpr int kRows = 4;
     ChainStats st{0, 0, 0};
     const ChainArgs A = chain_args(job);
-    const bool outputs = job.stage || job.dist || job.score;
     Neighbours nb{};
     uint32_t w = 0, won = 0;
-    int32_t stage = 0;
-    float dist = 0.0f, score = 0.0f;
     RawRow row[kRows];
     RowLabs labs[2];
     float4 lab_up[2] = {nb.up, nb.up};
@@ -1209,7 +1202,7 @@ __device__ __forceinline__ ChainStats raster_plain(const PlaceJob& job, const Ch
             nb.has_left = left != 0u;
             nb.up = select4(A.gw == 1, nb.left, lab_up[k & 1]);  // (one column: the previous winner)
             const Decision r = decide_from_row(job, S.counts, valid ? A.limit : kGuard, cur,
-                                               labs[k & 1], up, left, nb, outputs, valid, lane);
+                                               labs[k & 1], up, left, nb, valid, lane);
             w = r.w;
             const float4 lab = select4(r.rank < 64, labs[k & 1].l0, labs[k & 1].l1);
             const int32_t from = r.rank & 63;
@@ -1222,25 +1215,16 @@ __device__ __forceinline__ ChainStats raster_plain(const PlaceJob& job, const Ch
                 if (lane == 0) {
                     S.counts[w >> 2] += A.use;
                     S.ring[x] = w;
+                    if (r.reset && job.stage) gstore(job.stage, c, (uint8_t)r.stage);
                 }
             }
             asm volatile("" ::: "memory");
             x = x1;
-            // results wait one per lane for a store of 64 cells
-            const bool mine = lane == (c & 63);
-            won = mine ? w : won;
-            stage = mine ? r.stage : stage;
-            dist = mine ? r.dist : dist;
-            score = mine ? r.score : score;
+            won = lane == (c & 63) ? w : won;  // (stored 64 cells at a time)
         });
         if ((c4 & 63) == 64 - kRows || c4 + kRows >= A.cells) {
             const int32_t i = (c4 & ~63) + lane;
-            if (i < A.cells && i < c4 + kRows) {
-                gstore(job.grid, i, entry_material(won));
-                if (job.stage) gstore(job.stage, i, (uint8_t)stage);
-                if (job.dist) gstore(job.dist, i, dist);
-                if (job.score) gstore(job.score, i, score);
-            }
+            if (i < A.cells && i < c4 + kRows) gstore(job.grid, i, entry_material(won));
         }
     }
     return st;
@@ -1280,6 +1264,9 @@ __global__ __launch_bounds__(kChainThreads) void place_raster_kernel(
     for (int32_t i = tid; i < S.ring_n; i += kChainThreads) S.ring[i] = 0u;
     if (tid < kEvents) S.events[tid] = 0u;
     if (tid == 0) S.counts[0] = kGuard;
+    // every cell's stage is 0 but for those whose decision resets the counts
+    if (job.stage)
+        for (int32_t i = tid; i < cells; i += kChainThreads) gstore(job.stage, i, (uint8_t)0);
     __syncthreads();
 
     if (wave == 0) {
@@ -1312,6 +1299,44 @@ __global__ __launch_bounds__(kChainThreads) void place_raster_kernel(
         gstore(job.usage, i, S.counts[1 + i] >> (packed ? 16 : 0));
 }
 
+// What a raster run's cells won with, from the grid it left (and, for the
+// scores, its stages): a cell's up and left neighbours are those it was
+// decided against.  A wave to a cell, which finds the winner in its row.  The
+// chain itself keeps only the stages of resets: with distances and scores it
+// would score every cell (80 x 60 cells: 4.2 ms, the chain 0.27).
+__global__ __launch_bounds__(256) void place_outputs_kernel(PlaceJob job) {
+    const int lane = threadIdx.x & 63;
+    const int32_t c = __builtin_amdgcn_readfirstlane((int32_t)(blockIdx.x * 4 + (threadIdx.x >> 6)));
+    const int32_t gw = job.grid_w, cells = gw * job.grid_h;
+    if (c >= cells) return;
+    const RawRow row = load_row(job, c, cells, lane);
+    const int32_t x = c % gw, m = gload(job.grid, c);
+    const bool second = (int32_t)(uint32_t)row.r1 == m;
+    const uint64_t at = wave_ballot((int32_t)(uint32_t)row.r0 == m || second);
+    if (!at) return;  // (a placed tile is on its cell's row)
+    const float d = readlane_f(__uint_as_float((uint32_t)((second ? row.r1 : row.r0) >> 32)),
+                               __ffsll((unsigned long long)at) - 1);
+    if (lane != 0) return;
+    if (job.dist) gstore(job.dist, c, d);
+    if (!job.score) return;
+    float score = d;
+    if (job.weight > 0.0f && gload(job.stage, c) == 0) {
+        Neighbours nb{};
+        nb.has_up = c >= gw;
+        nb.has_left = x > 0;
+        if (nb.has_up) nb.up = load_lab(job, gload(job.grid, c - gw));
+        if (nb.has_left) nb.left = load_lab(job, gload(job.grid, c - 1));
+        score = exact_score(d, load_lab(job, m), nb, job.weight);
+    }
+    gstore(job.score, c, score);
+}
+
+void launch_place_outputs(const PlaceJob& job, hipStream_t stream) {
+    if (job.n <= 0 || !(job.dist || job.score)) return;
+    hipLaunchKernelGGL(place_outputs_kernel, dim3((job.grid_w * job.grid_h + 3) / 4), dim3(256), 0,
+                       stream, job);
+}
+
 size_t place_lds_bytes(int32_t cells, int32_t n) {
     return sizeof(int32_t) * ((size_t)cells + (size_t)n);
 }
@@ -1334,8 +1359,8 @@ size_t place_raster_lds_bytes(int32_t grid_w, int32_t n, int32_t form) {
 bool lists_taken(int32_t n, size_t max_lds) {
     return place_raster_lds_bytes(kLeastRingColumns, n, kRasterLists) <= max_lds;
 }
-int32_t raster_form(int32_t grid_w, int32_t n, bool outputs, bool labs, bool terms, size_t max_lds) {
-    const bool plain = grid_w < 3 || outputs || !terms;
+int32_t raster_form(int32_t grid_w, int32_t n, bool labs, bool terms, size_t max_lds) {
+    const bool plain = grid_w < 3 || !terms;
     for (int32_t form = plain ? kRasterPlain : labs ? kRasterLabs : kRasterLists; form >= 0; --form)
         if (place_raster_lds_bytes(grid_w, n, form) <= max_lds) return form;
     return -1;

@@ -217,9 +217,7 @@ int run_place(mh_context* ctx, const mh_library* lib, const float* d_cell_lab, i
               uint8_t* d_stage, float* d_dist, float* d_score, int32_t* d_stats,
               CandRec* cand_buf = nullptr) {
     const int32_t cells = gw * gh;
-    const int32_t form = raster ? raster_form(gw, lib->n, d_stage || d_dist || d_score, true,
-                                                   lib->has_terms, ctx->max_lds)
-                                     : -1;
+    const int32_t form = raster ? raster_form(gw, lib->n, true, lib->has_terms, ctx->max_lds) : -1;
     size_t lds =
         form >= 0 ? place_raster_lds_bytes(gw, lib->n, form) : place_lds_bytes(cells, lib->n);
     // state beyond LDS: the general chain with grid and counts in HBM (it
@@ -257,6 +255,7 @@ int run_place(mh_context* ctx, const mh_library* lib, const float* d_cell_lab, i
     job.stats = d_stats;
     phase_begin(ctx, MH_PHASE_PLACE);
     launch_place_single(job, raster && !hbm, lds, ctx->stream);
+    if (raster && !hbm) launch_place_outputs(job, ctx->stream);
     phase_end(ctx, MH_PHASE_PLACE);
     HIPCHK(hipGetLastError());
     return MH_OK;
@@ -1241,6 +1240,8 @@ int mh_place(mh_context* ctx, const mh_library* lib, const float* cell_lab,
     float *d_dist = nullptr, *d_score = nullptr;
     if (stage) {
         CHK(upload(ctx, S_OUT0, stage, (size_t)cells, &d_stage));
+    } else if (score) {  // (scores are made from the stages)
+        CHK(slot(ctx, S_OUT0, (size_t)cells, &d_stage));
     }
     if (dist) CHK(upload(ctx, S_OUT1, dist, (size_t)cells, &d_dist));
     if (score) CHK(upload(ctx, S_OUT2, score, (size_t)cells, &d_score));

@@ -89,7 +89,7 @@ int check_job(const mh_context* ctx, const mh_job& j, JobSpec* s) {
     s->strength = k < 0.0f ? 0.0f : (k > 1.0f ? 1.0f : k);  // src/main.rs:162
     s->adjust = s->strength > 0.0f;
     // placement state beyond LDS runs the chain with grid and counts in HBM
-    s->place_hbm = raster_form(s->gw, s->n, false, false, j.lib->has_terms, ctx->max_lds) < 0;
+    s->place_hbm = raster_form(s->gw, s->n, false, j.lib->has_terms, ctx->max_lds) < 0;
     s->anneal_kind = s->sa ? anneal_kind(s->cells, s->n, s->gw, s->gh, ctx->max_lds) : 0;
     if (s->anneal_kind < 0)
         return fail(MH_ERR_UNSUPPORTED, "annealing a %d x %d grid: a side of 65,536 or more", s->gw,
@@ -266,7 +266,7 @@ int build_plan(const std::vector<JobSpec>& specs, const std::vector<uint8_t*>& j
         pj.grid = grid;
         pj.usage = at<uint32_t>(m, s.o_usage);
         pj.zero_usage = 1;
-        pj.form = raster_form(s.gw, s.n, false, labs, lib->has_terms, lib->ctx->max_lds);
+        pj.form = raster_form(s.gw, s.n, labs, lib->has_terms, lib->ctx->max_lds);
         pj.grid_w = s.gw;
         pj.grid_h = s.gh;
         pj.max_usage = j.params.max_usage;

@@ -175,17 +175,20 @@ size_t place_lds_bytes(int32_t cells, int32_t n);
 // also the prepared candidate lists (kRasterLists), also the material Labs
 // (kRasterLabs; read from memory otherwise).  raster_form: the first of
 // kRasterLabs (if labs), kRasterLists, kRasterPlain that fits max_lds bytes,
-// the grid, the run (outputs: it wants every cell's stage, distance or score)
-// and the library (terms: lab4 holds its largest terms), -1 if none does.
+// the grid and the library (terms: lab4 holds its largest terms), -1 if none
+// does.
 // lists_taken: whether any grid's run takes a library of n materials in lists,
 // so that it needs its terms.
 constexpr int32_t kRasterPlain = 0, kRasterLists = 1, kRasterLabs = 2;
-int32_t raster_form(int32_t grid_w, int32_t n, bool outputs, bool labs, bool terms, size_t max_lds);
+int32_t raster_form(int32_t grid_w, int32_t n, bool labs, bool terms, size_t max_lds);
 bool lists_taken(int32_t n, size_t max_lds);
 size_t place_raster_lds_bytes(int32_t grid_w, int32_t n, int32_t form);
 // One job passed by value (kernel argument), or n_jobs jobs from a device
 // array; lds_bytes 0 (general chain): grid and counts in the job's buffers.
 void launch_place_single(const PlaceJob& job, bool raster, size_t lds_bytes, hipStream_t stream);
+// The distances and scores of a raster chain's run, after it (its stages too
+// are written if scores are wanted).  The general chain writes its own.
+void launch_place_outputs(const PlaceJob& job, hipStream_t stream);
 void launch_place_batch(const PlaceJob* d_jobs, int32_t n_jobs, bool raster, size_t lds_bytes,
                         hipStream_t stream);
 // Annealing variants: the grid in LDS with 16-bit material ids (libraries

@@ -20,8 +20,8 @@ PLAIN, LISTS = 0, 1
 
 def _rules(mh):
     lib = ctypes.CDLL(mh.LIB_PATH)
-    form = lib._ZN2mh11raster_formEiibbbm  # (grid_w, n, outputs, labs, terms, max_lds)
-    form.argtypes = [ctypes.c_int32, ctypes.c_int32] + [ctypes.c_bool] * 3 + [ctypes.c_size_t]
+    form = lib._ZN2mh11raster_formEiibbm   # (grid_w, n, labs, terms, max_lds)
+    form.argtypes = [ctypes.c_int32, ctypes.c_int32] + [ctypes.c_bool] * 2 + [ctypes.c_size_t]
     takes = lib._ZN2mh11lists_takenEim     # (n, max_lds)
     takes.restype = ctypes.c_bool
     takes.argtypes = [ctypes.c_int32, ctypes.c_size_t]
@@ -37,10 +37,10 @@ def test_lists_only_with_terms(mh):
         for gw in list(range(1, 140)) + [200, 500, 1000, 4000]:
             for labs in (False, True):
                 # whatever the library has, a run without terms is not on lists
-                assert form(gw, n, False, labs, False, LDS) < LISTS
+                assert form(gw, n, labs, False, LDS) < LISTS
                 # and where lists fit, the library has the terms
                 fits = gw >= 3 and words(gw, n, LISTS) <= LDS
-                assert (form(gw, n, False, labs, has, LDS) >= LISTS) == fits, (gw, n)
+                assert (form(gw, n, labs, has, LDS) >= LISTS) == fits, (gw, n)
 
 
 CASES = [
