@@ -717,8 +717,10 @@ __device__ __forceinline__ RowLabs load_labs(const PlaceJob& job, const RawRow& 
 }
 
 // The evaluation of a cell from its whole row, and the usage-reset fallback
-// (src/main.rs:385-475).  Estimates rule out all but the few candidates that
-// can win; when those are several, exact scores decide.
+// (src/main.rs:385-475).  The first candidate wins at once if the others lie
+// beyond the largest score it can have (two terms of at most 1); else
+// estimates rule out all but the few that can win, and when those are
+// several, exact scores decide.
 __device__ __forceinline__ Decision decide_from_row(const PlaceJob& job, uint32_t* counts,
                                                     uint32_t limit, const RawRow& row,
                                                     const RowLabs& labs, uint32_t up, uint32_t left,
@@ -738,15 +740,19 @@ __device__ __forceinline__ Decision decide_from_row(const PlaceJob& job, uint32_
     r.stage = 0;
     r.reset = false;
     if (b0 | b1) {
-        // keys: the scores' bits (no score is negative)
-        uint32_t k0 = lane_in(b0) ? __float_as_uint(d0) : kNone;
-        uint32_t k1 = lane_in(b1) ? __float_as_uint(d1) : kNone;
-        bool alone = false;
-        if (job.weight > 0.0f) {  // (otherwise the scores are the distances)
+        // (without a penalty the scores are the distances, which ascend)
+        const float first = b0 ? readlane_f(d0, __ffsll((unsigned long long)b0) - 1)
+                               : readlane_f(d1, __ffsll((unsigned long long)b1) - 1);
+        const float reach = first + (job.weight > 0.0f ? 2.0f * job.weight : 0.0f);
+        b0 &= wave_ballot(!(d0 > reach));
+        b1 &= wave_ballot(!(d1 > reach));
+        bool alone = __popcll(b0) + __popcll(b1) == 1;
+        if (!alone && job.weight > 0.0f) {
             const float e0 = score_estimate(d0, labs.l0, nb, job.weight);
             const float e1 = score_estimate(d1, labs.l1, nb, job.weight);
-            k0 = lane_in(b0) ? __float_as_uint(e0) : kNone;
-            k1 = lane_in(b1) ? __float_as_uint(e1) : kNone;
+            // keys: the scores' bits (no score is negative)
+            const uint32_t k0 = lane_in(b0) ? __float_as_uint(e0) : kNone;
+            const uint32_t k1 = lane_in(b1) ? __float_as_uint(e1) : kNone;
             const float far = rival_bound(__uint_as_float(wave_min_u32(k0 < k1 ? k0 : k1)), job.weight);
             b0 &= wave_ballot(!(e0 > far));
             b1 &= wave_ballot(!(e1 > far));
@@ -757,12 +763,10 @@ __device__ __forceinline__ Decision decide_from_row(const PlaceJob& job, uint32_
             const bool second = lane_in(b1 & ~b0);
             const float s =
                 exact_score(second ? d1 : d0, select4(second, labs.l1, labs.l0), nb, job.weight);
-            k0 = lane_in(b0) ? __float_as_uint(s) : kNone;
-            k1 = second ? __float_as_uint(s) : kNone;
+            const uint32_t k0 = lane_in(b0) ? __float_as_uint(s) : kNone;
+            uint32_t k1 = second ? __float_as_uint(s) : kNone;
             if (b0 & b1)
                 k1 = lane_in(b1) ? __float_as_uint(exact_score(d1, labs.l1, nb, job.weight)) : kNone;
-        }
-        if (!alone) {
             const uint32_t score = wave_min_u32(k0 < k1 ? k0 : k1);
             b0 &= wave_ballot(k0 == score);
             b1 &= wave_ballot(k1 == score);
@@ -1173,7 +1177,12 @@ __device__ __forceinline__ ChainStats chain_wave(const PlaceJob& job, const Chai
 // place for lists.  Bound by the latency of a scored row; the next cell's Labs and
 // the rows of the four after this one are in flight meanwhile (four cells an
 // iteration and no branch around the loads, so that the compiler's waits are
-// for the Labs alone: cells past the grid are evaluated and dropped).
+// for the Labs alone: cells past the grid are evaluated and dropped; one column
+// is compiled by itself, as a choice of the up neighbour's Lab at run time
+// waits for it a cell early).  Every candidate scored 0.67 us a cell of 36,000
+// materials, the first alone where it can be 0.57, without that wait 0.56; GUI
+// score 0.69, 0.65, 0.62.
+template <bool kOneColumn>
 __device__ __forceinline__ ChainStats raster_plain(const PlaceJob& job, const ChainShared& S, int lane) {
     constexpr int kRows = 4;
     ChainStats st{0, 0, 0};
@@ -1200,7 +1209,7 @@ __device__ __forceinline__ ChainStats raster_plain(const PlaceJob& job, const Ch
             row[k] = load_row(job, c + kRows, A.cells, lane);
             nb.has_up = up != 0u;
             nb.has_left = left != 0u;
-            nb.up = select4(A.gw == 1, nb.left, lab_up[k & 1]);  // (one column: the previous winner)
+            nb.up = kOneColumn ? nb.left : lab_up[k & 1];  // (one column: the previous winner)
             const Decision r = decide_from_row(job, S.counts, valid ? A.limit : kGuard, cur,
                                                labs[k & 1], up, left, nb, valid, lane);
             w = r.w;
@@ -1258,9 +1267,10 @@ __global__ __launch_bounds__(kChainThreads) void place_raster_kernel(
     if (S.labs)
         for (int32_t i = tid; i < n; i += kChainThreads) S.labs[i] = gload4(job.lab4, i);
     const bool packed = packs(job);
+    const bool terms = packed && job.form != kRasterPlain;
     for (int32_t i = tid; i < n; i += kChainThreads)
-        S.counts[1 + i] = packed ? bf16_up(gload4(job.lab4, i).w) >> 16
-                                 : (job.zero_usage ? 0u : gload(job.usage, i));
+        S.counts[1 + i] = terms ? bf16_up(gload4(job.lab4, i).w) >> 16
+                                : (job.zero_usage ? 0u : gload(job.usage, i));
     for (int32_t i = tid; i < S.ring_n; i += kChainThreads) S.ring[i] = 0u;
     if (tid < kEvents) S.events[tid] = 0u;
     if (tid == 0) S.counts[0] = kGuard;
@@ -1271,8 +1281,10 @@ __global__ __launch_bounds__(kChainThreads) void place_raster_kernel(
 
     if (wave == 0) {
         ChainStats st;
-        if (job.form == kRasterPlain)
-            st = raster_plain(job, S, lane);
+        if (job.form == kRasterPlain && gw == 1)
+            st = raster_plain<true>(job, S, lane);
+        else if (job.form == kRasterPlain)
+            st = raster_plain<false>(job, S, lane);
         else if (gw < kUpPrepColumns)
             st = chain_wave<kUpChain>(job, S, lane);
         else
@@ -1350,8 +1362,8 @@ size_t place_raster_lds_bytes(int32_t grid_w, int32_t n, int32_t form) {
 // Where each form stands: the lists take 28 KB and 4 bytes a material (to
 // about 33,700 materials), the Labs 16 bytes a material more.  A flagged
 // cell's Labs come from LDS in 0.4 us, from memory in 0.7-1 us.  Without room
-// for the lists (33,700 to 40,700 materials) a cell costs 0.67 us plain; one
-// wave that read ahead in registers took 0.59 there.
+// for the lists (33,800 to 40,700 materials) a cell costs 0.56 us plain, as
+// one wave that read ahead in registers did.
 //
 // Without the materials' largest terms a list's entries would all look safe,
 // so such a library's runs are plain; lists_taken says which libraries need
