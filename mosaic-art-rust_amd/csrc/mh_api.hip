@@ -424,7 +424,7 @@ int upload(mh_context* ctx, Slot s, const T* host, size_t count, T** dev) {
     int rc = slot(ctx, s, count, dev);
     if (rc) return rc;
     const size_t bytes = sizeof(T) * count;
-    if (staged(host, bytes))
+    if (staged_up(host, bytes))
         return stage_upload(ctx, reinterpret_cast<uint8_t*>(*dev),
                             {HostSpan{reinterpret_cast<const uint8_t*>(host), bytes}});
     if (count) HIPCHK(hipMemcpyAsync(*dev, host, bytes, hipMemcpyHostToDevice, ctx->stream));
@@ -434,7 +434,7 @@ int upload(mh_context* ctx, Slot s, const T* host, size_t count, T** dev) {
 template <typename T>
 int download(mh_context* ctx, T* host, const T* dev, size_t count) {
     const size_t bytes = sizeof(T) * count;
-    if (host && staged(host, bytes))
+    if (host && staged_down(host, bytes))
         return stage_download(ctx, reinterpret_cast<uint8_t*>(host),
                               reinterpret_cast<const uint8_t*>(dev), bytes);
     if (host && count) HIPCHK(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, ctx->stream));
@@ -889,7 +889,7 @@ int mh_library_from_pixels(mh_context* ctx, const uint8_t* rgb, int32_t n, int32
     int rc = MH_OK;
     hipError_t e = hipMalloc(&lib->d_pixels, bytes ? bytes : 16);
     if (e == hipSuccess && bytes) {
-        if (staged(rgb, bytes))
+        if (staged_up(rgb, bytes))
             rc = stage_upload(ctx, lib->d_pixels, {HostSpan{rgb, bytes}});
         else
             e = hipMemcpyAsync(lib->d_pixels, rgb, bytes, hipMemcpyHostToDevice, ctx->stream);

@@ -169,8 +169,10 @@ int set_device(mh_context* ctx);
 void phase_begin(mh_context* ctx, int phase);
 void phase_end(mh_context* ctx, int phase);
 int ensure(mh_context* ctx, DevBuf& b, size_t bytes);
-// Whether a copy of pageable host memory goes through the pinned buffers.
-bool staged(const void* host, size_t bytes);
+// Whether a copy of pageable host memory to or from the device goes through
+// the pinned buffers.
+bool staged_up(const void* host, size_t bytes);
+bool staged_down(const void* host, size_t bytes);
 // The spans, back to back, to dst: queued on the stream, the spans read.
 int stage_upload(mh_context* ctx, uint8_t* dst, const std::vector<HostSpan>& spans);
 // After everything queued on the stream: copied, host written.

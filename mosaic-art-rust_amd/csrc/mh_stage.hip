@@ -10,6 +10,16 @@
 // arrays 15.0 -> 2.8 ms, of which 1.2 are the caller's list; 1,500 images of
 // one size (74 MB) 4.0 -> 2.5 ms.  Three threads with 4 MiB buffers: 2.4 ms
 // for those 74 MB; 1 MiB buffers 3.0, 256 KiB 6.2; four or six threads the same.
+//
+// Starting the threads takes 30-60 us and the runtime keeps buffers it has
+// copied pinned, so one buffer is only staged from the size where that is no
+// slower even for a buffer copied again and again (us, runtime and staged):
+// up 6 MiB 228 and 318, 16 MiB 520 and 550, 24 MiB 750 and 750, 48 MiB 1,770
+// and 1,400 (buffers not seen before: equal at 12 MiB); down 4 MiB 226 and 240,
+// 6 MiB 341 and 290, 64 MiB 3,850 and 1,640.  Images to be gathered come
+// through here whatever they sum to, below kLeastShared on one thread: 0.8 MiB
+// 137 us (chunks of 512 KiB 161, three threads 175), 3.6 MiB 262 (282, 325), 4.8
+// MiB 300 (305, 340).
 #include <algorithm>
 #include <atomic>
 #include <cstring>
@@ -21,13 +31,15 @@ namespace mh {
 namespace host {
 
 namespace {
-constexpr size_t kBuffer = (size_t)4 << 20, kLeast = (size_t)1 << 20;
+constexpr size_t kBuffer = (size_t)4 << 20, kLeastChunk = (size_t)1 << 20;
+constexpr size_t kLeastUp = (size_t)24 << 20, kLeastDown = (size_t)6 << 20,
+                 kLeastShared = (size_t)5 << 20;
 
 // Bytes a buffer is filled with at a time: two rounds a thread for a copy of
 // a few MB, whole buffers for a large one (a copy costs 10 us by itself).
 size_t chunk_of(size_t total) {
     const size_t share = (total / (2 * kStageThreads) + 0xffff) & ~(size_t)0xffff;
-    return std::min(kBuffer, std::max(kLeast / 2, share));
+    return std::min(kBuffer, std::max(kLeastChunk, share));
 }
 
 int stage_ready(StageBuf& b) {
@@ -36,15 +48,15 @@ int stage_ready(StageBuf& b) {
     return MH_OK;
 }
 
-// f(thread) on kStageThreads threads, this one among them, and the first
-// error of any of them.  A thread that cannot be started is done without:
-// the threads share the chunks.
+// f(thread) on kStageThreads threads, this one among them (on this one alone
+// below kLeastShared bytes), and the first error of any of them.  A thread
+// that cannot be started is done without: the threads share the chunks.
 template <typename F>
-int on_threads(mh_context* ctx, size_t chunks, F&& f) {
+int on_threads(mh_context* ctx, size_t total, size_t chunks, F&& f) {
     int rc[kStageThreads] = {};
     std::string text[kStageThreads];
     std::thread helpers[kStageThreads];
-    for (int t = 1; t < kStageThreads && (size_t)t < chunks; ++t) {
+    for (int t = 1; t < kStageThreads && (size_t)t < chunks && total >= kLeastShared; ++t) {
         try {
             helpers[t] = std::thread([&, t]() {
                 rc[t] = set_device(ctx);
@@ -75,7 +87,12 @@ bool known_to_runtime(const void* p) {
 }
 }  // namespace
 
-bool staged(const void* host, size_t bytes) { return bytes >= kLeast && !known_to_runtime(host); }
+bool staged_up(const void* host, size_t bytes) {
+    return bytes >= kLeastUp && !known_to_runtime(host);
+}
+bool staged_down(const void* host, size_t bytes) {
+    return bytes >= kLeastDown && !known_to_runtime(host);
+}
 
 int stage_upload(mh_context* ctx, uint8_t* dst, const std::vector<HostSpan>& spans) {
     std::vector<size_t> at(spans.size() + 1, 0);  // where each span goes
@@ -83,7 +100,7 @@ int stage_upload(mh_context* ctx, uint8_t* dst, const std::vector<HostSpan>& spa
     const size_t total = at.back(), chunk = chunk_of(total), chunks = (total + chunk - 1) / chunk;
     std::lock_guard<std::mutex> g(ctx->stage_mu);
     std::atomic<size_t> next{0};
-    const int rc = on_threads(ctx, chunks, [&](int t) -> int {
+    const int rc = on_threads(ctx, total, chunks, [&](int t) -> int {
         for (int k = 0;; k ^= 1) {
             const size_t c = next.fetch_add(1);
             if (c >= chunks) return MH_OK;
@@ -116,7 +133,7 @@ int stage_download(mh_context* ctx, uint8_t* host, const uint8_t* src, size_t to
     const size_t chunk = chunk_of(total), chunks = (total + chunk - 1) / chunk;
     std::lock_guard<std::mutex> g(ctx->stage_mu);
     std::atomic<size_t> next{0};
-    const int rc = on_threads(ctx, chunks, [&](int t) -> int {
+    const int rc = on_threads(ctx, total, chunks, [&](int t) -> int {
         size_t mine[2];
         bool busy[2] = {false, false};
         for (int k = 0;; k ^= 1) {
