@@ -523,14 +523,25 @@ class Context:
         return Server(self, memory_budget, max_batch, streams)
 
 
+# An array's address costs 0.4 us to ask for, a copy of its bytes 0.1 us a KiB
+# (1,000 images: 768 B 730 us by address and 459 copied, 6.8 KiB 1,010 and 975,
+# 12 KiB 1,163 and 1,247).
+_COPY_BELOW = 8192
+
+
 def _image_table(images):
-    """RGB8 images where they lie: (arrays, base address, offsets from it, widths, heights).
-    The arrays must outlive the call that gets the table."""
+    """RGB8 images: (arrays, base address, offsets from it, widths, heights), images of less
+    than _COPY_BELOW bytes on average copied into one array, else where they lie.  The arrays
+    must outlive the call that gets the table."""
     arrs = [_c(im, np.uint8) for im in images]
-    at = np.array([a.__array_interface__["data"][0] for a in arrs], np.int64)
-    base = int(at.min()) if arrs else 0
     h = np.array([a.shape[0] for a in arrs], np.int32)
     w = np.array([a.shape[1] for a in arrs], np.int32)
+    sizes = np.array([a.size for a in arrs], np.int64)
+    if sizes.sum() < _COPY_BELOW * len(arrs):
+        buf = np.concatenate([a.reshape(-1) for a in arrs])
+        return buf, _ptr(buf), np.cumsum(sizes) - sizes, w, h
+    at = np.array([a.__array_interface__["data"][0] for a in arrs], np.int64)
+    base = int(at.min()) if arrs else 0
     return arrs, ctypes.c_void_p(base), at - base, w, h
 
 
