@@ -40,7 +40,8 @@ struct LabShared {
 //   rgb + (c / per_row) * block_row_stride + (c % per_row) * block_col_stride
 //       + py * row_stride + px * 3.
 // Pixel index -> (px, py) by umulhi with cw_magic = floor((2^32 - 1) / cw) + 1,
-// exact while pix * cw < 2^32 (pix < cw * ch), else by division.
+// exact while pix * cw < 2^32 (pix < cw * ch) and for cw > 1 (for 1 it would be
+// 2^32), else by division.
 template <int kCells, bool kOff32>
 __device__ __forceinline__ void cell_lab_block(const CellSeg& s, int32_t blk,
                                                const float* __restrict__ lut_g, LabShared& sh) {
@@ -56,7 +57,7 @@ __device__ __forceinline__ void cell_lab_block(const CellSeg& s, int32_t blk,
     const int32_t cw = s.cw, ch = s.ch, n_cells = s.n_cells, per_row = s.per_row;
     const int32_t npx = cw * ch;
     const uint32_t cw_magic = 0xffffffffu / (uint32_t)cw + 1u;
-    const bool magic_ok = (uint64_t)(uint32_t)npx * (uint32_t)cw < (1ull << 32);
+    const bool magic_ok = cw > 1 && (uint64_t)(uint32_t)npx * (uint32_t)cw < (1ull << 32);
     const uint32_t rs32 = (uint32_t)s.row_stride;
     // summing lane -> (cell, channel)
     const int sum_cell = tid / 3, sum_ch = tid % 3;
