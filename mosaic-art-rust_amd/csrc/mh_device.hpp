@@ -466,9 +466,9 @@ __device__ __forceinline__ float fmod_360(float a) {
 // product s * adj.w may be -0 (adj.w = -0) and keeps the general clamp.
 //
 // The HSV hue and saturation step, and the conversion back to u8, are
-// adjust_tail for one pixel in general form, and adjust_four for four pixels
-// of one adjustment in the kUnit form: without branches but for one around the
-// step, so that the four pixels' instructions fill each other's waits.
+// adjust_tail for one pixel in general form, and adjust_quad for up to four
+// pixels of one adjustment in the kUnit form: without branches but for one
+// around the step, so that the pixels' instructions fill each other's waits.
 __device__ __forceinline__ void adjust_tail(float4 adj, float br, float bg, float bb,
                                             uint32_t& ro, uint32_t& go, uint32_t& bo) {
     if (adj.z != 0.0f || adj.w != 1.0f) {
@@ -486,13 +486,14 @@ __device__ __forceinline__ void adjust_tail(float4 adj, float br, float bg, floa
 
 // (s * adj.w may be -0 where the general form keeps the sign: c = v s is then
 // -0, x too, m = v - c = v, and every sum with m >= +0 the same as with +0.)
-__device__ __forceinline__ void adjust_four(float4 adj, float (&r)[4], float (&g)[4], float (&b)[4],
-                                            uint32_t (&out)[12]) {
+template <int N>
+__device__ __forceinline__ void adjust_quad(float4 adj, float (&r)[N], float (&g)[N], float (&b)[N],
+                                            uint32_t (&out)[3 * N]) {
     if (adj.z != 0.0f || adj.w != 1.0f) {
-        float h[4], s[4], v[4];
+        float h[N], s[N], v[N];
         bool tiny = false;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < N; ++i) {
             rgb_to_hsv<true>(r[i], g[i], b[i], h[i], s[i], v[i]);
             // rem_euclid(360.0) of a value in [-240, 480] (fmodf's remainder is
             // a - 360, exact, from 360 on, else a itself)
@@ -502,14 +503,14 @@ __device__ __forceinline__ void adjust_four(float4 adj, float (&r)[4], float (&g
             tiny = tiny || tiny_hue(h[i]);
         }
         if (__builtin_expect(tiny, 0)) {
-            for (int i = 0; i < 4; ++i) hsv_to_rgb(h[i], s[i], v[i], r[i], g[i], b[i]);
+            for (int i = 0; i < N; ++i) hsv_to_rgb(h[i], s[i], v[i], r[i], g[i], b[i]);
         } else {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) hsv_to_rgb<true>(h[i], s[i], v[i], r[i], g[i], b[i]);
+            for (int i = 0; i < N; ++i) hsv_to_rgb<true>(h[i], s[i], v[i], r[i], g[i], b[i]);
         }
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < N; ++i) {
         out[3 * i] = to_u8<true>(r[i]);
         out[3 * i + 1] = to_u8<true>(g[i]);
         out[3 * i + 2] = to_u8<true>(b[i]);
