@@ -394,28 +394,35 @@ __device__ __forceinline__ void topk_run(const TopkSeg& s, int32_t q0, int32_t r
         sort_buffer(buf, count);
         // answer: the first k keys, ascending
         const int32_t out_stride = s.out_stride;
-        for (int32_t r = lane; r < out_stride; r += 64) {
-            const int64_t o = (int64_t)q * out_stride + r;
-            if (r < k) {
-                const uint64_t key = buf[r];
-                const int32_t m = (int32_t)(uint32_t)(key & 0xffffffffu);
-                prev[r] = m;
-                if (s.out_idx) gstore(s.out_idx, o, m);
-                if (s.out_d) gstore(s.out_d, o, __uint_as_float((uint32_t)(key >> 32)));
-                // the key is {m, d} as one little-endian word: m in the low
-                // half (CandRec::m, offset 0), the distance bits in the high;
-                // the GUI score's rows hold the distance itself (sqrt is
-                // monotone, so the order stands)
-                if (s.out_cand) {
-                    const float d = __uint_as_float((uint32_t)(key >> 32));
-                    gstore((uint64_t*)s.out_cand, o,
-                           s.root ? make_key(__float_as_uint(sqrtf(d)), m) : key);
+        auto write = [&](auto root) __attribute__((always_inline)) {
+            for (int32_t r = lane; r < out_stride; r += 64) {
+                const int64_t o = (int64_t)q * out_stride + r;
+                if (r < k) {
+                    const uint64_t key = buf[r];
+                    const int32_t m = (int32_t)(uint32_t)(key & 0xffffffffu);
+                    prev[r] = m;
+                    if (s.out_idx) gstore(s.out_idx, o, m);
+                    if (s.out_d) gstore(s.out_d, o, __uint_as_float((uint32_t)(key >> 32)));
+                    // the key is {m, d} as one little-endian word: m in the low
+                    // half (CandRec::m, offset 0), the distance bits in the high;
+                    // the GUI score's rows hold the distance itself (sqrt is
+                    // monotone, so the order stands)
+                    if (s.out_cand) {
+                        const float d = __uint_as_float((uint32_t)(key >> 32));
+                        gstore((uint64_t*)s.out_cand, o,
+                               root.value ? make_key(__float_as_uint(sqrtf(d)), m) : key);
+                    }
+                } else if (s.out_cand) {
+                    // padded (chain) rows: ranks beyond k, -1 with an infinite distance
+                    gstore((uint64_t*)s.out_cand, o, (uint64_t)0x7f800000u << 32 | 0xffffffffu);
                 }
-            } else if (s.out_cand) {
-                // padded (chain) rows: ranks beyond k, -1 with an infinite distance
-                gstore((uint64_t*)s.out_cand, o, (uint64_t)0x7f800000u << 32 | 0xffffffffu);
             }
-        }
+        };
+        // (apart: as one loop the root is computed for every row and dropped)
+        if (s.root)
+            write(std::true_type{});
+        else
+            write(std::false_type{});
         __syncthreads();
     }
 }
