@@ -511,6 +511,24 @@ MatBlocks library_blocks(const mh_library* lib) {
     return MatBlocks{lib->d_pL, lib->d_pA, lib->d_pB, lib->d_pidx, lib->d_box, lib->nb};
 }
 
+// A library's tables in their one allocation, in bytes from its start: the Lab
+// table, the blocks' boxes, the Lab table's columns, the block layout's.  Each
+// begins on 256 bytes, a block's 64 values so on two cache lines (three, at
+// any other start).
+TableLayout table_layout(int32_t n) {
+    const size_t m = n > 0 ? (size_t)n : 1, nb = (m + 63) / 64, slots = nb * 64;
+    TableLayout t{};
+    auto place = [&](size_t* at, size_t bytes) {
+        *at = t.bytes;
+        t.bytes += (bytes + 255) & ~(size_t)255;
+    };
+    place(&t.lab4, sizeof(float4) * m);
+    place(&t.box, sizeof(float4) * 2 * nb);
+    for (size_t* column : {&t.L, &t.A, &t.B}) place(column, sizeof(float) * m);
+    for (size_t* column : {&t.pL, &t.pA, &t.pB, &t.pidx}) place(column, sizeof(float) * slots);
+    return t;
+}
+
 }  // namespace host
 }  // namespace mh
 
@@ -744,21 +762,19 @@ static int library_alloc(mh_context* ctx, int32_t n, mh_library** out) {
     }
     lib->n = n;
     lib->h_lab.assign((size_t)n * 3, 0.0f);
-    // one allocation: the Lab table, its three columns, and the block layout
-    // (library_upload_lab fills it the same way)
-    const size_t m = n > 0 ? (size_t)n : 1, nb = (m + 63) / 64, slots = nb * 64;
-    const size_t bytes = sizeof(float4) * (m + 2 * nb) + sizeof(float) * (3 * m + 4 * slots);
-    hipError_t e = hipMalloc(&lib->d_tables, bytes);
+    const TableLayout t = table_layout(n);
+    hipError_t e = hipMalloc(&lib->d_tables, t.bytes);
     if (e == hipSuccess) {
-        lib->d_lab4 = static_cast<float4*>(lib->d_tables);
-        lib->d_box = lib->d_lab4 + m;
-        lib->d_L = reinterpret_cast<float*>(lib->d_box + 2 * nb);
-        lib->d_A = lib->d_L + m;
-        lib->d_B = lib->d_A + m;
-        lib->d_pL = lib->d_B + m;
-        lib->d_pA = lib->d_pL + slots;
-        lib->d_pB = lib->d_pA + slots;
-        lib->d_pidx = reinterpret_cast<int32_t*>(lib->d_pB + slots);
+        uint8_t* base = static_cast<uint8_t*>(lib->d_tables);
+        lib->d_lab4 = reinterpret_cast<float4*>(base + t.lab4);
+        lib->d_box = reinterpret_cast<float4*>(base + t.box);
+        lib->d_L = reinterpret_cast<float*>(base + t.L);
+        lib->d_A = reinterpret_cast<float*>(base + t.A);
+        lib->d_B = reinterpret_cast<float*>(base + t.B);
+        lib->d_pL = reinterpret_cast<float*>(base + t.pL);
+        lib->d_pA = reinterpret_cast<float*>(base + t.pA);
+        lib->d_pB = reinterpret_cast<float*>(base + t.pB);
+        lib->d_pidx = reinterpret_cast<int32_t*>(base + t.pidx);
     } else {
         mh_library_destroy(lib);
         return fail(e == hipErrorOutOfMemory ? MH_ERR_OUT_OF_MEMORY : MH_ERR_HIP, "library alloc: %s",
@@ -832,13 +848,15 @@ static int library_upload_lab(mh_library* lib) {
     const int32_t n = lib->n;
     if (n == 0) return MH_OK;
     const size_t nb = ((size_t)n + 63) / 64, slots = nb * 64;
-    std::vector<uint8_t> tables(sizeof(float4) * ((size_t)n + 2 * nb) +
-                                sizeof(float) * (3 * (size_t)n + 4 * slots));
-    float4* l4 = reinterpret_cast<float4*>(tables.data());
-    float4* box = l4 + n;
-    float *L = reinterpret_cast<float*>(box + 2 * nb), *A = L + n, *B = A + n;
-    float *pl = B + n, *pa = pl + slots, *pb = pa + slots;
-    int32_t* pidx = reinterpret_cast<int32_t*>(pb + slots);
+    const TableLayout t = table_layout(n);
+    std::vector<uint8_t> tables(t.bytes);
+    uint8_t* const base = tables.data();
+    float4 *l4 = reinterpret_cast<float4*>(base + t.lab4), *box = reinterpret_cast<float4*>(base + t.box);
+    float *L = reinterpret_cast<float*>(base + t.L), *A = reinterpret_cast<float*>(base + t.A),
+          *B = reinterpret_cast<float*>(base + t.B);
+    float *pl = reinterpret_cast<float*>(base + t.pL), *pa = reinterpret_cast<float*>(base + t.pA),
+          *pb = reinterpret_cast<float*>(base + t.pB);
+    int32_t* pidx = reinterpret_cast<int32_t*>(base + t.pidx);
     for (int32_t i = 0; i < n; ++i) {
         L[i] = lib->h_lab[3 * i];
         A[i] = lib->h_lab[3 * i + 1];

@@ -169,6 +169,10 @@ int set_device(mh_context* ctx);
 void phase_begin(mh_context* ctx, int phase);
 void phase_end(mh_context* ctx, int phase);
 int ensure(mh_context* ctx, DevBuf& b, size_t bytes);
+struct TableLayout {
+    size_t lab4, box, L, A, B, pL, pA, pB, pidx, bytes;
+};
+TableLayout table_layout(int32_t n);
 // Whether a copy of pageable host memory to or from the device goes through
 // the pinned buffers.
 bool staged_up(const void* host, size_t bytes);
