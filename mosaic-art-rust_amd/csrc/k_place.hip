@@ -925,7 +925,9 @@ __device__ __forceinline__ void leave_cycle(const ChainShared& S, uint32_t event
 //
 // kUpChain: up and ban, further instructions that keep the last 64 winners in
 // hist (cell c's in lane c mod 64, m0 = c) and take c + 1's up neighbour out
-// of u for c + 1 (ban: the mask of its entries); 28 cycles more a step.
+// of u for c + 1 (ban: the mask of its entries); 28 cycles more a step.  m0 is
+// the compiler's (a reserved register, which a clobber list cannot name): it is
+// put back on the way out.
 //
 // Entered with slot = 12 at cell g0, or after a full evaluation of the cell
 // in `slot` at its commit; left at a flagged cell with everything landed.
@@ -959,6 +961,8 @@ __device__ __forceinline__ void leave_cycle(const ChainShared& S, uint32_t event
     "s_add_u32 m0, m0, 1\n"                                             \
     "s_sub_u32 %[up], m0, %[gw]\n"                                      \
     "v_readlane_b32 %[up], %[hist], %[up]\n"
+#define MH_TAKE_M0 "s_mov_b32 %[m0s], m0\ns_mov_b32 m0, %[cell]\n"
+#define MH_GIVE_M0 "s_mov_b32 m0, %[m0s]\n"
 #define MH_UP(B) "v_cmp_eq_u32_e64 %[ban], %[up], %[a" #B "]\n"
 #define MH_READ(Q, ROW, T) "ds_read_b128 " Q ", %[" #ROW "] offset:" #T "*1024\n"
 // A flagged cell (its entry is read again: the registers may hold a later
@@ -987,9 +991,9 @@ __device__ __forceinline__ void leave_cycle(const ChainShared& S, uint32_t event
     "s_branch L_adv" #I2 "_%=\n"
 
 // (cell, a of c, c + 1, c + 2, entries of c + 1, c + 2, their counts, w)
-#define MH_RUN(BAN, KEEP, UP)                                                                   \
+#define MH_RUN(BAN, KEEP, UP, TAKE, GIVE)                                                       \
     asm volatile(                                                                               \
-        "s_mov_b32 m0, %[cell]\n"                                                               \
+        TAKE                                                                                    \
         "s_cmp_eq_u32 %[slot], 12\n"                                                            \
         "v_cmp_eq_u32_e32 vcc, %[w1], %[a0]\n"                                                  \
         "s_cbranch_scc1 L_dec0_%=\n"                                                            \
@@ -1041,18 +1045,20 @@ __device__ __forceinline__ void leave_cycle(const ChainShared& S, uint32_t event
         MH_FLAGGED(6, 0, 2, 0, 1) MH_FLAGGED(7, 1, 2, 1, 0) MH_FLAGGED(8, 2, 2, 2, 1)           \
         MH_FLAGGED(9, 0, 3, 0, 0) MH_FLAGGED(10, 1, 3, 1, 1) MH_FLAGGED(11, 2, 3, 2, 0)         \
         "L_exit_%=:\n"                                                                          \
+        GIVE                                                                                    \
         "s_waitcnt lgkmcnt(0)\n"                                                                \
         : "+{v[64:67]}"(q0), "+{v[68:71]}"(q1), [a0] "+v"(a0), [a1] "+v"(a1), [a2] "+v"(a2),    \
           [c0] "+v"(c0), [c1] "+v"(c1), [wins] "+v"(wins), [rc] "+v"(rows_c),                   \
           [rn] "+v"(rows_n), [ring] "+v"(ring_w), [t] "=&v"(t), [u] "+s"(u), [fl] "+s"(fl),     \
           [w0] "+s"(w0), [w1] "+s"(w1), [wp] "=&s"(prev), [f] "=&s"(f),                         \
           [slot] "+s"(slot), [g0] "+s"(g0),                                                     \
-          [per] "+s"(period), [so] "+s"(so), [hist] "+v"(hist), [up] "=&s"(up), [ban] "+s"(ban) \
+          [per] "+s"(period), [so] "+s"(so), [hist] "+v"(hist), [up] "=&s"(up), [ban] "+s"(ban), \
+          [m0s] "=&s"(m0_saved)                                                                 \
         : [mul] "v"(mul), [port] "v"(port), [one] "v"(one), [row0] "v"(row0),                   \
           [lim] "s"(A.limit), [rend] "s"(ring_end), [rlen] "s"(ring_b),                         \
           [ids] "s"(kEntryId), [counts] "n"(kCountBytes), [slotb] "n"(kSlotBytes),              \
           [unsafe] "n"(kUnsafeBit), [cell] "s"(cell), [gw] "s"(A.gw)                            \
-        : "memory", "vcc", "scc", "m0")
+        : "memory", "vcc", "scc")
 
 template <int kUp>
 __device__ __forceinline__ ChainStats chain_wave(const PlaceJob& job, const ChainShared& S, int lane) {
@@ -1092,12 +1098,12 @@ __device__ __forceinline__ ChainStats chain_wave(const PlaceJob& job, const Chai
         int32_t slot = kGroup;
         bool restart = false;
         while (!restart) {
-            uint32_t t, prev, up;
+            uint32_t t, prev, up, m0_saved;
             int32_t f;
             if constexpr (kUp == kUpPrep)
-                MH_RUN("", MH_NO, MH_NO);
+                MH_RUN("", MH_NO, MH_NO, "", "");
             else
-                MH_RUN(MH_BAN, MH_KEEP, MH_UP);
+                MH_RUN(MH_BAN, MH_KEEP, MH_UP, MH_TAKE_M0, MH_GIVE_M0);
             slot = __builtin_amdgcn_readfirstlane(slot);
             f = __builtin_amdgcn_readfirstlane(f);  // the flagged entry
             g0 = __builtin_amdgcn_readfirstlane(g0);
@@ -1170,6 +1176,8 @@ __device__ __forceinline__ ChainStats chain_wave(const PlaceJob& job, const Chai
 #undef MH_BAN
 #undef MH_KEEP
 #undef MH_UP
+#undef MH_TAKE_M0
+#undef MH_GIVE_M0
 
 // kRasterPlain: one cell at a time from the whole row, the row above in
 // S.ring.  For grids of one or two columns, where the lists would be prepared
