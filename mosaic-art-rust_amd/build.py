@@ -1,5 +1,6 @@
 """Builds libmosaic_hip.so (gfx950) in-tree from csrc/*.hip, then the C++
-host API (host/mosaic.cpp) with its test program (test_mosaic).
+host API (host/mosaic.cpp) with its test program (test_mosaic) and the device
+code's own checks (device_test/, libmosaic_hip_test.so).
 
 Flags: -ffp-contract=off keeps the reference's unfused f32 arithmetic;
 packed FP32 instructions are disabled (-packed-fp32-ops target feature).
@@ -53,6 +54,7 @@ def build(verbose=False):
     if verbose:
         print(f"built {LIB}")
     build_host(verbose)
+    build_device_test(verbose)
     return LIB
 
 
@@ -72,6 +74,21 @@ def build_host(verbose=False):
     os.replace(HOST_TESTS + ".tmp", HOST_TESTS)
     if verbose:
         print(f"built {HOST_TESTS}")
+
+
+DEVICE_TEST = os.path.join(HERE, "libmosaic_hip_test.so")
+
+
+def build_device_test(verbose=False):
+    """Checks of the device code that need kernels of their own."""
+    cmd = [HIPCC, *HIPFLAGS, "-shared", os.path.join(HERE, "device_test", "identities.hip"), "-o",
+           DEVICE_TEST + ".tmp"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"device test build failed: {' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
+    os.replace(DEVICE_TEST + ".tmp", DEVICE_TEST)
+    if verbose:
+        print(f"built {DEVICE_TEST}")
 
 
 if __name__ == "__main__":

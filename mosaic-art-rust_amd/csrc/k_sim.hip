@@ -59,8 +59,8 @@ __global__ __launch_bounds__(256) void sim_packed_kernel(const float4* __restric
 
 // lab[i].w = the largest adjacency term of material i to another material
 // (0 where there is none): its penalty in any cell is at most twice that,
-// times the weight.  The largest term is that of the smallest distance (by the
-// same operations as adj_term, all monotone).  A block takes 256 materials
+// times the weight.  The largest term is that of the smallest distance, by
+// adj_term's own function, which is monotone.  A block takes 256 materials
 // against one of kNearParts parts of the library, so that the smallest
 // library it matters for fills the device; non-negative floats order like
 // their bits, so the parts meet in an integer maximum.  w starts at 0.  Once
@@ -86,8 +86,7 @@ __global__ __launch_bounds__(256) void near_term_kernel(float4* __restrict__ lab
         }
     }
     if (i < n && best < __builtin_inff())
-        atomicMax(reinterpret_cast<uint32_t*>(&lab[i].w),
-                  __float_as_uint(1.0f / (sqrtf(best) + 1.0f)));
+        atomicMax(reinterpret_cast<uint32_t*>(&lab[i].w), __float_as_uint(term_of_square(best)));
 }
 
 void launch_near_terms(float4* lab, int32_t n, hipStream_t stream) {

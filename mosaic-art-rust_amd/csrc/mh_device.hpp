@@ -225,16 +225,20 @@ __device__ __forceinline__ float sq_distance(float ql, float qa, float qb, float
 // rounded ones, without the scaling for ranges that cannot occur: the sum of
 // squares is raised to 2^-64 at least (the distance is then lost in the + 1
 // anyway), and an infinite one gives NaN and so the final max's 0.  Equal to
-// 1.0f / (sqrtf(d) + 1.0f) for every non-negative float d: all 2^31 were
-// compared on the device.  19 instructions for 45.
-__device__ __forceinline__ float adj_term(float4 p, float4 q) {
-    const float dl = p.x - q.x, da = p.y - q.y, db = p.z - q.z;
-    const float d = __builtin_fmaxf(dl * dl + da * da + db * db, 0x1p-64f);
+// 1.0f / (sqrtf(d) + 1.0f) for every non-negative float d, and so monotone:
+// test_gpu_identities.py compares all of them on the device.  19 instructions
+// for 45.
+__device__ __forceinline__ float term_of_square(float sum) {
+    const float d = __builtin_fmaxf(sum, 0x1p-64f);
     const float r = __builtin_amdgcn_rsqf(d);
     const float g = d * r;
     const float x = __builtin_fmaf(__builtin_fmaf(-g, g, d), 0.5f * r, g) + 1.0f;
     const float c = __builtin_amdgcn_rcpf(x);
     return __builtin_fmaxf(__builtin_fmaf(__builtin_fmaf(-x, c, 1.0f), c, c), 0.0f);
+}
+__device__ __forceinline__ float adj_term(float4 p, float4 q) {
+    const float dl = p.x - q.x, da = p.y - q.y, db = p.z - q.z;
+    return term_of_square(dl * dl + da * da + db * db);
 }
 
 // ----------------------------------------------------------- counter RNG
@@ -264,8 +268,8 @@ __device__ __forceinline__ float clamp_unit(float v) { return __builtin_amdgcn_f
 
 // a / b, correctly rounded, for |a| <= b, 2^-60 < b <= 1 and a = 0 or
 // |a| > 2^-90: the hardware's reciprocal corrected by its fused residual is the
-// correctly rounded one (compared for every mantissa, as part of adj_term),
-// and a product with that, corrected once by its exact residual, the quotient
+// correctly rounded one (test_gpu_identities.py compares every such b on the
+// device), and a product with that, corrected once by its exact residual, the quotient
 // (Markstein).  6 instructions; the general division scales for ranges that do
 // not occur here, 12.  (rgb_to_hsv divides differences of values in [0, 1]
 // that are sums with a u8 / 255 table or with 0.5: no nonzero one is below
