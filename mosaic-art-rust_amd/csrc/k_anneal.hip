@@ -327,7 +327,9 @@ __device__ float total_cost_block(const G* grid, int32_t gw, int32_t gh, const T
 //   * expecting none: every lane reads the cells as they are, accepted lanes
 //     stamp theirs, and a lane with a lower lane's stamp on any of its ten
 //     cells ends the prefix: 20 p / cells.
-// The second is better for p < 5/9.
+// The second is better for p < 5/9, over the last eight rounds or so: a round of a
+// small grid decides a few proposals, too few to tell by (5,000 on 300 cells, 39%
+// accepted: 1,065 -> 977 us).
 //
 // Measured against one wave that gathered its terms from a matrix of all pairs
 // and added the initial cost one term after another: 1,000 proposals on 20 x
@@ -664,6 +666,7 @@ __device__ __forceinline__ void judge_wave(const AnnealJob& job, const AnnealSha
     const int32_t gw = job.grid_w, gh = job.grid_h;
     const int64_t max_iter = job.max_iter;
     int64_t kbase = P.evaluated, accepted = P.accepted, evaluated = P.evaluated, rounds = P.rounds;
+    int32_t lean = 0;  // accepted shares above 5/9, decaying
     // the last round's, for the traces
     const bool traced = job.trace_delta || job.trace_accept;
     float delta = 0.0f;
@@ -779,9 +782,10 @@ __device__ __forceinline__ void judge_wave(const AnnealJob& job, const AnnealSha
         // the accepted deltas for the cost wave (adding +0.0 changes no sum)
         S.pack[lane] = lane_in(accmask) ? delta : 0.0f;
         const int32_t n_acc = __popcll(accmask), n_ev = __popcll(nonskip & commit);
+        lean += 9 * n_acc - 5 * n_ev - lean / 8;
         if (lane == 0)
             S.ctrl[kCtrlRound] =
-                pack_round(first, !job.greedy && 9 * n_acc >= 5 * n_ev, !as_expected, n_acc);
+                pack_round(first, !job.greedy && lean >= 0, !as_expected, n_acc);
         accepted += n_acc;
         evaluated += n_ev;
         kbase += n_ev;
@@ -1007,6 +1011,9 @@ __device__ __forceinline__ int32_t neighbour_node(const Touch& T, int32_t block,
 // The rounds take over for good when the blocks, over the last sixteen or so,
 // commit less than rounds do in a block's time: a round commits some 0.55
 // sqrt(cells) if all is accepted, and a block takes 1.6 to 1.8 times as long.
+// The mean begins a quarter above that line: a run that begins cold leaves after
+// some four blocks, not after the 23 (300 cells) or 38 (48) that a mean that begins
+// at 64 takes to fall (1,000 proposals on 300 cells, 8% accepted, 195 -> 152 us).
 template <typename G>
 __device__ __forceinline__ void follow_blocks(const AnnealJob& job, const AnnealShared<G>& S, G* grid,
                                               const Touch& T, int w, int lane, Progress& P) {
@@ -1015,7 +1022,7 @@ __device__ __forceinline__ void follow_blocks(const AnnealJob& job, const Anneal
     const int32_t least =
         (int32_t)(16.0f * 0.88f * __builtin_sqrtf((float)(job.grid_w * job.grid_h)));
     int64_t filled = kRing;
-    int32_t block = 0, pending = 0, added_last = 0, mean = 16 * 64;
+    int32_t block = 0, pending = 0, added_last = 0, mean = least + least / 4;
     const bool traced = job.trace_delta || job.trace_accept;
     bool again = true;
     CostSum C;
