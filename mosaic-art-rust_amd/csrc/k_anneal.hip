@@ -66,12 +66,13 @@ struct TermLds {
 // Down, Left, Right, skipping p2), then of p2 (skipping p1), then the mutual
 // term when adjacent.  Absent terms are added as +0.0: the sums start at +0
 // and only grow, and x + (+0) == x bit for bit, so this equals skipping them.
-__device__ float swap_delta_dev(const int32_t* grid, int32_t gw, int32_t gh, const TermLab& T,
+// Bound by latency: all ten cells are read at once, then their Labs (a neighbour
+// outside reads its own cell, an empty one material 0's Lab).
+__device__ float swap_delta_dev(const int32_t* grid, int32_t gw, int32_t gh, const float4* lab4,
                                 int32_t x1, int32_t y1, int32_t x2, int32_t y2) {
     const int32_t p1 = y1 * gw + x1, p2 = y2 * gw + x2;
     const int32_t m1 = gget(grid, p1), m2 = gget(grid, p2);
-    if (m1 == kEmpty || m2 == kEmpty || m1 == m2) return 0.0f;
-    float old_cost = 0.0f, new_cost = 0.0f;
+    int32_t a[8];
     bool adjacent = false;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -81,13 +82,24 @@ __device__ float swap_delta_dev(const int32_t* grid, int32_t gw, int32_t gh, con
         const int32_t q = k == 0 ? p - gw : k == 1 ? p + gw : k == 2 ? p - 1 : p + 1;
         const bool self = in && q == (i < 4 ? p2 : p1);  // the swap partner
         adjacent = adjacent || self;
-        const int32_t a = in && !self ? gget(grid, q) : kEmpty;
-        const float t1 = a != kEmpty ? T(m1, a) : 0.0f, t2 = a != kEmpty ? T(m2, a) : 0.0f;
-        old_cost += i < 4 ? t1 : t2;
-        new_cost += i < 4 ? t2 : t1;
+        const int32_t v = gget(grid, in ? q : p);
+        a[i] = in && !self ? v : kEmpty;
+    }
+    if (m1 == kEmpty || m2 == kEmpty || m1 == m2) return 0.0f;
+    const float4 l1 = gload4(lab4, m1), l2 = gload4(lab4, m2);
+    float4 la[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) la[i] = gload4(lab4, max(a[i], 0));
+    float old_cost = 0.0f, new_cost = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const float t1 = adj_term(l1, la[i]), t2 = adj_term(l2, la[i]);
+        const bool there = a[i] != kEmpty;
+        old_cost += there ? (i < 4 ? t1 : t2) : 0.0f;
+        new_cost += there ? (i < 4 ? t2 : t1) : 0.0f;
     }
     if (adjacent) {
-        const float t = T(m1, m2);
+        const float t = adj_term(l1, l2);
         old_cost += t;
         new_cost += t;
     }
@@ -1400,7 +1412,7 @@ __global__ void swap_delta_kernel(const int32_t* __restrict__ grid, int32_t gw, 
     const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= p) return;
     const int32_t* q = pairs + 4 * (int64_t)i;
-    out[i] = swap_delta_dev(grid, gw, gh, TermLab{lab4}, q[0], q[1], q[2], q[3]);
+    out[i] = swap_delta_dev(grid, gw, gh, lab4, q[0], q[1], q[2], q[3]);
 }
 
 void launch_swap_deltas(const int32_t* grid, int32_t gw, int32_t gh, const float4* lab4,
