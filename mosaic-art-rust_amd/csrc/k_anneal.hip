@@ -794,7 +794,7 @@ __device__ __forceinline__ void judge_wave(const AnnealJob& job, const AnnealSha
         // the accepted deltas for the cost wave (adding +0.0 changes no sum)
         S.pack[lane] = lane_in(accmask) ? delta : 0.0f;
         const int32_t n_acc = __popcll(accmask), n_ev = __popcll(nonskip & commit);
-        lean += 9 * n_acc - 5 * n_ev - lean / 8;
+        lean = (lean - (lean >> 3)) + (9 * n_acc - 5 * n_ev);
         if (lane == 0)
             S.ctrl[kCtrlRound] =
                 pack_round(first, !job.greedy && lean >= 0, !as_expected, n_acc);
