@@ -536,8 +536,8 @@ def _image_table(images):
     arrs = [_c(im, np.uint8) for im in images]
     h = np.array([a.shape[0] for a in arrs], np.int32)
     w = np.array([a.shape[1] for a in arrs], np.int32)
-    sizes = np.array([a.size for a in arrs], np.int64)
-    if sizes.sum() < _COPY_BELOW * len(arrs):
+    if 3 * np.dot(w.astype(np.int64), h) < _COPY_BELOW * len(arrs):
+        sizes = np.array([a.size for a in arrs], np.int64)
         buf = np.concatenate([a.reshape(-1) for a in arrs])
         return buf, _ptr(buf), np.cumsum(sizes) - sizes, w, h
     at = np.array([a.__array_interface__["data"][0] for a in arrs], np.int64)
