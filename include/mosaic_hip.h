@@ -309,11 +309,9 @@ int mh_generate_device_result(mh_context *ctx, mh_job_result *result);
  * the library's resized tiles for the job's cell size must already exist
  * when d_image_out is given (any mh_generate / mh_generate_device /
  * mh_composite at that cell size builds them; else MH_ERR_UNSUPPORTED), and
- * the adjacency terms come from the Lab table instead of the library's term
- * matrix (the same bits).  Phase timing is not recorded.  Every call on one
- * GPU shares that GPU's array and leaves its contents behind: calls that
- * overlap on one GPU (two contexts, or two host threads) race, so callers
- * order them. */
+ * phase timing is not recorded.  Every call on one GPU shares that GPU's
+ * array and leaves its contents behind: calls that overlap on one GPU (two
+ * contexts, or two host threads) race, so callers order them. */
 #define MH_NOALLOC_SCRATCH_BYTES (64ull << 20)
 int mh_generate_device_noalloc(mh_context *ctx, const mh_library *lib, const uint8_t *d_target,
                                int32_t width, int32_t height, const mh_job_params *params,
@@ -401,7 +399,7 @@ int mh_batch_set_tuning(mh_batch *batch, const mh_batch_tuning *tuning);
  * allocated in chunks of 1 GiB (or one job's size, if larger) as admitted
  * jobs need it, never beyond memory_budget; a job that finds no device
  * memory while nothing else runs fails with MH_ERR_OUT_OF_MEMORY.  Libraries
- * stay resident with their term matrices and resized tiles.  The context's
+ * stay resident with their resized tiles.  The context's
  * other entry points must not run concurrently with a live server. */
 typedef struct {
     int64_t memory_budget;  /* bytes of device working memory (0 = 64 GiB) */

@@ -15,10 +15,12 @@
 // sqrt(sqdist) + penalty with everything else unchanged: its candidate rows
 // hold the square roots (k_topk.hip), and nothing here differs.
 //
-// Two kernels:
+// Three kernels:
 //  * place_raster_kernel -- what generate_mosaic runs: raster order from an
 //    empty grid, so only Up and Left can be filled.  One workgroup per job:
 //    a chain wave, and waves that prepare its candidates (below).
+//  * place_outputs_kernel -- the distances and scores of such a run's cells,
+//    after it, where the caller wants them.
 //  * place_chain_kernel -- any cell order over a pre-filled grid and usage
 //    (find_and_use_best_tile_with_position at arbitrary cells), one wave;
 //    grid and usage in LDS, all four neighbours read per cell.  Its HBM form

@@ -3,7 +3,7 @@
 //
 // A batch runs every job's whole pipeline with one launch per stage:
 //   cell Lab means -> K nearest -> placement chains (a workgroup per job) ->
-//   annealing chains (a wave per job) -> cell averages + adjustments ->
+//   annealing chains (a workgroup per job) -> cell averages + adjustments ->
 //   composite.
 // Wide stages find their job through a segment table (block -> job by
 // binary search over per-job block offsets); chain stages take a job array.
@@ -981,7 +981,7 @@ struct StreamSlot {
 // candidate lists (cell Labs, K nearest), which fill the device, run on two
 // wide streams, consecutive batches alternating (so one batch's launch tail
 // overlaps the next batch's start); each batch's chains (placement,
-// annealing: a workgroup or wave per job, latency-bound) run on one of a few chain
+// annealing: a workgroup per job, latency-bound) run on one of a few chain
 // streams after an event from the wide stream; its output stages
 // (adjustment, composite: wide again) run on that chain stream's output
 // stream after an event from the chain stream, so a batch's outputs never

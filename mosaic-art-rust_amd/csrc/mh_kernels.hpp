@@ -24,7 +24,7 @@ struct CandRec {
 };
 static_assert(sizeof(CandRec) == 8, "one 64-bit word per candidate");
 
-// One placement chain (one wave).  All pointers are device pointers.
+// One placement chain (one workgroup).  All pointers are device pointers.
 struct PlaceJob {
     const float4* lab4;      // n material Labs {l,a,b} and their largest adjacency terms
     int32_t n;
