@@ -1370,7 +1370,7 @@ size_t place_raster_lds_bytes(int32_t grid_w, int32_t n, int32_t form) {
 }
 
 // Where each form stands: the lists take 28 KB and 4 bytes a material (to
-// about 33,700 materials), the Labs 16 bytes a material more.  A flagged
+// about 33,800 materials), the Labs 16 bytes a material more.  A flagged
 // cell's Labs come from LDS in 0.4 us, from memory in 0.7-1 us.  Without room
 // for the lists (33,800 to 40,700 materials) a cell costs 0.56 us plain, as
 // one wave that read ahead in registers did.
